@@ -1136,16 +1136,13 @@ __device__ inline void neumann_walls(double * __restrict__ a, int i, int nx, int
 }
 
 // Multi-field line solver: one launch solves the x lines of up to four
-// fields (blockIdx.y selects the field).  256 lines per work-group, one line
-// per lane; x is streamed through LDS in chunks of CH values stored x-major
-// (tile[m][line]) so that the cooperative global accesses are contiguous
-// rows and each lane's walk along its line is bank-conflict free.
+// fields (blockIdx.y selects the field).
 struct LineField {
   const double * tab;        // {c0, rlast, flag, -, l[n], val[n], v[n]}
   const double * srca;       // increments from the three sources when srcg
   const double * srcb;       //   is non-null (per-function entry point) ...
   const double * srcg;
-  double * q;                // ... else q holds them; forward result goes to q
+  double * q;                // ... else q holds them
   double * field;
   int n, n0, i0;             // line length, padded x width, first DOF column
 };
@@ -1154,205 +1151,80 @@ struct LineJob {
   int nlines, ny, n1;        // lines per field, rows per plane, padded rows (0 in 2D)
   double ca, cb, cg;
   int images, nz;            // also write periodic halo images (fused schedule)
+  unsigned inv_ny;           // 2^32 / ny, rounded up: umulhi(j, inv_ny) = j / ny for j < 2^32 / ny
 };
 
-constexpr int kLLines = 256;
-constexpr int kLStride = 264;
-
-template <int CH>
-__device__ __forceinline__ void k_lines_body(const VBlock & vb, LineJob J) {
-  __shared__ double T[CH][kLStride];
-  __shared__ double U[CH][kLStride];
-  const LineField & F = J.f[vb.y];
-  const int tid = threadIdx.x;
-  const int line0 = vb.x * kLLines;
-  const int myline = line0 + tid;
-  const int n = F.n;
-  const int nlines = J.nlines;
-  const double c0 = F.tab[0], rlast = F.tab[1];
-  const bool flag = F.tab[2] != 0.;
-  const double * __restrict__ L = F.tab + 4;
-  const double * __restrict__ VAL = F.tab + 4 + n;
-  const double * __restrict__ V = F.tab + 4 + 2 * n;
-  double qprev = 0.;
-  for (int c = 0; c < n; c += CH) {
-    const int w = min(CH, n - c);
-    for (int e = tid; e < kLLines * CH; e += kLLines) {
-      const int ll = e / CH, m = e % CH;
-      const int line = line0 + ll;
-      if (m < w && line < nlines) {
-        const size_t g = (size_t)line * n + c + m;
-        T[m][ll] = F.srcg ? +J.ca * F.srca[g] + J.cb * F.srcb[g] + J.cg * F.srcg[g] : F.q[g];
-      }
-    }
-    __syncthreads();
-    if (myline < nlines) {
-#pragma unroll
-      for (int m = 0; m < CH; m++) {
-        if (m < w) {
-          const int ii = c + m;
-          double qi = T[m][tid];
-          if (ii == 0) {
-            qi = qi / c0;
-          } else if (ii < n - 1) {
-            qi = VAL[ii] * (qi - L[ii] * qprev);
-          } else {
-            qi = flag ? rlast * (qi - L[ii] * qprev) : 0.;
-          }
-          T[m][tid] = qi;
-          qprev = qi;
-        }
-      }
-    }
-    __syncthreads();
-    for (int e = tid; e < kLLines * CH; e += kLLines) {
-      const int ll = e / CH, m = e % CH;
-      const int line = line0 + ll;
-      if (m < w && line < nlines) F.q[(size_t)line * n + c + m] = T[m][ll];
-    }
-    __syncthreads();
-  }
-  double qnext = 0.;
-  const int last_c = ((n - 1) / CH) * CH;
-  for (int c = last_c; c >= 0; c -= CH) {
-    const int w = min(CH, n - c);
-    for (int e = tid; e < kLLines * CH; e += kLLines) {
-      const int ll = e / CH, m = e % CH;
-      const int line = line0 + ll;
-      if (m < w && line < nlines) {
-        T[m][ll] = F.q[(size_t)line * n + c + m];
-        const int jj = line % J.ny, kk = line / J.ny;
-        U[m][ll] = F.field[(size_t)(F.i0 + c + m) + (size_t)F.n0 * ((size_t)(jj + 1) + (size_t)J.n1 * (size_t)(kk + 1))];
-      }
-    }
-    __syncthreads();
-    if (myline < nlines) {
-#pragma unroll
-      for (int m = CH - 1; m >= 0; m--) {
-        if (m < w) {
-          const int ii = c + m;
-          double qi = T[m][tid];
-          if (ii < n - 1) qi -= V[ii] * qnext;
-          qnext = qi;
-          U[m][tid] += qi;
-        }
-      }
-    }
-    __syncthreads();
-    for (int e = tid; e < kLLines * CH; e += kLLines) {
-      const int ll = e / CH, m = e % CH;
-      const int line = line0 + ll;
-      if (m < w && line < nlines) {
-        const int jj = line % J.ny, kk = line / J.ny;
-        F.field[(size_t)(F.i0 + c + m) + (size_t)F.n0 * ((size_t)(jj + 1) + (size_t)J.n1 * (size_t)(kk + 1))] = U[m][ll];
-      }
-    }
-    __syncthreads();
-  }
-}
-
-template <int CH>
-__global__ __launch_bounds__(kLLines) void k_lines(LineJob J) {
-  k_lines_body<CH>(hw_block(), J);
-}
-
-// Whole-line variant: a work-group keeps `lpb` complete lines in LDS (odd
-// row stride, so the lanes walking different lines hit different banks).
-// Phase 1 copies the increments (one contiguous block: the lines of a group
-// are adjacent) into LDS with every lane and several loads in flight,
-// phase 2 runs forward elimination and back substitution on-chip with one
-// lane per line, phase 3 adds the solution to the field rows.  Traffic per
-// DOF: increments once, field read and write once.
+// A work-group keeps `lpb` complete lines in LDS.  Phase 1 copies the
+// increments (one contiguous block: the lines of a group are adjacent) into
+// LDS with every lane and several loads in flight, phase 2 runs forward
+// elimination and back substitution on-chip (lines_sweep_rows, 16 lines per
+// wavefront), phase 3 adds the solution to the field rows.  Traffic per DOF:
+// increments once, field read and write once.  Bound by HBM: 256^3 (four
+// fields, 1.64 GB) 495 -> 338 us (4.85 TB/s, the copy rate is 5.3); where the
+// chip is not filled, by the serial sweep: 128 x 256 20.5 -> 10.6 us, 512 x
+// 1024 65 -> 31 us.  78 VGPRs and 25 KiB of LDS let six work-groups share a
+// CU; 32 rows per lane instead of 16 (127 VGPRs, four groups) took 366 us, 5
+// and 8 loads per batch 340 and 349, work-groups of 128, 192 and 512 threads
+// 380, 334 (but 65 instead of 59 us on 150 x 135 x 100) and 391.
 constexpr int kWThreads = 256;
-constexpr int kWUnroll = 4;
+constexpr int kWUnroll = 6;
 
-// Phases of the x-line solve of `nl` lines starting at line0, their values
-// staged in S (row stride ld).  Phase 1: increments into S, by threads
-// t = 0..nt-1; element e = t + nt r, (ll, m) tracked incrementally.
-__device__ __forceinline__ void lines_fill(const LineField & F, const LineJob & J, double * S, int ld, int line0,
-                                           int nl, int t, int nt) {
-  const int n = F.n;
-  const int total = nl * n;
-  const size_t g0 = (size_t)line0 * n;
-  {
-    int e = t, ll = t / n, m = t - (t / n) * n;
-    while (e < total) {
-      double v[kWUnroll];
-      int lls[kWUnroll], ms[kWUnroll], cnt = 0;
+// Phases 1 and 3 walk the (line, 64-row chunk) pairs of a group: wavefront w
+// of nw owns pairs w, w + nw, ..., kWUnroll at a time with all their loads
+// issued (indices clamped, so that no branch separates them) before the
+// first value is used.  Line, row, plane and chunk are wave-uniform.  Pair p
+// is chunk p % nch of line p / nch; the quotient comes from a 16-bit
+// reciprocal (a group has at most 192 pairs and nch <= 128).
+__device__ __forceinline__ int pair_line(int p, int inv) { return (p * inv) >> 16; }
+
+struct LineGroup {             // the lines of one work-group, uniform
+  int n, ld, np, nch, inv;     // rows, LDS stride, pairs, chunks of a line and their reciprocal
+  int j0, k0, nw, lane;        // row and plane of the first line; wavefronts
+  size_t g0;                   // its first increment
+};
+
+// the increments of pairs p0 + nw u into registers
+__device__ __forceinline__ void lines_load(const LineField & F, const LineGroup & G, int p0, double * v) {
 #pragma unroll
-      for (int u = 0; u < kWUnroll; u++) {
-        if (e < total) {
-          const size_t g = g0 + e;
-          v[u] = F.srcg ? +J.ca * F.srca[g] + J.cb * F.srcb[g] + J.cg * F.srcg[g] : F.q[g];
-          lls[u] = ll;
-          ms[u] = m;
-          cnt = u + 1;
-          e += nt;
-          m += nt;
-          while (m >= n) { m -= n; ll++; }
-        }
-      }
+  for (int u = 0; u < kWUnroll; u++) {
+    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
+    v[u] = F.q[G.g0 + (size_t)(l * G.n + min(64 * (p - l * G.nch) + G.lane, G.n - 1))];
+  }
+}
+// ... and into S (clamped lanes and pairs repeat a value of their wavefront)
+__device__ __forceinline__ void lines_stage(const LineGroup & G, double * S, int p0, const double * v) {
 #pragma unroll
-      for (int u = 0; u < kWUnroll; u++)
-        if (u < cnt) S[lls[u] * ld + ms[u]] = v[u];
-    }
+  for (int u = 0; u < kWUnroll; u++) {
+    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
+    S[l * G.ld + min(64 * (p - l * G.nch) + G.lane, G.n - 1)] = v[u];
   }
 }
 
-// phase 2: forward elimination and back substitution of one line q[0..n-1]
-// (the reference's gtsv with the shared factors of the table)
-__device__ __forceinline__ void lines_sweep(const LineField & F, double * q) {
-  const int n = F.n;
-  {
-    const double c0 = F.tab[0], rlast = F.tab[1];
-    const bool flag = F.tab[2] != 0.;
-    const double * __restrict__ L = F.tab + 4;
-    const double * __restrict__ VAL = F.tab + 4 + n;
-    const double * __restrict__ V = F.tab + 4 + 2 * n;
-    double qprev = q[0] / c0;
-    q[0] = qprev;
-    int i = 1;
-    for (; i + 4 <= n - 1; i += 4) {
-      double a0 = q[i], a1 = q[i + 1], a2 = q[i + 2], a3 = q[i + 3];
-      a0 = VAL[i] * (a0 - L[i] * qprev);
-      a1 = VAL[i + 1] * (a1 - L[i + 1] * a0);
-      a2 = VAL[i + 2] * (a2 - L[i + 2] * a1);
-      a3 = VAL[i + 3] * (a3 - L[i + 3] * a2);
-      q[i] = a0; q[i + 1] = a1; q[i + 2] = a2; q[i + 3] = a3;
-      qprev = a3;
-    }
-    for (; i < n - 1; i++) {
-      const double a = VAL[i] * (q[i] - L[i] * qprev);
-      q[i] = a;
-      qprev = a;
-    }
-    {
-      const double a = flag ? rlast * (q[n - 1] - L[n - 1] * qprev) : 0.;
-      q[n - 1] = a;
-      qprev = a;
-    }
-    double qnext = qprev;
-    i = n - 2;
-    for (; i - 3 >= 0; i -= 4) {
-      double a0 = q[i], a1 = q[i - 1], a2 = q[i - 2], a3 = q[i - 3];
-      a0 -= V[i] * qnext;
-      a1 -= V[i - 1] * a0;
-      a2 -= V[i - 2] * a1;
-      a3 -= V[i - 3] * a2;
-      q[i] = a0; q[i - 1] = a1; q[i - 2] = a2; q[i - 3] = a3;
-      qnext = a3;
-    }
-    for (; i >= 0; i--) {
-      const double a = q[i] - V[i] * qnext;
-      q[i] = a;
-      qnext = a;
-    }
+// row j and plane k (0-based) of line l of the group, and its first DOF
+__device__ __forceinline__ size_t lines_row(const LineField & F, const LineJob & J, const LineGroup & G, int l, int & j,
+                                            int & k) {
+  const int t = G.j0 + l, c = (int)__umulhi((unsigned)t, J.inv_ny);
+  j = t - c * J.ny;
+  k = G.k0 + c;
+  return (size_t)F.i0 + (size_t)F.n0 * ((size_t)(j + 1) + (size_t)J.n1 * (size_t)(k + 1));
+}
+
+// the field values of the same pairs
+__device__ __forceinline__ void lines_field(const LineField & F, const LineJob & J, const LineGroup & G, int p0,
+                                            double * v) {
+#pragma unroll
+  for (int u = 0; u < kWUnroll; u++) {
+    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
+    int j, k;
+    const size_t r = lines_row(F, J, G, l, j, k);
+    v[u] = F.field[r + (size_t)min(64 * (p - l * G.nch) + G.lane, G.n - 1)];
   }
 }
 
-// The same by a whole wavefront (the one-kernel predictor, whose waves have
-// nothing else to do meanwhile): lane l < nl eliminates line l (rows at
-// q0 + l ld); the other lanes follow line 0 without storing.  The factors
+// phase 2 by a whole wavefront (the one-kernel predictor, whose lines may
+// start at any LDS row): forward elimination and back substitution, lane l <
+// nl eliminates line l (rows at q0 + l ld); the other lanes follow line 0
+// without storing.  The factors
 // L, VAL, V of 64 consecutive rows are loaded one row per lane (a coalesced
 // vector load, issued one chunk ahead) and each row's pair is broadcast with
 // v_readlane, so that neither scalar loads (whose out-of-order return makes
@@ -1437,86 +1309,306 @@ __device__ __forceinline__ void lines_sweep_wave(const double * tab, int n, doub
   }
 }
 
-// phase 3: field rows += solution by wavefronts w = 0..nw-1 (lane = lane
-// index).  Wavefront w owns lines w, w + nw, ... (two per pass), so a
-// line's row / plane, its address and whether it has periodic halo images
-// are wave-uniform; lanes walk x contiguously.
-__device__ __forceinline__ void lines_update(const LineField & F, const LineJob & J, const double * S, int ld,
-                                             int line0, int nl, int w, int nw, int lane) {
-  const int n = F.n;
-  {
-    for (int la = w; la < nl; la += 2 * nw) {
-      const int lb = la + nw;
-      const bool hb = lb < nl;
-      const int linea = line0 + la, lineb = line0 + (hb ? lb : la);
-      const int ja = linea % J.ny, ka = linea / J.ny;
-      const int jb = lineb % J.ny, kb = lineb / J.ny;
-      double * __restrict__ ra = F.field + F.i0 + (size_t)F.n0 * ((size_t)(ja + 1) + (size_t)J.n1 * (size_t)(ka + 1));
-      double * __restrict__ rb = F.field + F.i0 + (size_t)F.n0 * ((size_t)(jb + 1) + (size_t)J.n1 * (size_t)(kb + 1));
-      const double * sa = S + la * ld;
-      const double * sb = S + (hb ? lb : la) * ld;
-      for (int m0 = 0; m0 < n; m0 += 64 * kWUnroll) {
-        double va[kWUnroll], vb[kWUnroll];
+// Phase 2 of k_lines_lds: one wavefront eliminates up to 16 lines (line l at
+// S + l ld) with the rows in registers.  Lane 16 h + l holds rows 128 p + 32 h
+// .. + 31 of line l (pass p), so a line runs through the four 16-lane DPP rows
+// in turn: row h works under its exec mask, then hands x of its last row on
+// (rot_up / rot_dn).  The factors of a lane row's 32 matrix rows sit in two
+// registers per factor, one matrix row per lane, and reach all 16 lanes by a
+// 64-bit row_newbcast move; a serial row is then 2 moves + 3 FP64 operations
+// forward and 1 + 2 backward, with no LDS access and no scalar load (whose
+// out-of-order return makes each use wait for everything outstanding) on the
+// recurrence.  LDS is read and written 16 bytes at a time, twice per pass.
+// At 256 rows the sweep takes 7.6 us with the tables loaded on use, against
+// 11.2 us with rows read from LDS two groups of 8 ahead and v_readlane
+// factors, 14.7 us with one group ahead, 15.1 us with scalar-load factors
+// (16 lines, three work-groups per CU).
+// Per line the operations are gtsv's: q[0] / c0 (then row 0 is a row with L =
+// 0, VAL = 1), q[i] = VAL[i] (q[i] - L[i] q[i-1]) with VAL = rlast in the last
+// row (0 there when the last pivot is singular), back substitution q[i] -=
+// V[i] q[i+1].  Rows past the last one hold no line's data; they are dropped
+// where the back substitution starts.
+extern "C" __device__ long long vof_update_dpp_i64(long long, long long, int, int, int, bool)
+    __asm("llvm.amdgcn.update.dpp.i64");
+// lane E of each 16-lane row to the whole row
+template <int E>
+__device__ __forceinline__ double row_lane(double v) {
+  return __longlong_as_double(vof_update_dpp_i64(0ll, __double_as_longlong(v), 0x150 + E, 0xf, 0xf, true));
+}
+// v_permlane16_swap / v_permlane32_swap of v with itself: a has the even
+// 16-lane rows (lower 32 lanes) in both places, b the odd (upper) ones
+__device__ __forceinline__ void rows_swap16(double v, double & a, double & b) {
+  const unsigned long long z = (unsigned long long)__double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)z, (unsigned)z, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(z >> 32), (unsigned)(z >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ void rows_swap32(double v, double & a, double & b) {
+  const unsigned long long z = (unsigned long long)__double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)z, (unsigned)z, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(z >> 32), (unsigned)(z >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+// 16-lane row h takes the value of row h - 1 (h + 1), modulo 4
+__device__ __forceinline__ double rot_up(double v, int h) {
+  double a, b, c, d;
+  rows_swap16(v, a, b);
+  rows_swap32(b, c, d);
+  return (h & 1) ? a : h == 2 ? c : d;
+}
+__device__ __forceinline__ double rot_dn(double v, int h) {
+  double a, b, c, d;
+  rows_swap16(v, a, b);
+  rows_swap32(a, c, d);
+  return (h & 1) ? (h == 1 ? d : c) : b;
+}
+
+constexpr int kSwLines = 16;   // lines per sweeping wavefront
+constexpr int kSwRows = 16;    // rows per lane and pass
+constexpr int kSwTab = kSwRows / 16;   // factor registers of a lane
+
+template <int R>
+struct SweepRows {             // rows R .. kSwRows - 1 forward, R .. 0 backward
+  static __device__ __forceinline__ void fwd(double2 * x, const double * tl, const double * tv, double & prev) {
+    if constexpr (R < kSwRows) {
+      double & xr = (R & 1) ? x[R >> 1].y : x[R >> 1].x;
+      xr = row_lane<R & 15>(tv[R >> 4]) * (xr - row_lane<R & 15>(tl[R >> 4]) * prev);
+      prev = xr;
+      SweepRows<R + 1>::fwd(x, tl, tv, prev);
+    }
+  }
+  static __device__ __forceinline__ void bwd(double2 * x, const double * tw, double & prev) {
+    if constexpr (R >= 0) {
+      double & xr = (R & 1) ? x[R >> 1].y : x[R >> 1].x;
+      xr -= row_lane<R & 15>(tw[R >> 4]) * prev;
+      prev = xr;
+      SweepRows<R - 1>::bwd(x, tw, prev);
+    }
+  }
+  // the segment of the last row (row - base = top): rows from it on stay
+  static __device__ __forceinline__ void bwd_top(double2 * x, const double * tw, double & prev, int top, bool flag) {
+    if constexpr (R >= 0) {
+      double & xr = (R & 1) ? x[R >> 1].y : x[R >> 1].x;
+      const double a = xr - row_lane<R & 15>(tw[R >> 4]) * prev;
+      xr = R < top ? a : flag ? xr : 0.;
+      prev = xr;
+      SweepRows<R - 1>::bwd_top(x, tw, prev, top, flag);
+    }
+  }
+};
+
+struct SweepHead {             // what a sweep needs first, loadable ahead of it
+  double c0, flag;
+  double tl[kSwTab], tv[kSwTab];   // L and VAL of pass 0
+};
+// L and VAL (fwd) or V (bwd) of a lane's matrix rows in pass p
+__device__ __forceinline__ void sweep_fwd_tab(const double * tab, int n, int p, int lane, double * tl, double * tv) {
 #pragma unroll
-        for (int u = 0; u < kWUnroll; u++) {
-          const int m = m0 + 64 * u + lane;
-          if (m < n) {
-            va[u] = ra[m] + sa[m];
-            if (hb) vb[u] = rb[m] + sb[m];
-          }
-        }
+  for (int k = 0; k < kSwTab; k++) {
+    const int row = kSwRows * (4 * p + (lane >> 4)) + 16 * k + (lane & 15), r = min(row, n - 1);
+    const double a = tab[4 + r], b = tab[4 + n + r];
+    tl[k] = row == 0 ? 0. : a;
+    tv[k] = row == 0 ? 1. : b;
+  }
+}
+__device__ __forceinline__ void sweep_bwd_tab(const double * tab, int n, int p, int lane, double * tw) {
 #pragma unroll
-        for (int u = 0; u < kWUnroll; u++) {
-          const int m = m0 + 64 * u + lane;
-          if (m < n) {
-            st_stream(&ra[m], va[u]);
-            if (hb) st_stream(&rb[m], vb[u]);
-          }
-        }
+  for (int k = 0; k < kSwTab; k++)
+    tw[k] = tab[4 + 2 * n + min(kSwRows * (4 * p + (lane >> 4)) + 16 * k + (lane & 15), n - 1)];
+}
+__device__ __forceinline__ SweepHead sweep_head(const double * tab, int n, int lane) {
+  SweepHead h;
+  h.c0 = tab[0];
+  h.flag = tab[2];
+  sweep_fwd_tab(tab, n, 0, lane, h.tl, h.tv);
+  return h;
+}
+
+__device__ __forceinline__ void lines_sweep_rows(const SweepHead & hd, const double * tab, int n, double * S, int ld,
+                                                 int nl, int lane) {
+  const int h = lane >> 4, l = lane & 15;
+  const bool act = l < nl;   // the other lanes repeat the last line without storing
+  double2 * q2 = reinterpret_cast<double2 *>(S + (size_t)min(l, nl - 1) * ld);
+  const int nseg = (n + kSwRows - 1) / kSwRows, np = (nseg + 3) >> 2;
+  double2 x[kSwRows / 2];
+  double tl[kSwTab], tv[kSwTab], tw[kSwTab];
+#pragma unroll
+  for (int k = 0; k < kSwTab; k++) {
+    tl[k] = hd.tl[k];
+    tv[k] = hd.tv[k];
+  }
+  double prev = 0.;
+  auto load = [&](int p) {
+    const int s = min(4 * p + h, nseg - 1);
+#pragma unroll
+    for (int u = 0; u < kSwRows / 2; u++) x[u] = q2[(kSwRows / 2) * s + u];
+  };
+  auto store = [&](int p) {
+    const int s = 4 * p + h;
+    if (act && s < nseg) {
+#pragma unroll
+      for (int u = 0; u < kSwRows / 2; u++) q2[(kSwRows / 2) * s + u] = x[u];
+    }
+  };
+  for (int p = 0; p < np; p++) {
+    load(p);
+    double nl_[kSwTab], nv_[kSwTab];
+    if (p + 1 < np) sweep_fwd_tab(tab, n, p + 1, lane, nl_, nv_);
+    else sweep_bwd_tab(tab, n, p, lane, tw);
+    if (p == 0) {
+      const double d = x[0].x / hd.c0;
+      x[0].x = h == 0 ? d : x[0].x;
+    }
+    const int hm = min(4, nseg - 4 * p);
+    for (int hh = 0; hh < hm; hh++) {
+      if (h == hh) SweepRows<0>::fwd(x, tl, tv, prev);
+      prev = rot_up(prev, h);
+    }
+    if (p + 1 < np) {
+      store(p);
+#pragma unroll
+      for (int k = 0; k < kSwTab; k++) {
+        tl[k] = nl_[k];
+        tv[k] = nv_[k];
       }
-      if (J.images) {
-        // rows / planes next to the periodic halo: the entries just stored
-        // go to their images too, and the Dirichlet wall entries of the row
-        // (constants the loop never changes) take their images as the
-        // reference's halo copy would (overwriting values left from the
-        // initial load)
+    }
+  }
+  for (int p = np - 1; p >= 0; p--) {
+    if (p + 1 < np) load(p);
+    double nw_[kSwTab];
+    sweep_bwd_tab(tab, n, max(p - 1, 0), lane, nw_);
+    for (int hh = min(4, nseg - 4 * p) - 1; hh >= 0; hh--) {
+      const int seg = 4 * p + hh;
+      if (h == hh) {
+        if (seg == nseg - 1) SweepRows<kSwRows - 1>::bwd_top(x, tw, prev, n - 1 - kSwRows * seg, hd.flag != 0.);
+        else SweepRows<kSwRows - 1>::bwd(x, tw, prev);
+      }
+      prev = rot_dn(prev, h);
+    }
+    store(p);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          if (h == 1 && !hb) break;
-          const int jj = h ? jb : ja, kk = h ? kb : ka;
-          const bool edge = jj + 1 < 2 || jj + 1 >= J.ny
+    for (int k = 0; k < kSwTab; k++) tw[k] = nw_[k];
+  }
+}
+
+// LDS row stride of lines of n rows: whole segments, and 2 mod 4, so that
+// the lanes' 16-byte accesses to different lines fall in distinct banks
+__host__ __device__ inline int lines_stride(int n) { return kSwRows * ((n + kSwRows - 1) / kSwRows) + 2; }
+
+// rows next to the periodic halo, whose entries have images
+__device__ __forceinline__ bool lines_edge(const LineJob & J, int j, int k) {
+  return J.images && (j == 0 || j == J.ny - 1
 #if NDIMS == 3
-                            || kk + 1 < 2 || kk + 1 >= J.nz
+                      || k == 0 || k == J.nz - 1
 #endif
-              ;
-          if (!edge) continue;
-          const double * row = h ? rb : ra;
-          for (int m = lane; m < n; m += 64)
-            store_images(F.field, F.i0 + m, F.n0, J.n1, jj + 1, kk + 1, J.ny, J.nz, 1, row[m]);
-          if (lane < 2) {
-            const int xw = lane == 0 ? F.i0 - 1 : F.i0 + n;
-            const double wv = F.field[(size_t)xw + (size_t)F.n0 * ((size_t)(jj + 1) + (size_t)J.n1 * (size_t)(kk + 1))];
-            store_images(F.field, xw, F.n0, J.n1, jj + 1, kk + 1, J.ny, J.nz, 1, wv);
-          }
-        }
+                     );
+}
+
+// phase 3: field rows += solution.  Rows next to the periodic halo keep the
+// new values in S too, from where a second, rolled loop stores their images.
+// The Dirichlet wall entries of those rows (constants the loop never changes)
+// take their images as the reference's halo copy would (overwriting values
+// left from the initial load).
+__device__ __forceinline__ void lines_update(const LineField & F, const LineJob & J, const LineGroup & G, double * S,
+                                             int p0, const double * v) {
+  bool any = false;
+#pragma unroll
+  for (int u = 0; u < kWUnroll; u++) {
+    const int p = p0 + G.nw * u;
+    if (p < G.np) {
+      const int l = pair_line(p, G.inv), m = 64 * (p - l * G.nch) + G.lane;
+      int j, k;
+      const size_t r = lines_row(F, J, G, l, j, k);
+      const double x = v[u] + S[l * G.ld + min(m, G.n - 1)];
+      if (m < G.n) st_stream(&F.field[r + (size_t)m], x);
+      if (lines_edge(J, j, k)) {
+        any = true;
+        if (m < G.n) S[l * G.ld + m] = x;
       }
+    }
+  }
+  if (!any) return;
+#pragma unroll 1
+  for (int u = 0; u < kWUnroll; u++) {
+    const int p = p0 + G.nw * u;
+    if (p >= G.np) break;
+    const int l = pair_line(p, G.inv), m = 64 * (p - l * G.nch) + G.lane;
+    int j, k;
+    const size_t r = lines_row(F, J, G, l, j, k);
+    if (!lines_edge(J, j, k)) continue;
+    if (m < G.n) store_images(F.field, F.i0 + m, F.n0, J.n1, j + 1, k + 1, J.ny, J.nz, 1, S[l * G.ld + m]);
+    if (m < 2) {
+      const int xw = m == 0 ? F.i0 - 1 : F.i0 + G.n;
+      store_images(F.field, xw, F.n0, J.n1, j + 1, k + 1, J.ny, J.nz, 1, F.field[r - (size_t)F.i0 + (size_t)xw]);
     }
   }
 }
 
+// Work-group barrier that waits for LDS operations only: global loads issued
+// before it stay in flight (a __syncthreads fence would wait for them).  The
+// release / acquire fences are scoped to the work-group and to LDS ("local"),
+// so the compiler orders the LDS accesses around the barrier itself and
+// waits on the LDS counter only (s_waitcnt lgkmcnt(0); s_barrier).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJob & J, int lpb) {
-  extern __shared__ double S[];
+  extern __shared__ __align__(16) double S[];
   const LineField & F = J.f[vb.y];
-  const int ld = F.n | 1;
-  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
   const int line0 = vb.x * lpb;
   const int nl = min(lpb, J.nlines - line0);
   if (nl <= 0) return;
-  lines_fill(F, J, S, ld, line0, nl, tid, kWThreads);
-  __syncthreads();
-  if (tid < nl) lines_sweep(F, S + tid * ld);
-  __syncthreads();
-  lines_update(F, J, S, ld, line0, nl, tid >> 6, kWThreads / 64, tid & 63);
+  LineGroup G;
+  G.n = F.n;
+  G.ld = lines_stride(F.n);
+  G.nch = (F.n + 63) >> 6;
+  G.np = nl * G.nch;
+  G.inv = (65536 + G.nch - 1) / G.nch;
+  G.k0 = line0 / J.ny;
+  G.j0 = line0 - G.k0 * J.ny;
+  G.nw = kWThreads / 64;
+  G.lane = lane;
+  G.g0 = (size_t)line0 * G.n;
+  const int step = G.nw * kWUnroll;
+  // every load of a batch is issued (indices clamped: a branch between loads
+  // makes the compiler wait for the ones in flight) before its first use; the
+  // first batch's field rows are loaded with its increments and stay in
+  // registers across the sweep (the LDS barriers leave them in flight)
+  double v[kWUnroll], f[kWUnroll];
+  lines_load(F, G, w, v);
+  const SweepHead h = sweep_head(F.tab, G.n, lane);
+  lines_field(F, J, G, w, f);
+  if (F.srcg) {
+    // increments formed here from the three sources (per-function entry
+    // point); the slab just read is not used
+#pragma unroll 1
+    for (int p = w; p < G.np; p += G.nw) {
+      const int l = pair_line(p, G.inv), m = min(64 * (p - l * G.nch) + lane, G.n - 1);
+      const size_t g = G.g0 + (size_t)(l * G.n + m);
+      S[l * G.ld + m] = +J.ca * F.srca[g] + J.cb * F.srcb[g] + J.cg * F.srcg[g];
+    }
+  } else {
+    lines_stage(G, S, w, v);
+    for (int p0 = w + step; p0 < G.np; p0 += step) {
+      lines_load(F, G, p0, v);
+      lines_stage(G, S, p0, v);
+    }
+  }
+  lds_barrier();
+  for (int l = kSwLines * w; l < nl; l += kSwLines * G.nw)
+    lines_sweep_rows(h, F.tab, G.n, S + (size_t)l * G.ld, G.ld, min(kSwLines, nl - l), lane);
+  lds_barrier();
+  lines_update(F, J, G, S, w, f);
+  for (int p0 = w + step; p0 < G.np; p0 += step) {
+    lines_field(F, J, G, p0, f);
+    lines_update(F, J, G, S, p0, f);
+  }
 }
 
 __global__ __launch_bounds__(kWThreads) void k_lines_lds(LineJob J, int lpb) {
@@ -3468,17 +3560,6 @@ __global__ __launch_bounds__(kIThreads) void k_iface_fused_fz(Grid g, const doub
   k_iface_fused_fz_body<FZ>(hw_block(), g, vof, normal, curv, fz);
 }
 #endif
-
-// Work-group barrier that waits for LDS operations only: global loads issued
-// before it stay in flight (a __syncthreads fence would wait for them).  The
-// release / acquire fences are scoped to the work-group and to LDS ("local"),
-// so the compiler orders the LDS accesses around the barrier itself and
-// waits on the LDS counter only (s_waitcnt lgkmcnt(0); s_barrier).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 #if NDIMS == 3
 // k_iface_fused marching in z: a 32 x 8 tile of (x, y) walks KZ planes.

@@ -1484,7 +1484,8 @@ static void build_tab(double * tab, int n, double prefactor, const double * lapx
     tab[2] = 0.;
   }
   tab[3] = 0.;
-  VAL[n - 1] = 0.;
+  // the last row as a row like the others (0 where its pivot is singular)
+  VAL[n - 1] = tab[1];
   V[n - 1] = 0.;
 }
 
@@ -1636,6 +1637,7 @@ static int predict_impl(const domain_t * domain, size_t rkstep, double dt, fluid
   lj.ca = ca; lj.cb = cb; lj.cg = cg;
   lj.images = images;
   lj.nz = nz;
+  lj.inv_ny = 0xffffffffu / (unsigned)ny + 1u;
   if (vof_old) {
     vofk::FusedRhs fr{};
     fr.base = base;
@@ -1761,16 +1763,19 @@ static int predict_impl(const domain_t * domain, size_t rkstep, double dt, fluid
     F.i0 = 1;
   }
   {
-    // lines per work-group: an LDS tile of about 16 KiB (8 lines at nx = 256,
-    // the measured optimum between more resident groups and longer serial
-    // sweeps per group)
-    const int line_bytes = (int)(sizeof(double) * (nx | 1));
-    int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : (16384 + line_bytes - 1) / line_bytes;
-    if (lpb > 64) lpb = 64;
-    if (lpb < 1) lpb = 1;
+    // lines per work-group: 48 (line, 64-row chunk) pairs, two full batches
+    // of each wavefront's loads and an LDS tile of about 25 KiB, so that six
+    // work-groups share a CU (256^3: 338 us at 12 lines, 342 at 11, 351 at
+    // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12, 66 at 20); fewer
+    // where that leaves compute units idle (128 x 256: 10.5 us at 4 lines,
+    // 12.4 at 16)
+    const int nch = (nx + 63) / 64;
+    int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(48 / nch, max(4, lj.nlines * nj / 256));
+    lpb = max(1, min(lpb, 64));
     if (sizeof(double) * (nx | 1) > 65536) return fail("x solver: nx = %d exceeds the LDS line tile", nx);
-    if ((size_t)lpb * (nx | 1) * sizeof(double) > 65536) lpb = (int)(65536 / (sizeof(double) * (nx | 1)));
-    const size_t shm = sizeof(double) * (size_t)lpb * (nx | 1);
+    const size_t row = sizeof(double) * (size_t)vofk::lines_stride(nx);   // at least ux's
+    if ((size_t)lpb * row > 65536) lpb = max(1, (int)(65536 / row));
+    const size_t shm = (size_t)lpb * row;
     const int ngroups = (lj.nlines + lpb - 1) / lpb;
     KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body, vofk::k_lines_lds,
         dim3((unsigned)ngroups, (unsigned)nj), dim3(vofk::kWThreads), shm, lj, lpb);
