@@ -1574,6 +1574,29 @@ static int pred_rows_for(const vof_ctx * ctx, int * xw) {
   return rt;
 }
 
+// the x-line solves of the nj fields of lj
+static int launch_lines(vof_ctx * ctx, vofk::LineJob & lj, int nj) {
+  const int nx = ctx->nx;
+  lj.inv_ny = 0xffffffffu / (unsigned)lj.ny + 1u;
+  // lines per work-group: 48 (line, 64-row chunk) pairs, two full batches
+  // of each wavefront's loads and an LDS tile of about 25 KiB, so that six
+  // work-groups share a CU (256^3: 338 us at 12 lines, 342 at 11, 351 at
+  // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12, 66 at 20); fewer
+  // where that leaves compute units idle (128 x 256: 10.5 us at 4 lines,
+  // 12.4 at 16)
+  const int nch = (nx + 63) / 64;
+  int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(48 / nch, max(4, lj.nlines * nj / 256));
+  lpb = max(1, min(lpb, 64));
+  if (sizeof(double) * (nx | 1) > 65536) return fail("x solver: nx = %d exceeds the LDS line tile", nx);
+  const size_t row = sizeof(double) * (size_t)vofk::lines_stride(nx);   // at least ux's
+  if ((size_t)lpb * row > 65536) lpb = max(1, (int)(65536 / row));
+  const size_t shm = (size_t)lpb * row;
+  const int ngroups = (lj.nlines + lpb - 1) / lpb;
+  KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body, vofk::k_lines_lds,
+      dim3((unsigned)ngroups, (unsigned)nj), dim3(vofk::kWThreads), shm, lj, lpb);
+  return 0;
+}
+
 static int predict_impl(const domain_t * domain, size_t rkstep, double dt, fluid_t * fluid,
                         const interface_t * interface, int fused, const double * vof_old = nullptr,
                         int images = 0, bool one_kernel = false) {
@@ -1637,7 +1660,6 @@ static int predict_impl(const domain_t * domain, size_t rkstep, double dt, fluid
   lj.ca = ca; lj.cb = cb; lj.cg = cg;
   lj.images = images;
   lj.nz = nz;
-  lj.inv_ny = 0xffffffffu / (unsigned)ny + 1u;
   if (vof_old) {
     vofk::FusedRhs fr{};
     fr.base = base;
@@ -1762,24 +1784,7 @@ static int predict_impl(const domain_t * domain, size_t rkstep, double dt, fluid
     F.n0 = kind == 0 ? nx + 1 : nx + 2;
     F.i0 = 1;
   }
-  {
-    // lines per work-group: 48 (line, 64-row chunk) pairs, two full batches
-    // of each wavefront's loads and an LDS tile of about 25 KiB, so that six
-    // work-groups share a CU (256^3: 338 us at 12 lines, 342 at 11, 351 at
-    // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12, 66 at 20); fewer
-    // where that leaves compute units idle (128 x 256: 10.5 us at 4 lines,
-    // 12.4 at 16)
-    const int nch = (nx + 63) / 64;
-    int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(48 / nch, max(4, lj.nlines * nj / 256));
-    lpb = max(1, min(lpb, 64));
-    if (sizeof(double) * (nx | 1) > 65536) return fail("x solver: nx = %d exceeds the LDS line tile", nx);
-    const size_t row = sizeof(double) * (size_t)vofk::lines_stride(nx);   // at least ux's
-    if ((size_t)lpb * row > 65536) lpb = max(1, (int)(65536 / row));
-    const size_t shm = (size_t)lpb * row;
-    const int ngroups = (lj.nlines + lpb - 1) / lpb;
-    KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body, vofk::k_lines_lds,
-        dim3((unsigned)ngroups, (unsigned)nj), dim3(vofk::kWThreads), shm, lj, lpb);
-  }
+  if (launch_lines(ctx, lj, nj)) return 1;
   if (images) return 0;
   for (int f = 0; f < nj; f++) {
     double * fld = (double *)jobs[f].field->data;
@@ -3492,12 +3497,7 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
           if (upload_tab(ctx, 0, rk, pm, &tx) || upload_tab(ctx, 1, rk, pm, &ty)) return 1;
           lj.f[0] = vofk::LineField{tx, nullptr, nullptr, nullptr, vx, qx, nx - 1, nx + 1, 1};
           lj.f[1] = vofk::LineField{ty, nullptr, nullptr, nullptr, vy, qy, nx, nx + 2, 1};
-          int lpb = (int)(32768 / (sizeof(double) * (nx | 1)));
-          lpb = lpb > 64 ? 64 : (lpb < 1 ? 1 : lpb);
-          const size_t shm = sizeof(double) * (size_t)lpb * (nx | 1);
-          hipLaunchKernelGGL(vofk::k_lines_lds, dim3((unsigned)((ny + lpb - 1) / lpb), 2), dim3(vofk::kWThreads), shm,
-                             st, lj, lpb);
-          LAUNCHCHK();
+          if (launch_lines(ctx, lj, 2)) return 1;
         }
         // R7 vof source (before anything else adds to lambda_vof)
         hipLaunchKernelGGL(vofa::ka_vof_src, gc, blk, 0, st, g, kRk[rk][0] * dt, kRk[rk][1] * dt,

@@ -197,3 +197,29 @@ def test_torch_autograd_binding(tmp_path):
         assert abs(ad - fd) <= 1e-6 * abs(fd), (ad, fd)
     finally:
         s.close()
+
+
+def test_adjoint_on_a_ragged_grid(tmp_path):
+    """70 x 60 cells: x lines that are no multiple of the line solver's 16-row
+    segments, more lines than one of its work-groups holds.  Central
+    differences of a loss of order 1 carry its rounding, about 1e-15, over
+    2 eps."""
+    ic = droplet_2d_divfree(nx=70, ny=60, radius=0.2, urms=0.05, nmodes=8, seed=3, We=10.0)
+    ref = sva.solver_from_ic(ic, str(tmp_path / "ref"))
+    try:
+        dts = [ref.integrate() for _ in range(3)]
+    finally:
+        ref.close()
+    s = sva.solver_from_ic(ic, str(tmp_path / "adj"))
+    try:
+        loss, gux, guy = s.adjoint_gradient(dts, every=2)
+        fr = Frozen(s, dts)
+        assert fr.loss0 == loss, (fr.loss0, loss)
+        rng = np.random.default_rng(7)
+        for d in range(4):
+            vx, vy = _unit_direction(ic, rng)
+            ad = float(gux @ vx + guy @ vy)
+            fd = fr.central(vx, vy, 1e-6)
+            assert abs(ad - fd) <= 1e-6 * abs(ad) + 1e-15 / 2e-6, (d, ad, fd)
+    finally:
+        s.close()
