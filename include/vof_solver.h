@@ -412,6 +412,8 @@ int vof_batch_autotune(vof_batch_t * batch, int steps, char * report, size_t len
  * partitions (segments of 2 .. 8 rows, one lane each, and a reduced system
  * of the segments' end rows) where 4 <= nx <= 256, 0 in sequence (this one
  * changes results by rounding only, a few 1e-14 relative to each line);
+ * where nx > 256 and the lines are few, 1 runs the sequential order with
+ * factors kept from domain_init, 0 forms them on each call (same results);
  * "fft_radix" = 16 (default: 256-point transforms on the register
  * radix-16 path) or 4 (every length on the mixed-radix 4/2/3/5 path; this
  * one changes results by rounding only, about 1e-16 relative);

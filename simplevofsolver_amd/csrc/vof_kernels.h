@@ -1426,6 +1426,10 @@ __device__ __forceinline__ SweepHead sweep_head(const double * tab, int n, int l
   return h;
 }
 
+// F32: the stored rows of both directions are rounded to float (a float2
+// spectrum), the recurrences carry unrounded values, as k_thomas_spec does;
+// for the singular line only (hd.flag 0: the back substitution starts from 0)
+template <bool F32 = false>
 __device__ __forceinline__ void lines_sweep_rows(const SweepHead & hd, const double * tab, int n, double * S, int ld,
                                                  int nl, int lane) {
   const int h = lane >> 4, l = lane & 15;
@@ -1465,6 +1469,10 @@ __device__ __forceinline__ void lines_sweep_rows(const SweepHead & hd, const dou
     for (int hh = 0; hh < hm; hh++) {
       if (h == hh) SweepRows<0>::fwd(x, tl, tv, prev);
       prev = rot_up(prev, h);
+    }
+    if constexpr (F32) {
+#pragma unroll
+      for (int u = 0; u < kSwRows / 2; u++) x[u] = make_double2((double)(float)x[u].x, (double)(float)x[u].y);
     }
     if (p + 1 < np) {
       store(p);
@@ -2171,107 +2179,6 @@ __global__ __launch_bounds__(64) void k_thomas_spec(int nx, int nlines, int nh, 
   k_thomas_spec_body<T2, U>(hw_block(), nx, nlines, nh, pl, pu, ey, ez, spec, vbuf, store_v);
 }
 
-// The elimination of k_thomas_spec for one whole line, both components by
-// one lane (per component the operations and their order are those of
-// k_thomas_spec with store_v; the gauge choice of its last row included).
-template <class T2>
-__device__ void thomas_line_seq(int n, int nlines, int line, double eval, const double * __restrict__ pl,
-                                const double * __restrict__ pu, T2 * __restrict__ spec, double * __restrict__ vbuf) {
-  T2 * q = spec + line;
-  double * v = vbuf + line;
-  const size_t st = (size_t)nlines;
-  double cc = -pl[0] - pu[0] + eval;
-  cc += pl[0];
-  double vprev = pu[0] / cc;
-  double2 qprev = to_d2(q[0]);
-  qprev.x = qprev.x / cc;
-  qprev.y = qprev.y / cc;
-  q[0] = from_d2<T2>(qprev);
-  v[0] = vprev;
-  for (int i = 1; i < n - 1; i++) {
-    const double c = -pl[i] - pu[i] + eval;
-    const double val = 1. / (c - pl[i] * vprev);
-    const double vi = val * (pu[i]);
-    double2 qi = to_d2(q[(size_t)i * st]);
-    qi.x = val * (qi.x - pl[i] * qprev.x);
-    qi.y = val * (qi.y - pl[i] * qprev.y);
-    q[(size_t)i * st] = from_d2<T2>(qi);
-    v[(size_t)i * st] = vi;
-    qprev = qi;
-    vprev = vi;
-  }
-  {
-    const int i = n - 1;
-    double c = -pl[i] - pu[i] + eval;
-    c += pu[i];
-    const double val = c - pl[i] * vprev;
-    double2 qi = to_d2(q[(size_t)i * st]);
-    const bool gauge = sizeof(T2) == sizeof(float2) && eval == 0.;
-    if (!gauge && fabs(val) > DBL_EPSILON) {
-      const double r = 1. / val;
-      qi.x = r * (qi.x - pl[i] * qprev.x);
-      qi.y = r * (qi.y - pl[i] * qprev.y);
-    } else {
-      qi = make_double2(0., 0.);
-    }
-    q[(size_t)i * st] = from_d2<T2>(qi);
-    qprev = qi;
-  }
-  for (int i = n - 2; i >= 0; i--) {
-    double2 qi = to_d2(q[(size_t)i * st]);
-    const double vi = v[(size_t)i * st];
-    qi.x -= vi * qprev.x;
-    qi.y -= vi * qprev.y;
-    q[(size_t)i * st] = from_d2<T2>(qi);
-    qprev = qi;
-  }
-}
-
-// The elimination of k_thomas_spec for one line staged in LDS (ql), both
-// components by one lane, with the line's factors given (tab: c0, rlast,
-// flag; val and v of rows 0 .. n-1 in vl, fl; the rows' lower coefficients
-// in pl): per component the operations of k_thomas_spec with the divisions
-// done in advance, its gauge choice for the last row included
-template <class T2>
-__device__ void thomas_line_tab(int n, const double * tab, const double * pl, const double * vl,
-                                const double * fl, double2 * ql) {
-  const double c0 = tab[0], rlast = tab[1];
-  const bool flag = tab[2] != 0.;
-  double2 qprev = ql[0];
-  qprev.x = qprev.x / c0;
-  qprev.y = qprev.y / c0;
-  ql[0] = to_d2(from_d2<T2>(qprev));
-#pragma unroll 4
-  for (int i = 1; i < n - 1; i++) {
-    double2 qi = ql[i];
-    qi.x = vl[i] * (qi.x - pl[i] * qprev.x);
-    qi.y = vl[i] * (qi.y - pl[i] * qprev.y);
-    ql[i] = to_d2(from_d2<T2>(qi));
-    qprev = qi;
-  }
-  {
-    const int i = n - 1;
-    double2 qi = ql[i];
-    const bool gauge = sizeof(T2) == sizeof(float2);
-    if (!gauge && flag) {
-      qi.x = rlast * (qi.x - pl[i] * qprev.x);
-      qi.y = rlast * (qi.y - pl[i] * qprev.y);
-    } else {
-      qi = make_double2(0., 0.);
-    }
-    ql[i] = to_d2(from_d2<T2>(qi));
-    qprev = qi;
-  }
-#pragma unroll 4
-  for (int i = n - 2; i >= 0; i--) {
-    double2 qi = ql[i];
-    qi.x -= fl[i] * qprev.x;
-    qi.y -= fl[i] * qprev.y;
-    ql[i] = to_d2(from_d2<T2>(qi));
-    qprev = qi;
-  }
-}
-
 // Partitioned x elimination of the spectrum: the tri-diagonal systems of
 // k_thomas_spec (solve_linear_systems, dft.c:364-395: c = -l - u + lambda,
 // Neumann folds in the first and last rows), solved in another order.  Each
@@ -2291,15 +2198,16 @@ __device__ void thomas_line_tab(int n, const double * tab, const double * pl, co
 // factors.  All systems but one are strictly diagonally dominant (lambda < 0),
 // so no pivoting is needed in either elimination; the results differ from
 // the sequential order's by rounding (a few 1e-14 of the line's largest
-// entry).  The (ky, kz) = (0, 0) line (lambda = 0) is singular, Neumann in
-// x; it keeps the sequential elimination and its choice of the constant: its
-// segment lanes stage the line in LDS, where one lane eliminates it while
-// the other lines solve their reduced systems, with the factors of that
-// line's sweep (stab, built once on the host by the same operations) staged
-// beside it (thomas_line_tab: no division left on the recurrence).  Only
-// line 0 has lambda = 0 (every other eigenvalue is negative), and it is line
-// t = 0 of the first work-group; a singular line elsewhere would take
-// thomas_line_seq on global memory.
+// entry).  The (ky, kz) = (0, 0) line (lambda = 0), Neumann in x, is singular;
+// it keeps the sequential elimination and its choice of the constant, with
+// the factors of that line's sweep built once on the host (stab, laid out as
+// the predictor's tables).  The first work-group does only that line: its
+// components are two lines of lines_sweep_rows.  No other line has lambda =
+// 0: every other eigenvalue is negative.
+// Latency-bound where the chip is not filled (128 x 256: 18.9 us with the
+// singular line swept by one lane among its work-group's other lines, 9.2 us
+// now; 256 x 256 2D 27 -> 13), by HBM at 256^3 (64.7 -> 60.7 us, a copy of the
+// spectrum takes 51).
 constexpr int kTpLines = 8;    // lines per work-group
 constexpr int kTpSeg = 32;     // segment lanes per line
 constexpr int kTpRows = 8;     // rows of the longest segment (nx <= 256)
@@ -2308,8 +2216,7 @@ template <class T2>
 __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, int nlines, int nh,
                                                    const double * __restrict__ pl, const double * __restrict__ pu,
                                                    const double * __restrict__ ey, const double * __restrict__ ez,
-                                                   const double * __restrict__ stab, T2 * __restrict__ spec,
-                                                   double * __restrict__ vbuf) {
+                                                   const double * __restrict__ stab, T2 * __restrict__ spec) {
   // the end rows of every segment: r1 (first row: lower, diagonal, upper,
   // right-hand side re, im), r2 (last row: lower, upper, right-hand side re,
   // im; its diagonal is 1).  Segments of a line are contiguous, lines 33
@@ -2317,18 +2224,42 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
   // reduction then publishes its rows in r1 and leaves each segment's x_s
   // and x_e (re, im) in r2.
   constexpr int RS = kTpSeg + 1;
-  __shared__ double r1s[5][kTpLines][RS];
-  __shared__ double r2s[4][kTpLines][RS];
-  __shared__ double2 sline[kTpSeg * kTpRows];   // the staged singular line
-  __shared__ double sval[kTpSeg * kTpRows];      // its factors and lower coefficients
-  __shared__ double sfac[kTpSeg * kTpRows];
-  __shared__ double spl[kTpSeg * kTpRows];
+  constexpr int kN1 = 5 * kTpLines * RS, kN2 = 4 * kTpLines * RS;
+  __shared__ __align__(16) double sh[kN1 + kN2];
+  double (&r1s)[5][kTpLines][RS] = *reinterpret_cast<double (*)[5][kTpLines][RS]>(sh);
+  double (&r2s)[4][kTpLines][RS] = *reinterpret_cast<double (*)[4][kTpLines][RS]>(sh + kN1);
   const int tid = (int)threadIdx.x;
-  const int t = tid % kTpLines, seg = tid / kTpLines;   // 8 consecutive lines per segment: 128-byte rows
-  const int line = (int)vb.x * kTpLines + t;
   const int n = nx;
+  const size_t st = (size_t)nlines;
+  if (vb.x == 0) {
+    // the singular line, in the same LDS (2 lines of 256 rows at most)
+    static_assert(2 * (kTpSeg * kTpRows + 2) <= kN1 + kN2, "the singular line does not fit");
+    const int ld = lines_stride(n);
+    SweepHead h;
+    if (tid < 64) h = sweep_head(stab, n, tid);
+    for (int e = tid; e < n; e += kTpLines * kTpSeg) {
+      const double2 v = to_d2(spec[(size_t)e * st]);
+      sh[e] = v.x;
+      sh[ld + e] = v.y;
+    }
+    // an FP32 spectrum is compatible to FP32 rounding only, which the last
+    // pivot would blow up: its line always takes the gauge branch
+    constexpr bool f32 = sizeof(T2) == sizeof(float2);
+    if (f32) h.flag = 0.;
+    lds_barrier();
+    if (tid < 64) lines_sweep_rows<f32>(h, stab, n, sh, ld, 2, tid);
+    lds_barrier();
+    for (int e = tid; e < n; e += kTpLines * kTpSeg) spec[(size_t)e * st] = from_d2<T2>(make_double2(sh[e], sh[ld + e]));
+    return;
+  }
+  const int t = tid % kTpLines, seg = tid / kTpLines;   // 8 consecutive lines per segment: 128-byte rows
+  VBlock rest = vb;   // the other groups, each XCD a contiguous run of lines
+  rest.x = vb.x - 1;
+  rest.gx = vb.gx - 1;
+  const int line0 = (int)xcd_tile(rest).x * kTpLines;
+  const int line = line0 + t;
   const int P = min(kTpSeg, n / 2);
-  const bool has_line = line < nlines;
+  const bool has_line = line > 0 && line < nlines;
   double eval = 0.;
   if (has_line) {
 #if NDIMS == 2
@@ -2338,30 +2269,9 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
     eval = ey[line % nh] + ez[line / nh];
 #endif
   }
-  const bool sing = eval == 0.;
-  const bool stage = has_line && sing && t == 0 && seg < P;   // rows of the staged singular line
-  // the work-group of the singular line (its line t = 0) stages its factors
-  {
-    const int l0 = (int)vb.x * kTpLines;
-    bool wsing = false;
-    if (l0 < nlines) {
-#if NDIMS == 2
-      wsing = ey[l0 % nh] == 0.;
-#else
-      wsing = ey[l0 % nh] + ez[l0 / nh] == 0.;
-#endif
-    }
-    if (wsing)
-      for (int e = tid; e < n; e += kTpLines * kTpSeg) {
-        sval[e] = stab[3 + e];
-        sfac[e] = stab[3 + n + e];
-        spl[e] = pl[e];
-      }
-  }
-  const bool act = has_line && !sing && seg < P;
+  const bool act = has_line && seg < P;
   const int s = seg * n / P, e = (seg + 1) * n / P - 1;
   const int m = e - s + 1;
-  const size_t st = (size_t)nlines;
   T2 * __restrict__ q = spec + line;
   // row i of the line: lower, diagonal and upper coefficients (the folds
   // as in k_thomas_spec; no lower entry in row 0, no upper in row n - 1)
@@ -2381,11 +2291,6 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
   double A[kTpRows], C[kTpRows];
   double2 D[kTpRows];
   double2 xs = make_double2(0., 0.), xe = make_double2(0., 0.);
-  if (stage) {
-#pragma unroll
-    for (int r = 0; r < kTpRows; r++)
-      if (r < m) sline[s + r] = to_d2(q[(size_t)(s + r) * st]);
-  }
   if (act) {
 #pragma unroll
     for (int r = 0; r < kTpRows; r++)
@@ -2455,9 +2360,8 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
     r2s[3][t][seg] = de.y;
   }
   __syncthreads();
-  if (tid == 0 && has_line && sing) thomas_line_tab<T2>(n, stab, spl, sval, sfac, sline);
-  // the reduced system of a line, one wavefront per two lines (lanes 0-31
-  // line 2w, 32-63 line 2w + 1; lane k for segment k).  Segment k's rows
+  // the reduced system of a line, one wavefront per two lines, lane k of 32
+  // for segment k.  Segment k's rows
   //   r1:  l1 x_e(k-1) + d1 x_s(k) + u1 x_e(k) = r1
   //   r2:  a2 x_s(k) + x_e(k) + c2 x_s(k+1) = r2
   // with x_s(k) and x_s(k+1) taken from the r1 rows of segments k and k + 1
@@ -2471,18 +2375,8 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
   // barrier: the wavefront-scope fences only keep the compiler from moving
   // one step's reads across the previous step's writes.
   {
-    const int lw = tid & 63;
-    const int tl = 2 * (tid >> 6) + (lw >> 5);
-    const int k = lw & 31;
-    const int lr = (int)vb.x * kTpLines + tl;
-    bool on = false;
-    if (lr < nlines && k < P) {
-#if NDIMS == 2
-      on = ey[lr % nh] != 0.;
-#else
-      on = ey[lr % nh] + ez[lr / nh] != 0.;
-#endif
-    }
+    const int tl = tid / kTpSeg, k = tid % kTpSeg;
+    const bool on = line0 + tl > 0 && line0 + tl < nlines && k < P;
     double l1 = 0., d1 = 1., u1 = 0., q1x = 0., q1y = 0.;
     double own[5] = {0., 1., 0., 0., 0.};
     double rd = 1.;
@@ -2583,23 +2477,211 @@ __device__ __forceinline__ void k_thomas_part_body(const VBlock & vb, int nx, in
     }
     q[(size_t)e * st] = from_d2<T2>(xe);
   }
-  if (stage) {
-#pragma unroll
-    for (int r = 0; r < kTpRows; r++)
-      if (r < m) q[(size_t)(s + r) * st] = from_d2<T2>(sline[s + r]);
-  }
-  if (has_line && sing && t != 0 && seg == 0) thomas_line_seq<T2>(n, nlines, line, eval, pl, pu, spec, vbuf);
 }
 
 template <class T2>
 __global__ __launch_bounds__(kTpLines * kTpSeg) void k_thomas_part(int nx, int nlines, int nh,
-                                                                    const double * __restrict__ pl,
-                                                                    const double * __restrict__ pu,
-                                                                    const double * __restrict__ ey,
-                                                                    const double * __restrict__ ez,
-                                                                    const double * __restrict__ stab,
-                                                                    T2 * __restrict__ spec, double * __restrict__ vbuf) {
-  k_thomas_part_body<T2>(hw_block(), nx, nlines, nh, pl, pu, ey, ez, stab, spec, vbuf);
+                                                                 const double * __restrict__ pl,
+                                                                 const double * __restrict__ pu,
+                                                                 const double * __restrict__ ey,
+                                                                 const double * __restrict__ ez,
+                                                                 const double * __restrict__ stab,
+                                                                 T2 * __restrict__ spec) {
+  k_thomas_part_body<T2>(hw_block(), nx, nlines, nh, pl, pu, ey, ez, stab, spec);
+}
+
+// The sequential elimination of k_thomas_spec where the lines are too few to
+// fill the chip (2D: ny / 2 + 1 of them), with its factors built once per grid
+// by the same operations (k_thomas_fac; they depend on the grid alone).  One
+// wavefront runs 8 lines, the components being 16 systems, as lines_sweep_rows
+// does: lane 16 h + s holds rows 128 p + 32 h .. + 31 of system s in pass p.
+// The spectrum's 8 lines are one 128-byte row per x, so a pass loads straight
+// into that layout, one pass ahead.  Per component the operations and their
+// order are those of k_thomas_spec.  Latency-bound by the serial rows: 513
+// lines of 512 rows 140.6 -> 28.2 us (16 rows per lane 37.2, 32 rows with
+// every address formed on its own 35.2).  With the chip full it loses to
+// k_thomas_spec, which moves 8 B per row less: 33024 lines of 512 float2 rows
+// 255 against 194 us.
+//   rec[i][line]: c0 (row 0), 1 / (c - l v[i-1]), last row 0 where singular
+//   v[i][line]
+__global__ __launch_bounds__(64) void k_thomas_fac(int n, int nlines, int nh, const double * __restrict__ pl,
+                                                   const double * __restrict__ pu, const double * __restrict__ ey,
+                                                   const double * __restrict__ ez, double * __restrict__ rec,
+                                                   double * __restrict__ v) {
+  const int line = (int)(blockIdx.x * 64 + threadIdx.x);
+  if (line >= nlines) return;
+#if NDIMS == 2
+  const double eval = ey[line];
+  (void)ez;
+  (void)nh;
+#else
+  const double eval = ey[line % nh] + ez[line / nh];
+#endif
+  const size_t st = (size_t)nlines;
+  rec += line;
+  v += line;
+  double cc = -pl[0] - pu[0] + eval;
+  cc += pl[0];
+  double vprev = pu[0] / cc;
+  rec[0] = cc;
+  v[0] = vprev;
+  for (int i = 1; i < n - 1; i++) {
+    const double c = -pl[i] - pu[i] + eval;
+    const double val = 1. / (c - pl[i] * vprev);
+    vprev = val * (pu[i]);
+    rec[(size_t)i * st] = val;
+    v[(size_t)i * st] = vprev;
+  }
+  double c = -pl[n - 1] - pu[n - 1] + eval;
+  c += pu[n - 1];
+  const double val = c - pl[n - 1] * vprev;
+  rec[(size_t)(n - 1) * st] = fabs(val) > DBL_EPSILON ? 1. / val : 0.;
+  v[(size_t)(n - 1) * st] = 0.;
+}
+
+constexpr int kSeqRows = 32;   // rows per lane and pass
+// rows R .. kSeqRows - 1 forward, with each lane's own factors f
+template <int R>
+struct SeqRows {
+  static __device__ __forceinline__ void fwd(double * x, const double * f, const double * tl, double & prev) {
+    if constexpr (R < kSeqRows) {
+      x[R] = f[R] * (x[R] - row_lane<R & 15>(tl[R >> 4]) * prev);
+      prev = x[R];
+      SeqRows<R + 1>::fwd(x, f, tl, prev);
+    }
+  }
+};
+
+constexpr int kSeqLines = 8;   // lines per wavefront
+template <class T2>
+__device__ __forceinline__ void k_thomas_seq_body(const VBlock & vb, int n, int nlines, const double * __restrict__ pl,
+                                                  const double * __restrict__ rec, const double * __restrict__ v,
+                                                  T2 * __restrict__ spec) {
+  using S = typename Cx<T2>::S;
+  const int lane = (int)threadIdx.x, h = lane >> 4, s = lane & 15;
+  const int c0 = (int)vb.x * 2 * kSeqLines;            // first component system
+  const bool act = c0 + s < 2 * nlines;
+  const int sys = min(c0 + s, 2 * nlines - 1), line = sys >> 1;
+  S * __restrict__ q = reinterpret_cast<S *>(spec);
+  const size_t st = (size_t)nlines, sq = 2 * st;   // rows apart
+  const int nseg = (n + kSeqRows - 1) / kSeqRows, np = (nseg + 3) >> 2, last = n - 1;
+  double x[kSeqRows], f[kSeqRows], prev = 0.;
+  S xn[kSeqRows];
+  double fn[kSeqRows];
+  // whole passes address a lane's first row once (32-bit lane offsets: the
+  // host checks that the spectrum has fewer than 2^32 bytes) and step by a
+  // uniform stride; the last pass clamps its rows
+  auto load = [&](int p, const double * __restrict__ fac) {
+    const int row0 = kSeqRows * (4 * p + h);
+    if (4 * kSeqRows * (p + 1) <= n) {
+      const unsigned oq = (unsigned)row0 * (unsigned)sq + (unsigned)sys, of = (unsigned)row0 * (unsigned)st + (unsigned)line;
+#pragma unroll
+      for (int r = 0; r < kSeqRows; r++) {
+        xn[r] = (q + (size_t)r * sq)[oq];
+        fn[r] = (fac + (size_t)r * st)[of];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < kSeqRows; r++) {
+        const unsigned row = (unsigned)min(row0 + r, last);
+        xn[r] = q[row * (unsigned)sq + (unsigned)sys];
+        fn[r] = fac[row * (unsigned)st + (unsigned)line];
+      }
+    }
+  };
+  auto take = [&](bool data) {
+#pragma unroll
+    for (int r = 0; r < kSeqRows; r++) {
+      if (data) x[r] = (double)xn[r];
+      f[r] = fn[r];
+    }
+  };
+  auto store = [&](int p) {
+    const int row0 = kSeqRows * (4 * p + h);
+    const unsigned oq = (unsigned)row0 * (unsigned)sq + (unsigned)sys;
+    if (!act) return;
+    if (4 * kSeqRows * (p + 1) <= n) {
+#pragma unroll
+      for (int r = 0; r < kSeqRows; r++) (q + (size_t)r * sq)[oq] = (S)x[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < kSeqRows; r++)
+        if (row0 + r < n) (q + (size_t)r * sq)[oq] = (S)x[r];
+    }
+  };
+  const double cc = rec[line];
+  // an FP32 spectrum is compatible to FP32 rounding only: its singular line
+  // (0, 0) always takes the gauge branch
+  const bool flag = rec[(size_t)last * st + line] != 0. && !(sizeof(T2) == sizeof(float2) && line == 0);
+  load(0, rec);
+  double tl[kSeqRows / 16], tn[kSeqRows / 16];
+  auto load_l = [&](int p, double * l) {
+#pragma unroll
+    for (int k = 0; k < kSeqRows / 16; k++) l[k] = pl[min(kSeqRows * (4 * p + h) + 16 * k + s, last)];
+  };
+  load_l(0, tl);
+  for (int p = 0; p < np; p++) {
+    take(true);
+    if (p + 1 < np) {
+      load(p + 1, rec);
+      load_l(p + 1, tn);
+    } else {
+      load(p, v);   // the last pass stays in registers: only its factors are used
+    }
+    if (p == 0) {
+      const double d = x[0] / cc;
+      x[0] = h == 0 ? d : x[0];
+      f[0] = h == 0 ? 1. : f[0];
+      if (lane == 0) tl[0] = 0.;
+    }
+    const int hm = min(4, nseg - 4 * p);
+    for (int hh = 0; hh < hm; hh++) {
+      if (h == hh) SeqRows<0>::fwd(x, f, tl, prev);
+      prev = rot_up(prev, h);
+    }
+    if (p + 1 < np) store(p);
+#pragma unroll
+    for (int k = 0; k < kSeqRows / 16; k++) tl[k] = tn[k];
+  }
+  // the stored forward values are what the back substitution reads; it
+  // starts from the last row's unrounded one
+  {
+    const int top = last - kSeqRows * (4 * (np - 1) + h);
+#pragma unroll
+    for (int r = 0; r < kSeqRows; r++) x[r] = r == top ? x[r] : (double)(S)x[r];
+  }
+  for (int p = np - 1; p >= 0; p--) {
+    take(p + 1 < np);
+    if (p > 0) load(p - 1, v);
+    for (int hh = min(4, nseg - 4 * p) - 1; hh >= 0; hh--) {
+      const int top = last - kSeqRows * (4 * p + hh);   // the last row within this segment, or past it
+      if (h == hh) {
+        if (top < kSeqRows) {
+#pragma unroll
+          for (int r = kSeqRows - 1; r >= 0; r--) {
+            const double a = x[r] - f[r] * prev;
+            x[r] = r < top ? a : flag ? x[r] : 0.;
+            prev = x[r];
+          }
+        } else {
+#pragma unroll
+          for (int r = kSeqRows - 1; r >= 0; r--) {
+            x[r] -= f[r] * prev;
+            prev = x[r];
+          }
+        }
+      }
+      prev = rot_dn(prev, h);
+    }
+    store(p);
+  }
+}
+
+template <class T2>
+__global__ __launch_bounds__(64) void k_thomas_seq(int n, int nlines, const double * __restrict__ pl,
+                                                   const double * __restrict__ rec, const double * __restrict__ v,
+                                                   T2 * __restrict__ spec) {
+  k_thomas_seq_body<T2>(hw_block(), n, nlines, pl, rec, v, spec);
 }
 
 // inverse real transform in y (c2r: the imaginary parts of the k = 0 and

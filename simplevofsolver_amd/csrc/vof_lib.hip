@@ -269,7 +269,7 @@ struct vof_ctx {
   double * d_pu;
   double * d_ey;                         // eigenvalues in y, z (dft.c:263-291)
   double * d_ez;
-  double * d_stab;                       // factors of the (0, 0) line: c0, rlast, flag, val[nx], v[nx]
+  double * d_stab;                       // factors of the (0, 0) line: c0, rlast, flag, -, l[nx], val[nx], v[nx]
   double2 * d_spec;
   // mixed-precision Poisson (refinements < 0: plain FP64)
   int poisson_refine;
@@ -277,6 +277,7 @@ struct vof_ctx {
   float2 * d_twy32;
   float2 * d_twz32;
   double * d_vbuf;
+  double * d_rec;              // reciprocal pivots of k_thomas_seq (null: it does not run)
   bool vbuf_ready;             // the Thomas back-substitution factors are in d_vbuf
   // scratch
   double * d_delta;                      // x1 pencil of increments
@@ -942,6 +943,11 @@ static std::vector<double2> make_twiddles(int n) {
 // ---------------------------------------------------------------------------
 // domain
 
+// lines few enough for k_thomas_seq (8 lines per wavefront): up to two
+// wavefronts per SIMD (513 lines of 512 rows: 28 us against 141 for
+// k_thomas_spec; 33024 lines 255 against 194)
+static bool thomas_seq_lines(size_t nlines) { return nlines <= 16384; }
+
 static int ctx_create(domain_t * domain) {
   vof_ctx * ctx = new vof_ctx();
   domain->info = ctx;
@@ -1073,20 +1079,22 @@ static int ctx_create(domain_t * domain) {
     // elimination factors of the (ky, kz) = (0, 0) line, whose eigenvalue is
     // 0 in every step: the operations of k_thomas_spec's sweep for it, once
     // (the partitioned solve eliminates that line with them)
-    std::vector<double> st(3 + 2 * (size_t)nx, 0.);
+    std::vector<double> st(4 + 3 * (size_t)nx, 0.);
     if (nx >= 2) {
       const double eval = 0.;
       double cc = -l[0] - u[0] + eval;
       cc += l[0];
       st[0] = cc;
       double vprev = u[0] / cc;
-      st[3 + nx] = vprev;
+      double * L = &st[4], * VAL = L + nx, * V = VAL + nx;
+      for (int i = 0; i < nx; i++) L[i] = l[i];
+      V[0] = vprev;
       for (int i = 1; i < nx - 1; i++) {
         const double c = -l[i] - u[i] + eval;
         const double val = 1. / (c - l[i] * vprev);
         const double vi = val * (u[i]);
-        st[3 + i] = val;
-        st[3 + nx + i] = vi;
+        VAL[i] = val;
+        V[i] = vi;
         vprev = vi;
       }
       const int i = nx - 1;
@@ -1095,6 +1103,7 @@ static int ctx_create(domain_t * domain) {
       const double val = c - l[i] * vprev;
       st[2] = fabs(val) > DBL_EPSILON ? 1. : 0.;
       st[1] = st[2] != 0. ? 1. / val : 0.;
+      VAL[nx - 1] = st[1];
     }
     HIPCHK(hipMalloc(&ctx->d_stab, sizeof(double) * st.size()));
     HIPCHK(hipMemcpy(ctx->d_stab, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice));
@@ -1146,6 +1155,15 @@ static int ctx_create(domain_t * domain) {
   HIPCHK(hipMalloc(&ctx->d_spec, sizeof(double2) * nx * nline));
   HIPCHK(hipMalloc(&ctx->d_vbuf, sizeof(double) * nx * nline));
   ctx->vbuf_ready = false;
+  ctx->d_rec = nullptr;
+  if (nx > 256 && thomas_seq_lines(nline) && sizeof(double2) * nx * nline < ((size_t)1 << 32)) {
+    HIPCHK(hipMalloc(&ctx->d_rec, sizeof(double) * nx * nline));
+    hipLaunchKernelGGL(vofk::k_thomas_fac, dim3((unsigned)((nline + 63) / 64)), dim3(64), 0, ctx->stream, nx, (int)nline,
+                       ctx->nh, (const double *)ctx->d_pl, (const double *)ctx->d_pu, (const double *)ctx->d_ey,
+                       (const double *)ctx->d_ez, ctx->d_rec, ctx->d_vbuf);
+    LAUNCHCHK();
+    ctx->vbuf_ready = true;
+  }
   HIPCHK(hipMalloc(&ctx->d_delta, sizeof(double) * ncell * (NDIMS + 1)));
   ctx->npart = 8192;
   HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * ctx->npart * vofk::kDiagN));
@@ -1229,7 +1247,7 @@ extern "C" int domain_finalise(domain_t * domain) {
     dev_free(ctx->d_twy); if (ctx->d_twz) dev_free(ctx->d_twz);
     dev_free(ctx->d_pl); dev_free(ctx->d_pu); dev_free(ctx->d_ey); dev_free(ctx->d_ez); dev_free(ctx->d_stab);
     dev_free(ctx->d_spec32); dev_free(ctx->d_twy32); dev_free(ctx->d_twz32);
-    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_delta); dev_free(ctx->d_part);
+    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_rec); dev_free(ctx->d_delta); dev_free(ctx->d_part);
     if (ctx->d_vof_spare) dev_free(ctx->d_vof_spare);
     for (int m = 0; m < 4; m++) dev_free(ctx->d_fspare[m]);
     for (void * b : ctx->freeze_slots) dev_free(b);
@@ -1812,16 +1830,26 @@ extern "C" int fluid_predict_field(const domain_t * domain, const size_t rkstep,
 // images and Neumann walls (the residual reads them)
 // x eliminations of the spectrum: the partitioned solve (k_thomas_part, one
 // lane per segment of 2 .. 8 rows) for 4 <= nx <= 256 unless thomas_part is
-// 0, else k_thomas_spec with ctx->thomas_rows rows per prefetched chunk (the
-// arithmetic does not depend on it)
+// 0; for longer lines the sequential one, by k_thomas_seq with factors kept
+// from the grid's creation where the lines are few (thomas_seq_lines), else
+// (and with thomas_part 0) by k_thomas_spec with ctx->thomas_rows rows per
+// prefetched chunk (the same values bit for bit)
 template <class T2>
 static int launch_thomas(vof_ctx * ctx, const char * name, T2 * spec, int nlines) {
+  constexpr bool f32 = sizeof(T2) == sizeof(float2);
   if (ctx->thomas_part && ctx->nx >= 4 && ctx->nx <= 256) {
-    // timing label of the kernel that runs
-    const char * pname = sizeof(T2) == sizeof(float2) ? "k_thomas_part32" : "k_thomas_part";
-    const dim3 g((unsigned)((nlines + vofk::kTpLines - 1) / vofk::kTpLines)), b(vofk::kTpLines * vofk::kTpSeg);
+    // timing label of the kernel that runs; the first work-group does the
+    // singular line
+    const char * pname = f32 ? "k_thomas_part32" : "k_thomas_part";
+    const dim3 g(1u + (unsigned)((nlines + vofk::kTpLines - 1) / vofk::kTpLines)), b(vofk::kTpLines * vofk::kTpSeg);
     KLB(ctx, pname, vofk::kTpLines * vofk::kTpSeg, (vofk::k_thomas_part_body<T2>), (vofk::k_thomas_part<T2>), g, b, 0,
-        ctx->nx, nlines, ctx->nh, ctx->d_pl, ctx->d_pu, ctx->d_ey, ctx->d_ez, ctx->d_stab, spec, ctx->d_vbuf);
+        ctx->nx, nlines, ctx->nh, ctx->d_pl, ctx->d_pu, ctx->d_ey, ctx->d_ez, ctx->d_stab, spec);
+    return 0;
+  }
+  if (ctx->thomas_part && ctx->d_rec) {
+    const dim3 g((unsigned)((nlines + vofk::kSeqLines - 1) / vofk::kSeqLines));
+    KLB(ctx, f32 ? "k_thomas_seq32" : "k_thomas_seq", 64, (vofk::k_thomas_seq_body<T2>), (vofk::k_thomas_seq<T2>), g,
+        dim3(64), 0, ctx->nx, nlines, ctx->d_pl, (const double *)ctx->d_rec, (const double *)ctx->d_vbuf, spec);
     return 0;
   }
   // two lanes per line (real and imaginary parts)
@@ -3459,17 +3487,7 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
                              dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y, (const double2 *)ctx->d_twy,
                              (const double *)b, 1. / (double)ny, ctx->d_spec);
         }
-        if (ctx->thomas_part && nx >= 4 && nx <= 256) {
-          hipLaunchKernelGGL(vofk::k_thomas_part<double2>, dim3((ctx->nh + vofk::kTpLines - 1) / vofk::kTpLines),
-                             dim3(vofk::kTpLines * vofk::kTpSeg), 0, st, nx, ctx->nh, ctx->nh,
-                             (const double *)ctx->d_pl, (const double *)ctx->d_pu, (const double *)ctx->d_ey,
-                             (const double *)ctx->d_ez, (const double *)ctx->d_stab, ctx->d_spec, ctx->d_vbuf);
-        } else {
-          hipLaunchKernelGGL(vofk::k_thomas_spec<double2>, dim3((2 * ctx->nh + 63) / 64), dim3(64), 0, st, nx, ctx->nh,
-                             ctx->nh, (const double *)ctx->d_pl, (const double *)ctx->d_pu,
-                             (const double *)ctx->d_ey, (const double *)ctx->d_ez, ctx->d_spec, ctx->d_vbuf,
-                             vbuf_store(ctx));
-        }
+        if (launch_thomas<double2>(ctx, "k_thomas_spec", ctx->d_spec, ctx->nh)) return 1;
         if (use1024) {
           hipLaunchKernelGGL(vofk::k_irfft_y_psi<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y,
                              (const double2 *)ctx->d_twy, (const double2 *)ctx->d_spec, x, 1);
