@@ -283,6 +283,7 @@ struct vof_ctx {
   double * d_delta;                      // x1 pencil of increments
   double * d_part;
   int npart;
+  unsigned * d_ticket;                   // work-groups of k_dt_partial that have finished
   double * h_scalar;                     // pinned
   // statistics accumulators (statistics.c), allocated by statistics.init
   double * d_stat[9];
@@ -542,10 +543,6 @@ struct vof_batch {
   double * h_tab;
   double * d_tab;
   size_t tab_doubles;
-  // dt gather
-  double * d_dt;
-  double * h_dt;
-  const double ** d_dt_src;
   // a batch of 8 cases or more is 2 batches of alternate cases (4 from 16
   // cases on: case c in part c % 4), each with its own stream, tables and
   // graphs, stepped in turn: while the host reads one part's dt and records
@@ -1167,6 +1164,8 @@ static int ctx_create(domain_t * domain) {
   HIPCHK(hipMalloc(&ctx->d_delta, sizeof(double) * ncell * (NDIMS + 1)));
   ctx->npart = 8192;
   HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * ctx->npart * vofk::kDiagN));
+  HIPCHK(hipMalloc(&ctx->d_ticket, sizeof(unsigned)));
+  HIPCHK(hipMemset(ctx->d_ticket, 0, sizeof(unsigned)));
   HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * 64));
   // Thomas tables: header 4 + l, val, v
   ctx->tab_stride = 4 + 3 * (size_t)nx;
@@ -1247,7 +1246,7 @@ extern "C" int domain_finalise(domain_t * domain) {
     dev_free(ctx->d_twy); if (ctx->d_twz) dev_free(ctx->d_twz);
     dev_free(ctx->d_pl); dev_free(ctx->d_pu); dev_free(ctx->d_ey); dev_free(ctx->d_ez); dev_free(ctx->d_stab);
     dev_free(ctx->d_spec32); dev_free(ctx->d_twy32); dev_free(ctx->d_twz32);
-    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_rec); dev_free(ctx->d_delta); dev_free(ctx->d_part);
+    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_rec); dev_free(ctx->d_delta); dev_free(ctx->d_part); dev_free(ctx->d_ticket);
     if (ctx->d_vof_spare) dev_free(ctx->d_vof_spare);
     for (int m = 0; m < 4; m++) dev_free(ctx->d_fspare[m]);
     for (void * b : ctx->freeze_slots) dev_free(b);
@@ -1414,6 +1413,9 @@ static int decide_dt_enqueue(vof_ctx * ctx, const fluid_t * fluid) {
   const unsigned gx = (unsigned)((ctx->nx + 63) / 64);
   unsigned gy = (unsigned)((ctx->ny + 3) / 4);
   unsigned gz = NDIMS == 3 ? (unsigned)((ctx->nz + 15) / 16) : 1u;
+  if (NDIMS == 2) gy = min(gy, max(1u, 128u / gx));
+  if (NDIMS == 3 && ctx->rec)
+    while (gz > 1 && gx * gy * gz > 256u) gz--;
   while (gz > 1 && (size_t)gx * gy * gz > (size_t)ctx->npart) gz--;
   while (gy > 1 && (size_t)gx * gy * gz > (size_t)ctx->npart) gy--;
   if ((size_t)gx * gy * gz > (size_t)ctx->npart) return fail("decide_dt: %u x-tiles exceed the partial buffer", gx);
@@ -1423,15 +1425,19 @@ static int decide_dt_enqueue(vof_ctx * ctx, const fluid_t * fluid) {
 #else
   const double * uz = nullptr;
 #endif
+  // up to 256 work-groups the last to finish reduces their minima (every one
+  // takes a ticket from one counter); more of them, which only large 3D grids
+  // have, are reduced by k_min_final.  Either writes the minimum to pinned
+  // host memory: the stream's synchronisation makes it visible, and no copy
+  // is queued.  The cases of a batch record the same launches whatever their
+  // sizes
+  const bool one = nb <= 256 || ctx->rec;
   KLB(ctx, "k_dt_partial", vofk::kRedThreads, vofk::k_dt_partial_body, vofk::k_dt_partial, dim3(gx, gy, gz),
       dim3(vofk::kRedThreads), 0, ctx->grid, (const double *)fluid->ux.data, (const double *)fluid->uy.data,
-      uz, ctx->d_part);
-  KLB(ctx, "k_min_final", vofk::kRedThreads, vofk::k_min_final_body, vofk::k_min_final, dim3(1),
-      dim3(vofk::kRedThreads), 0, (const double *)ctx->d_part, nb, ctx->d_part + ctx->npart);
-  // a batch gathers the minima of all its cases itself
-  if (!ctx->rec)
-    HIPCHK(hipMemcpyAsync(ctx->h_scalar, ctx->d_part + ctx->npart, sizeof(double),
-                          hipMemcpyDeviceToHost, ctx->stream));
+      uz, ctx->d_part, one ? ctx->d_ticket : nullptr, ctx->h_scalar);
+  if (!one)
+    KLB(ctx, "k_min_final", vofk::kRedThreads, vofk::k_min_final_body, vofk::k_min_final, dim3(1),
+        dim3(vofk::kRedThreads), 0, (const double *)ctx->d_part, nb, ctx->h_scalar);
   return 0;
 }
 
@@ -2536,11 +2542,6 @@ extern "C" int vof_set_poisson_mixed(domain_t * domain, int refinements) {
 // ---------------------------------------------------------------------------
 // batch of cases advanced together (see "Batched execution" above)
 
-__global__ void k_gather_dt(const double * const * __restrict__ src, int n, double * __restrict__ dst) {
-  const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (c < n) dst[c] = *src[c];
-}
-
 static void batch_drop_graph(vof_batch * B, int ph) {
   if (B->gexec[ph]) (void)hipGraphExecDestroy(B->gexec[ph]);
   B->gexec[ph] = nullptr;
@@ -2572,13 +2573,13 @@ struct BatchGroup {
   std::vector<int> cases;
 };
 
-// phase ph of the step: `pre` and `post` enqueue the phase's other copies
-// and launches (Thomas tables before a stage; the dt gather after phase 0).
+// phase ph of the step: `pre` enqueues the phase's other copies (the Thomas
+// tables of a stage).
 // With graphs on, the whole phase is captured once and replayed while its
 // signature (groups, kernel instantiations, grids, table offsets, staging
 // buffers) is unchanged; the argument tables themselves are refilled on the
 // host every step and copied by the graph's first node.
-static int batch_run(vof_batch * B, int ph, const std::function<int()> & pre, const std::function<int()> & post) {
+static int batch_run(vof_batch * B, int ph, const std::function<int()> & pre) {
   const size_t n = B->ctx.size();
   const size_t nrec = B->rec[0].recs.size();
   for (size_t c = 1; c < n; c++) {
@@ -2622,7 +2623,7 @@ static int batch_run(vof_batch * B, int ph, const std::function<int()> & pre, co
       if (r0.merge(B, groups[q].r, groups[q].cases, nullptr, B->d_stage[ph] + off[q]) == 0)
         return fail("batch: launch of %s failed", r0.name);
     }
-    return post ? post() : 0;
+    return 0;
   };
   if (!B->graphs) {
     if (enqueue()) return 1;
@@ -2708,13 +2709,11 @@ static int batch_create_one(int ncases, const domain_t * const domains[], fluid_
   tab = B->tab_doubles;
   if (hipHostMalloc(&B->h_tab, sizeof(double) * tab) != hipSuccess || hipMalloc(&B->d_tab, sizeof(double) * tab) != hipSuccess)
     rc = fail("vof_batch_create: table allocation failed");
-  std::vector<const double *> src(ncases);
   for (int c = 0; c < ncases && !rc; c++) {
     vof_ctx * ctx = B->ctx[c];
     rc = ensure_vof_spare(ctx, B->interface[c]);
     if (!rc && (ctx->fuse & F_PRED)) rc = ensure_field_spares(ctx, B->fluid[c]);
     if (!rc && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = fail("vof_batch_create: case stream failed");
-    src[c] = ctx->d_part + ctx->npart;
   }
   if (!rc) {
     size_t o = 0;
@@ -2727,11 +2726,6 @@ static int batch_create_one(int ncases, const domain_t * const domains[], fluid_
       ctx->tab_shared = true;
       o += ctx->tab_stride * 4;
     }
-    if (hipMalloc(&B->d_dt, sizeof(double) * ncases) != hipSuccess ||
-        hipHostMalloc(&B->h_dt, sizeof(double) * ncases) != hipSuccess ||
-        hipMalloc(&B->d_dt_src, sizeof(double *) * ncases) != hipSuccess ||
-        hipMemcpy(B->d_dt_src, src.data(), sizeof(double *) * ncases, hipMemcpyHostToDevice) != hipSuccess)
-      rc = fail("vof_batch_create: dt buffers failed");
   }
   if (rc) {
     vof_batch_destroy(B);
@@ -2819,7 +2813,8 @@ extern "C" int vof_batch_integrate(vof_batch_t * B, double dts[]) {
       }
     return 0;
   };
-  // dt of every case (decide_dt.c:104-145): batched reductions, one copy back
+  // dt of every case (decide_dt.c:104-145): batched reductions, each into its
+  // case's pinned scalar
   B->pool.run((int)n, [&](int c) {
     B->rec[c].recs.clear();
     B->ctx[c]->rec = &B->rec[c];
@@ -2828,18 +2823,10 @@ extern "C" int vof_batch_integrate(vof_batch_t * B, double dts[]) {
     if (rcs[c]) errs[c] = g_err;
   });
   if (gather_rc()) return 1;
-  auto gather = [&]() -> int {
-    hipLaunchKernelGGL(k_gather_dt, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, B->stream,
-                       (const double * const *)B->d_dt_src, (int)n, B->d_dt);
-    LAUNCHCHK();
-    HIPCHK(hipMemcpyAsync(B->h_dt, B->d_dt, sizeof(double) * n, hipMemcpyDeviceToHost, B->stream));
-    return 0;
-  };
-  if (batch_run(B, 0, nullptr, gather)) return 1;
+  if (batch_run(B, 0, nullptr)) return 1;
   HIPCHK(hipStreamSynchronize(B->stream));
   std::vector<double> dt(n);
   for (size_t c = 0; c < n; c++) {
-    B->ctx[c]->h_scalar[0] = B->h_dt[c];
     if (decide_dt_finish(B->ctx[c], B->domain[c], B->fluid[c], &dt[c], false)) return 1;
   }
   // the RK stages of every case, recorded then merged stage by stage: the
@@ -2859,7 +2846,7 @@ extern "C" int vof_batch_integrate(vof_batch_t * B, double dts[]) {
                             hipMemcpyHostToDevice, B->stream));
       return 0;
     };
-    if (batch_run(B, (int)rk + 1, tables, nullptr)) return 1;
+    if (batch_run(B, (int)rk + 1, tables)) return 1;
   }
   if (dts)
     for (size_t c = 0; c < n; c++) dts[c] = dt[c];
@@ -2949,9 +2936,6 @@ extern "C" int vof_batch_destroy(vof_batch_t * B) {
   }
   host_free(B->h_tab);
   dev_free(B->d_tab);
-  dev_free(B->d_dt);
-  host_free(B->h_dt);
-  dev_free((void *)B->d_dt_src);
   if (B->stream) (void)hipStreamDestroy(B->stream);
   delete B;
   return rc;
