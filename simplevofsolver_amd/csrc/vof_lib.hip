@@ -212,10 +212,13 @@ static const char * const kParamNames[P_COUNT] = {
 };
 
 struct Recorder;
+struct StepGraph;
+constexpr int kTabRing = 4;    // steps whose tables may be on their way at once
 
 struct vof_ctx {
   Recorder * rec;              // non-null: launches are recorded for a batch, not issued
   bool tab_shared;             // Thomas tables live in a batch's block
+  StepGraph * sg;              // this case's step graph (null until its second step)
   double ** tape;              // non-null: stage states (vof, ux, uy) are copied here per RK stage
   double adj_floor;            // |grad vof| dx below which corner normals are constants in the adjoint
   int nx, ny, nz;              // nz = 1 in 2D
@@ -260,6 +263,14 @@ struct vof_ctx {
   double * d_tab;
   double * h_tab;                        // pinned
   hipEvent_t tab_done[4 * 3];
+  // all tables of one step, in one copy: kTabRing pinned slots and one device
+  // block, laid out [stage][ux, uy = uz, t]
+  double * h_step;
+  double * d_step;
+  hipEvent_t step_done[4];
+  bool step_copied[4];                   // a copy left the slot that step_done does not cover
+  int step_slot;
+  const double * step_tab[3][4];         // device tables of the running step; null outside of one
   // Poisson
   int nh;
   FftPlan plan_y, plan_z;
@@ -450,11 +461,36 @@ struct LaunchRec {
   dim3 grid, block;
   size_t shm;
   std::vector<unsigned char> pack;
+  // a step graph's record instead: the kernel and its parameters as it takes
+  // them (pack holds their values, off their places in it)
+  const void * kern;
+  std::vector<unsigned> off;
 };
 
 struct Recorder {
   std::vector<LaunchRec> recs;
+  bool graph = false;          // recorded for a single case's step graph
 };
+
+// the three RK stages of one case as a linear graph of kernel nodes
+struct StepGraph {
+  Recorder rec;
+  std::vector<LaunchRec> in;   // what the executable graph's nodes hold
+  std::vector<hipGraphNode_t> nodes;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  bool warm = false;           // a step has run by plain launches
+  bool off = false;            // the runtime refused a graph: plain launches from then on
+};
+
+static void step_graph_drop(StepGraph * S) {
+  if (S->exec) (void)hipGraphExecDestroy(S->exec);
+  if (S->graph) (void)hipGraphDestroy(S->graph);
+  S->exec = nullptr;
+  S->graph = nullptr;
+  S->nodes.clear();
+  S->in.clear();
+}
 
 // Host worker threads of a batch: run(n, f) calls f(0 .. n-1) spread over
 // the workers and the calling thread and returns when all calls are done.
@@ -593,14 +629,27 @@ static size_t merge_launch(vof_batch * B, size_t idx, const std::vector<int> & c
   return hipGetLastError() == hipSuccess ? bytes : 0;
 }
 
-template <auto Body, unsigned BOUNDS, class... A>
-static void record_launch(Recorder * rec, const char * name, dim3 g, dim3 b, size_t shm, A... args) {
+template <auto Body, unsigned BOUNDS, class... P, class... A>
+static void record_launch(Recorder * rec, const char * name, void (*kern)(P...), dim3 g, dim3 b, size_t shm, A... args) {
   LaunchRec r;
   r.merge = &merge_launch<Body, BOUNDS, A...>;
   r.name = name;
   r.grid = g;
   r.block = b;
   r.shm = shm;
+  r.kern = (const void *)kern;
+  if (rec->graph) {
+    auto put = [&](const auto & v) {
+      size_t o = (r.pack.size() + alignof(std::decay_t<decltype(v)>) - 1) / alignof(std::decay_t<decltype(v)>) *
+                 alignof(std::decay_t<decltype(v)>);
+      r.pack.resize(o + sizeof(v), 0);
+      memcpy(r.pack.data() + o, &v, sizeof(v));
+      r.off.push_back((unsigned)o);
+    };
+    (put(static_cast<P>(args)), ...);
+    rec->recs.push_back(std::move(r));
+    return;
+  }
   const Pack<A...> p = make_pack(args...);
   r.pack.resize(sizeof(p));
   memcpy(r.pack.data(), &p, sizeof(p));
@@ -612,7 +661,7 @@ static void record_launch(Recorder * rec, const char * name, dim3 g, dim3 b, siz
 #define KLB(ctx, name, BOUNDS, BODY, kern, g, b, shm, ...)                           \
   do {                                                                             \
     if ((ctx)->rec) {                                                              \
-      record_launch<BODY, BOUNDS>((ctx)->rec, name, g, b, shm, __VA_ARGS__);        \
+      record_launch<BODY, BOUNDS>((ctx)->rec, name, kern, g, b, shm, __VA_ARGS__);  \
     } else {                                                                       \
       hipEvent_t e0_ = prof_begin(ctx);                                            \
       hipLaunchKernelGGL(kern, g, b, shm, (ctx)->stream, __VA_ARGS__);             \
@@ -1163,16 +1212,22 @@ static int ctx_create(domain_t * domain) {
   }
   HIPCHK(hipMalloc(&ctx->d_delta, sizeof(double) * ncell * (NDIMS + 1)));
   ctx->npart = 8192;
-  HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * ctx->npart * vofk::kDiagN));
-  HIPCHK(hipMalloc(&ctx->d_ticket, sizeof(unsigned)));
-  HIPCHK(hipMemset(ctx->d_ticket, 0, sizeof(unsigned)));
-  HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * 64));
   // Thomas tables: header 4 + l, val, v
   ctx->tab_stride = 4 + 3 * (size_t)nx;
+  // one block each: reduction partials, a step's tables and k_dt_partial's
+  // count on the device; a scalar and the tables' slots in pinned memory
+  {
+    const size_t part = (size_t)ctx->npart * vofk::kDiagN, step = ctx->tab_stride * 9;
+    HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * (part + step + 1)));
+    ctx->d_step = ctx->d_part + part;
+    ctx->d_ticket = (unsigned *)(ctx->d_step + step);
+    HIPCHK(hipMemsetAsync(ctx->d_ticket, 0, sizeof(unsigned), ctx->stream));
+    HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * (64 + step * kTabRing)));
+    ctx->h_step = ctx->h_scalar + 64;
+  }
   ctx->tab_rk = 4 * ctx->tab_stride;
   HIPCHK(hipMalloc(&ctx->d_tab, sizeof(double) * ctx->tab_stride * 12));
   HIPCHK(hipHostMalloc(&ctx->h_tab, sizeof(double) * ctx->tab_stride * 12));
-  for (int m = 0; m < 12; m++) HIPCHK(hipEventCreateWithFlags(&ctx->tab_done[m], hipEventDisableTiming));
   return 0;
 }
 
@@ -1242,11 +1297,14 @@ extern "C" int domain_finalise(domain_t * domain) {
       dev_free(ctx->d_tab);
       host_free(ctx->h_tab);
     }
-    for (int m = 0; m < 12; m++) (void)hipEventDestroy(ctx->tab_done[m]);
+    for (int m = 0; m < 12; m++)
+      if (ctx->tab_done[m]) (void)hipEventDestroy(ctx->tab_done[m]);
+    for (int m = 0; m < kTabRing; m++)
+      if (ctx->step_done[m]) (void)hipEventDestroy(ctx->step_done[m]);
     dev_free(ctx->d_twy); if (ctx->d_twz) dev_free(ctx->d_twz);
     dev_free(ctx->d_pl); dev_free(ctx->d_pu); dev_free(ctx->d_ey); dev_free(ctx->d_ez); dev_free(ctx->d_stab);
     dev_free(ctx->d_spec32); dev_free(ctx->d_twy32); dev_free(ctx->d_twz32);
-    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_rec); dev_free(ctx->d_delta); dev_free(ctx->d_part); dev_free(ctx->d_ticket);
+    dev_free(ctx->d_spec); dev_free(ctx->d_vbuf); dev_free(ctx->d_rec); dev_free(ctx->d_delta); dev_free(ctx->d_part);
     if (ctx->d_vof_spare) dev_free(ctx->d_vof_spare);
     for (int m = 0; m < 4; m++) dev_free(ctx->d_fspare[m]);
     for (void * b : ctx->freeze_slots) dev_free(b);
@@ -1261,6 +1319,8 @@ extern "C" int domain_finalise(domain_t * domain) {
       (void)hipEventDestroy(ctx->ev_main);
       (void)hipStreamDestroy(ctx->side);
     }
+    if (ctx->sg) step_graph_drop(ctx->sg);
+    delete ctx->sg;
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     domain->info = nullptr;
@@ -1518,6 +1578,10 @@ static void build_tab(double * tab, int n, double prefactor, const double * lapx
 static int upload_tab(vof_ctx * ctx, int field, int rkstep, double prefactor, const double ** dtab) {
   if (!ctx->h_tab || !ctx->d_tab)
     return fail("this case has no Thomas tables (their allocation failed when its batch was destroyed)");
+  if (ctx->step_tab[rkstep][field]) {
+    *dtab = ctx->step_tab[rkstep][field];
+    return 0;
+  }
   const int slot = field * 3 + rkstep;
   double * h = ctx->h_tab + ctx->tab_rk * rkstep + ctx->tab_stride * field;
   double * d = ctx->d_tab + ctx->tab_rk * rkstep + ctx->tab_stride * field;
@@ -1528,13 +1592,55 @@ static int upload_tab(vof_ctx * ctx, int field, int rkstep, double prefactor, co
     *dtab = d;
     return 0;
   }
-  HIPCHK(hipEventSynchronize(ctx->tab_done[slot]));
+  if (ctx->tab_done[slot])
+    HIPCHK(hipEventSynchronize(ctx->tab_done[slot]));
+  else
+    HIPCHK(hipEventCreateWithFlags(&ctx->tab_done[slot], hipEventDisableTiming));
   build_tab(h, n, prefactor, field == 0 ? ctx->lapx_ux.data() : ctx->lapx_c.data());
   HIPCHK(hipMemcpyAsync(d, h, sizeof(double) * ctx->tab_stride, hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(hipEventRecord(ctx->tab_done[slot], ctx->stream));
   *dtab = d;
   return 0;
 }
+
+// the tables of all three stages of a step with time step dt, in one copy on
+// the context's stream; upload_tab then hands them out until step_tabs_end.
+// A table is built once where fields share it (uy and uz always; t too where
+// its diffusivity is the momentum's).  `idle`: everything issued before on the
+// stream is done (integrate has just waited for dt), so no slot is in use and
+// the copy needs no event
+static int step_tabs_begin(vof_ctx * ctx, const fluid_t * fluid, double dt, bool idle) {
+  if (!ctx->h_tab || !ctx->d_tab)
+    return fail("this case has no Thomas tables (their allocation failed when its batch was destroyed)");
+  const size_t n = ctx->tab_stride;
+  if (idle)
+    for (int m = 0; m < kTabRing; m++) ctx->step_copied[m] = false;
+  const int slot = ctx->step_slot = (ctx->step_slot + 1) % kTabRing;
+  if (!idle) {
+    if (!ctx->step_done[slot]) HIPCHK(hipEventCreateWithFlags(&ctx->step_done[slot], hipEventDisableTiming));
+    if (ctx->step_copied[slot])
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+    else
+      HIPCHK(hipEventSynchronize(ctx->step_done[slot]));
+  }
+  double * h = ctx->h_step + n * 9 * slot;
+  const bool t_own = fluid->t_dif != fluid->m_dif;
+  for (int rk = 0; rk < 3; rk++) {
+    const double pm = 0.5 * kRk[rk][2] * dt * fluid->m_dif;
+    const double pt = 0.5 * kRk[rk][2] * dt * fluid->t_dif;
+    build_tab(h + n * (3 * rk + 0), ctx->nx - 1, pm, ctx->lapx_ux.data());
+    build_tab(h + n * (3 * rk + 1), ctx->nx, pm, ctx->lapx_c.data());
+    if (t_own) build_tab(h + n * (3 * rk + 2), ctx->nx, pt, ctx->lapx_c.data());
+    ctx->step_tab[rk][0] = ctx->d_step + n * (3 * rk + 0);
+    ctx->step_tab[rk][1] = ctx->step_tab[rk][2] = ctx->d_step + n * (3 * rk + 1);
+    ctx->step_tab[rk][3] = ctx->d_step + n * (3 * rk + (t_own ? 2 : 1));
+  }
+  HIPCHK(hipMemcpyAsync(ctx->d_step, h, sizeof(double) * n * 9, hipMemcpyHostToDevice, ctx->stream));
+  ctx->step_copied[slot] = idle;
+  if (!idle) HIPCHK(hipEventRecord(ctx->step_done[slot], ctx->stream));
+  return 0;
+}
+static void step_tabs_end(vof_ctx * ctx) { memset(ctx->step_tab, 0, sizeof(ctx->step_tab)); }
 
 static void swap_data(array_t * a, array_t * b) {
   void * tmp = a->data;
@@ -2215,6 +2321,8 @@ static int ensure_side(vof_ctx * ctx) {
   return 0;
 }
 
+static int graph_stages(const domain_t * domain, fluid_t * fluid, interface_t * interface, double dt);
+
 static int integrate_fused(const domain_t * domain, fluid_t * fluid, interface_t * interface, double * dt) {
   vof_ctx * ctx = ctx_of(domain);
   if ((ctx->fuse & F_VOF) && ensure_vof_spare(ctx, interface)) return 1;
@@ -2233,12 +2341,15 @@ static int integrate_fused(const domain_t * domain, fluid_t * fluid, interface_t
     ctx->stream = main_stream;
     if (rc) return 1;
     ctx->iface_ready = true;
-    const int rs = integrate_fused_stages(domain, fluid, interface, *dt);
+    const int rs = step_tabs_begin(ctx, fluid, *dt, true) || integrate_fused_stages(domain, fluid, interface, *dt);
+    step_tabs_end(ctx);
     ctx->iface_ready = false;
     return rs;
   }
   if (fluid_decide_dt(domain, fluid, dt)) return 1;
-  return integrate_fused_stages(domain, fluid, interface, *dt);
+  const int rs = step_tabs_begin(ctx, fluid, *dt, true) || graph_stages(domain, fluid, interface, *dt);
+  step_tabs_end(ctx);
+  return rs;
 }
 
 #if NDIMS == 2
@@ -2310,6 +2421,83 @@ static int launch_iface(vof_ctx * ctx, interface_t * interface) {
     KLB(ctx, "k_iface_fused", vofk::kIThreads, vofk::k_iface_fused_body, vofk::k_iface_fused, gi,
         dim3(vofk::kIThreads), 0, ctx->grid, v, nrm, cu);
   }
+  return 0;
+}
+
+static hipKernelNodeParams node_params(LaunchRec & r, std::vector<void *> & args) {
+  args.clear();
+  for (unsigned o : r.off) args.push_back(r.pack.data() + o);
+  hipKernelNodeParams p;
+  memset(&p, 0, sizeof(p));
+  p.func = const_cast<void *>(r.kern);
+  p.gridDim = r.grid;
+  p.blockDim = r.block;
+  p.sharedMemBytes = (unsigned)r.shm;
+  p.kernelParams = args.data();
+  return p;
+}
+
+// the stages of one step of a case on one stream, as a graph launch.  Small
+// grids are bound by the launches: 24 dependent kernels take 111 us by plain
+// launches and 53 us as a graph on an idle stream (65 and 30 us of the host's
+// time).  The launches are recorded as a batch's are, and nodes whose
+// parameters differ from the executable graph's (time step, the VOF buffers'
+// swap) are updated; another sequence of kernels or grids (tuning, precision)
+// builds a new graph.  The nodes are updated while no launch of the graph is
+// under way: integrate has just waited for dt behind the last one.  The first
+// step runs by plain launches, so that a single step does not pay for a graph.
+static int graph_stages(const domain_t * domain, fluid_t * fluid, interface_t * interface, double dt) {
+  vof_ctx * ctx = ctx_of(domain);
+  if (!ctx->sg) ctx->sg = new StepGraph();
+  StepGraph * S = ctx->sg;
+  if (S->off || !S->warm || (ctx->fuse & 63) != 63 || ctx->rec || ctx->tape || ctx->prof_on || ctx->freeze_mode) {
+    S->warm = true;
+    return integrate_fused_stages(domain, fluid, interface, dt);
+  }
+  S->rec.recs.clear();
+  S->rec.graph = true;
+  ctx->rec = &S->rec;
+  const int rc = integrate_fused_stages(domain, fluid, interface, dt);
+  ctx->rec = nullptr;
+  if (rc) return 1;
+  std::vector<LaunchRec> & now = S->rec.recs;
+  auto same = [](const LaunchRec & a, const LaunchRec & b) {
+    return a.kern == b.kern && a.grid.x == b.grid.x && a.grid.y == b.grid.y && a.grid.z == b.grid.z &&
+           a.block.x == b.block.x && a.block.y == b.block.y && a.block.z == b.block.z && a.shm == b.shm;
+  };
+  bool fits = S->exec && S->in.size() == now.size();
+  for (size_t i = 0; fits && i < now.size(); i++) fits = same(S->in[i], now[i]);
+  std::vector<void *> args;
+  hipError_t e = hipSuccess;
+  if (fits) {
+    for (size_t i = 0; e == hipSuccess && i < now.size(); i++) {
+      if (S->in[i].pack == now[i].pack) continue;
+      const hipKernelNodeParams p = node_params(now[i], args);
+      e = hipGraphExecKernelNodeSetParams(S->exec, S->nodes[i], &p);
+      S->in[i].pack = now[i].pack;
+    }
+  } else {
+    step_graph_drop(S);
+    e = hipGraphCreate(&S->graph, 0);
+    for (size_t i = 0; e == hipSuccess && i < now.size(); i++) {
+      const hipKernelNodeParams p = node_params(now[i], args);
+      hipGraphNode_t node;
+      e = hipGraphAddKernelNode(&node, S->graph, i ? &S->nodes.back() : nullptr, i ? 1 : 0, &p);
+      if (e == hipSuccess) S->nodes.push_back(node);
+    }
+    if (e == hipSuccess) e = hipGraphInstantiate(&S->exec, S->graph, nullptr, nullptr, 0);
+    S->in = now;
+  }
+  if (e == hipSuccess) e = hipGraphLaunch(S->exec, ctx->stream);
+  if (e == hipSuccess) return 0;
+  // nothing of the step has been issued: its recorded launches go out plainly
+  (void)hipGetLastError();
+  S->off = true;
+  for (LaunchRec & r : now) {
+    const hipKernelNodeParams p = node_params(r, args);
+    HIPCHK(hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes, ctx->stream));
+  }
+  step_graph_drop(S);
   return 0;
 }
 
@@ -3234,13 +3422,21 @@ extern "C" int vof_set_freeze(domain_t * domain, int mode) {
 
 // one step with a given dt (the frozen dt sequence of the adjoint and its
 // finite-difference checks); fused schedule
+// the stages of one step with a given dt, nothing waited for before
+static int stages_fixed_dt(const domain_t * domain, fluid_t * fluid, interface_t * interface, double dt) {
+  vof_ctx * ctx = ctx_of(domain);
+  const int rc = step_tabs_begin(ctx, fluid, dt, false) || integrate_fused_stages(domain, fluid, interface, dt);
+  step_tabs_end(ctx);
+  return rc;
+}
+
 extern "C" int vof_integrate_fixed_dt(const domain_t * domain, fluid_t * fluid, interface_t * interface,
                                       double dt) {
   CTX_OR_FAIL(domain);
   if (ctx->schedule != 1 || (ctx->fuse & 63) != 63) return fail("vof_integrate_fixed_dt: fused schedule only");
   if (ensure_vof_spare(ctx, interface)) return 1;
   if ((ctx->fuse & F_PRED) && ensure_field_spares(ctx, fluid)) return 1;
-  return integrate_fused_stages(domain, fluid, interface, dt);
+  return stages_fixed_dt(domain, fluid, interface, dt);
 }
 
 #if NDIMS == 2
@@ -3391,7 +3587,7 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
   // forward with checkpoints
   for (int n = 0; n < nsteps; n++) {
     if (n % every == 0 && save(n / every)) return 1;
-    if (integrate_fused_stages(domain, fluid, interface, dts[n])) return 1;
+    if (stages_fixed_dt(domain, fluid, interface, dts[n])) return 1;
   }
   // loss and its vof gradient on the host
   std::vector<double> hv(bvof / sizeof(double)), hg;
@@ -3435,12 +3631,17 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
     if (restore(c)) return 1;
     for (int n = s0; n < s1; n++) {
       ctx->tape = &tape[9 * (size_t)(n - s0)];
-      const int rc = integrate_fused_stages(domain, fluid, interface, dts[n]);
+      const int rc = stages_fixed_dt(domain, fluid, interface, dts[n]);
       ctx->tape = nullptr;
       if (rc) return 1;
     }
     for (int n = s1 - 1; n >= s0; n--) {
       const double dt = dts[n];
+      struct TabsEnd {
+        vof_ctx * ctx;
+        ~TabsEnd() { step_tabs_end(ctx); }
+      } tabs_end{ctx};
+      if (step_tabs_begin(ctx, fluid, dt, false)) return 1;
       for (int rk = 2; rk >= 0; rk--) {
         double ** t = &tape[9 * (size_t)(n - s0) + 3 * rk];
         const double * vof = t[0];
