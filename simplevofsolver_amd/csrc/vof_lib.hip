@@ -4067,32 +4067,36 @@ struct tdm_info_t_ {
 };
 
 namespace vofk {
-// factor table of one system of `n` rows:
-//   [0, n)        v[i]   (upper factors, rows 0 .. m-2 of the gtsv part)
-//   [n, 2n)       rec[i] (reciprocal pivots of rows 1 .. m-1; rec[0] = c[0], a divisor)
-//   [2n, 3n)      q1[i]  (periodic: the solved correction vector, rows 0 .. n-2)
-//   3n            1 if the last gtsv pivot is singular (|pivot| <= DBL_EPSILON, tdm.c:39-44)
-//   3n + 1        den of the Sherman-Morrison update (tdm.c:93)
-//   3n + 2        1 if |den| < DBL_EPSILON (tdm.c:94)
-// m = n for a non-periodic system, n - 1 for a periodic one
-__host__ __device__ constexpr size_t tdm_table_len(int n) { return 3 * (size_t)n + 3; }
+// factor table of one system of `n` rows, m of them solved by gtsv (m = n, or
+// n - 1 for a periodic system):
+//   [0] c[0], the divisor of row 0    [1] 1 / last gtsv pivot (0 if singular)
+//   [2] 0 if that pivot is singular (|pivot| <= DBL_EPSILON, tdm.c:39-44), else 1
+//   [3] den of the Sherman-Morrison update (tdm.c:93), 0 where |den| < DBL_EPSILON (tdm.c:94)
+//   [4, 4 + m)             l[i]
+//   [4 + m, 4 + 2m)        reciprocal pivots of rows 1 .. m-1
+//   [4 + 2m, 4 + 3m)       v[i] (upper factors, rows 0 .. m-2)
+//   [4 + 3m, 4 + 3m + n)   q1[i] (periodic: the solved correction vector, rows 0 .. n-2)
+// (the first part is laid out as the predictor's tables, so that lines are
+// swept by lines_sweep_rows)
+__host__ __device__ constexpr size_t tdm_table_len(int n) { return 4 * (size_t)n + 4; }
+__device__ __forceinline__ const double * tdm_q1(const double * tab, int m) { return tab + 4 + 3 * (size_t)m; }
 
 // forward and backward sweeps of gtsv (tdm.c:26-48) over one strided line with the
 // table's factors: q[k * st] is row k
-__device__ __forceinline__ void tdm_sweeps(int m, const double * __restrict__ tab, int n,
-                                           const double * __restrict__ l, double * q, size_t st) {
-  const double * v = tab;
-  const double * rec = tab + n;
-  double prev = q[0] / rec[0];
+__device__ __forceinline__ void tdm_sweeps(int m, const double * __restrict__ tab, double * q, size_t st) {
+  const double * l = tab + 4;
+  const double * rec = tab + 4 + m;
+  const double * v = tab + 4 + 2 * (size_t)m;
+  double prev = q[0] / tab[0];
   q[0] = prev;
   for (int i = 1; i < m - 1; i++) {
     prev = rec[i] * (q[i * st] - l[i] * prev);
     q[i * st] = prev;
   }
-  if (tab[3 * n] != 0.) {
+  if (tab[2] == 0.) {
     prev = 0.;
   } else {
-    prev = rec[m - 1] * (q[(m - 1) * st] - l[m - 1] * prev);
+    prev = tab[1] * (q[(m - 1) * st] - l[m - 1] * prev);
   }
   q[(m - 1) * st] = prev;
   for (int i = m - 2; i >= 0; i--) {
@@ -4101,129 +4105,276 @@ __device__ __forceinline__ void tdm_sweeps(int m, const double * __restrict__ ta
   }
 }
 
-// one thread: the factors (tdm.c:27,33-34,38), the periodic correction q1
-// (tdm.c:80-86) and the Sherman-Morrison denominator (tdm.c:93)
-__global__ void k_tdm_table(int n, int periodic, const double * __restrict__ l, const double * __restrict__ c,
-                            const double * __restrict__ u, double * __restrict__ tab) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// rows of an LDS line: whole segments of the sweep; 2 mod 4 where several
+// lines share the work-group (distinct banks)
+__host__ __device__ inline int tdm_stride(int n, int nsys) { return lines_stride(n) - (nsys > 1 ? 0 : 2); }
+
+constexpr int kTdmT = 256;       // threads of k_tdm_table
+constexpr int kTdmChunk = 512;   // rows staged at a time
+constexpr int kTdmLine = 4096;   // longest correction vector swept in LDS
+
+// one work-group: the factors (tdm.c:27,33-34,38), the periodic correction q1
+// (tdm.c:80-86) and the Sherman-Morrison denominator (tdm.c:93).  One lane
+// runs the factor recurrence (bound by its division, 48 ns a row) on rows
+// staged in LDS by all, the next rows on their way meanwhile; q1 is one line
+// of lines_sweep_rows.  256 rows: 52 -> 20 us, 375 periodic rows 167 ->
+// 45 (from global memory, one load after the other, before). A row costs the latency of its division.
+__global__ __launch_bounds__(kTdmT) void k_tdm_table(int n, int periodic, const double * __restrict__ l,
+                                                     const double * __restrict__ c, const double * __restrict__ u,
+                                                     double * __restrict__ tab) {
+  __shared__ __align__(16) double sh[kTdmLine];
+  static_assert(5 * kTdmChunk <= kTdmLine, "the staged rows do not fit");
+  double * sl = sh, * sc = sh + kTdmChunk, * su = sh + 2 * kTdmChunk, * sr = sh + 3 * kTdmChunk, * sv = sh + 4 * kTdmChunk;
+  const int tid = (int)threadIdx.x;
   const int m = periodic ? n - 1 : n;
-  double * v = tab;
-  double * rec = tab + n;
-  v[0] = u[0] / c[0];
-  rec[0] = c[0];
-  for (int i = 1; i < m - 1; i++) {
-    const double val = 1. / (c[i] - l[i] * v[i - 1]);
-    rec[i] = val;
-    v[i] = val * (u[i]);
+  double * L = tab + 4, * VAL = L + m, * V = VAL + m, * q1 = V + m;
+  constexpr int PT = kTdmChunk / kTdmT;
+  double rl[PT], rc[PT], ru[PT];
+  auto fetch = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+      const int i = min(i0 + tid + kTdmT * k, m - 1);
+      rl[k] = l[i];
+      rc[k] = c[i];
+      ru[k] = u[i];
+    }
+  };
+  fetch(0);
+  double vprev = 0.;
+  for (int i0 = 0; i0 < m; i0 += kTdmChunk) {
+    const int nr = min(kTdmChunk, m - i0);
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+      sl[tid + kTdmT * k] = rl[k];
+      sc[tid + kTdmT * k] = rc[k];
+      su[tid + kTdmT * k] = ru[k];
+    }
+    __syncthreads();
+    if (i0 + kTdmChunk < m) fetch(i0 + kTdmChunk);
+    if (tid == 0) {
+      int r = 0;
+      if (i0 == 0) {
+        vprev = su[0] / sc[0];
+        sr[0] = sc[0];
+        sv[0] = vprev;
+        r = 1;
+      }
+      const int re = min(nr, m - 1 - i0);   // rows before the last one
+      for (; r + 8 <= re; r += 8) {
+        double a[8], b[8], d[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          a[k] = sl[r + k];
+          b[k] = sc[r + k];
+          d[k] = su[r + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const double val = 1. / (b[k] - a[k] * vprev);
+          vprev = val * d[k];
+          sr[r + k] = val;
+          sv[r + k] = vprev;
+        }
+      }
+      for (; r < re; r++) {
+        const double val = 1. / (sc[r] - sl[r] * vprev);
+        vprev = val * (su[r]);
+        sr[r] = val;
+        sv[r] = vprev;
+      }
+      if (i0 + nr == m) {
+        const double val = sc[nr - 1] - sl[nr - 1] * vprev;
+        const bool singular = !(fabs(val) > DBL_EPSILON);
+        const double rlast = singular ? 0. : 1. / val;
+        sr[nr - 1] = rlast;
+        sv[nr - 1] = 0.;
+        tab[1] = rlast;
+        tab[2] = singular ? 0. : 1.;
+      }
+      if (i0 == 0) tab[0] = sc[0];
+    }
+    __syncthreads();
+    for (int r = tid; r < nr; r += kTdmT) {
+      L[i0 + r] = sl[r];
+      VAL[i0 + r] = sr[r];
+      V[i0 + r] = sv[r];
+    }
+    __syncthreads();
   }
-  const double val = c[m - 1] - l[m - 1] * v[m - 2];
-  const bool singular = !(fabs(val) > DBL_EPSILON);
-  rec[m - 1] = singular ? 0. : 1. / val;
-  tab[3 * n] = singular ? 1. : 0.;
   if (!periodic) {
-    tab[3 * n + 1] = 0.;
-    tab[3 * n + 2] = 0.;
+    if (tid == 0) tab[3] = 0.;
     return;
   }
-  double * q1 = tab + 2 * n;
-  for (int i = 0; i < n - 1; i++) q1[i] = i == 0 ? -l[i] : i == n - 2 ? -u[i] : 0.;
-  tdm_sweeps(m, tab, n, l, q1, 1);
-  const double den = c[n - 1] + u[n - 1] * q1[0] + l[n - 1] * q1[n - 2];
-  tab[3 * n + 1] = den;
-  tab[3 * n + 2] = fabs(den) < DBL_EPSILON ? 1. : 0.;
+  const bool inlds = m <= kTdmLine;
+  double * q = inlds ? sh : q1;
+  for (int i = tid; i < m; i += kTdmT) q[i] = i == 0 ? -l[i] : i == n - 2 ? -u[i] : 0.;
+  __syncthreads();
+  if (inlds) {
+    if (tid < 64) lines_sweep_rows(sweep_head(tab, m, tid), tab, m, sh, tdm_stride(m, 1), 1, tid);
+    __syncthreads();
+    for (int i = tid; i < m; i += kTdmT) q1[i] = sh[i];
+  } else if (tid == 0) {
+    tdm_sweeps(m, tab, q1, 1);
+  }
+  if (tid == 0) {
+    const double den = c[n - 1] + u[n - 1] * q[0] + l[n - 1] * q[n - 2];
+    tab[3] = fabs(den) < DBL_EPSILON ? 0. : den;
+  }
 }
 
 // the periodic update of one line (tdm.c:92-98)
-__device__ __forceinline__ void tdm_periodic_fix(int n, const double * __restrict__ tab,
-                                                 const double * __restrict__ l, const double * __restrict__ u,
-                                                 double * q, size_t st) {
-  const double * q1 = tab + 2 * n;
-  const double num = q[(n - 1) * st] - u[n - 1] * q[0] - l[n - 1] * q[(n - 2) * st];
-  const double last = tab[3 * n + 2] != 0. ? 0. : num / tab[3 * n + 1];
-  q[(n - 1) * st] = last;
-  for (int i = 0; i < n - 1; i++) q[i * st] = q[i * st] + last * q1[i];
+__device__ __forceinline__ double tdm_periodic_last(int n, const double * __restrict__ tab, const double * __restrict__ l,
+                                                    const double * __restrict__ u, double qlast, double q0, double qn2) {
+  const double num = qlast - u[n - 1] * q0 - l[n - 1] * qn2;
+  return tab[3] == 0. ? 0. : num / tab[3];
 }
 
-// tdm_solve (tdm.c:66-106) over nrhs contiguous lines of n rows with ncomp
+// tdm_solve (tdm.c:66-106) over nrhs contiguous lines of n rows with NC
 // interleaved components (1 real, 2 = the real and imaginary parts of a
 // complex value, which the reference's real-by-complex arithmetic treats as
 // two independent systems with the same coefficients).
 //
-// lpb > 0: a work-group loads lpb consecutive lines (one contiguous run of
-// lpb * n * ncomp doubles, coalesced) into LDS with one system per LDS row of
-// odd stride (lanes of one wavefront hit distinct banks), one lane per
-// system runs the sweeps there, and the work-group stores the run back.
-// lpb == 0: lines too long for LDS; one lane per system in global memory.
-__global__ __launch_bounds__(256) void k_tdm_lines(int n, int nrhs, int periodic, int ncomp, int lpb,
-                                                   const double * __restrict__ l, const double * __restrict__ u,
-                                                   const double * __restrict__ tab, double * __restrict__ data) {
+// A work-group holds lpb consecutive lines (one contiguous run) in LDS, a
+// system per row there: (line, 64-row chunk) pairs are loaded by wavefronts,
+// kWUnroll at a time, each wavefront sweeps 16 systems (lines_sweep_rows), and
+// the pairs are stored back, with the periodic update.  Bound by HBM at 65536
+// lines of 256 rows (154 -> 76 us, 268 MB), by the sweep where the chip is
+// not filled (1500 complex periodic lines of 375 rows 65 -> 21).
+template <int NC>
+__global__ __launch_bounds__(kWThreads) void k_tdm_lines(int n, int nrhs, int periodic, int lpb,
+                                                         const double * __restrict__ l, const double * __restrict__ u,
+                                                         const double * __restrict__ tab, double * __restrict__ data) {
+  struct T {                     // 8-byte aligned, as the caller's data may be
+    double c[NC];
+  };
+  extern __shared__ __align__(16) double S[];
   const int m = periodic ? n - 1 : n;
-  if (lpb == 0) {
-    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= (long)nrhs * ncomp) return;
-    double * q = data + (s / ncomp) * (size_t)n * ncomp + (s % ncomp);
-    tdm_sweeps(m, tab, n, l, q, (size_t)ncomp);
-    if (periodic) tdm_periodic_fix(n, tab, l, u, q, (size_t)ncomp);
-    return;
-  }
-  extern __shared__ double lds[];
-  const int stride = n | 1;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  constexpr int nw = kWThreads / 64;
   const long j0 = (long)blockIdx.x * lpb;
-  const int lines = (int)min((long)lpb, (long)nrhs - j0);
-  const int run = lines * n * ncomp;
-  double * g = data + j0 * (size_t)n * ncomp;
-  for (int e = threadIdx.x; e < run; e += blockDim.x) {
-    const int jl = e / (n * ncomp);
-    const int rem = e - jl * n * ncomp;
-    const int i = rem / ncomp;
-    const int r = rem - i * ncomp;
-    lds[(jl * ncomp + r) * stride + i] = g[e];
+  const int lines = (int)min((long)lpb, (long)nrhs - j0), nsys = lines * NC;
+  const int ld = tdm_stride(m, lpb * NC);
+  double * qlast = S + (size_t)lpb * NC * ld;   // periodic: row n - 1 of every system, then its solution
+  const int nch = (n + 63) >> 6, np = lines * nch;
+  T * g = reinterpret_cast<T *>(data) + j0 * (size_t)n;
+  auto place = [&](int p, int & ll, int & i) {
+    ll = p / nch;
+    i = 64 * (p - ll * nch) + lane;
+  };
+  for (int p0 = w; p0 < np; p0 += nw * kWUnroll) {
+    T v[kWUnroll];
+#pragma unroll
+    for (int k = 0; k < kWUnroll; k++) {
+      int ll, i;
+      place(min(p0 + nw * k, np - 1), ll, i);
+      v[k] = g[(size_t)ll * n + min(i, n - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < kWUnroll; k++) {
+      int ll, i;
+      place(min(p0 + nw * k, np - 1), ll, i);
+      const int r = min(i, n - 1);
+#pragma unroll
+      for (int e = 0; e < NC; e++) {
+        const double x = v[k].c[e];
+        double * at = r < m ? S + (size_t)(ll * NC + e) * ld + r : qlast + ll * NC + e;
+        *at = x;
+      }
+    }
   }
+  const SweepHead h = sweep_head(tab, m, lane);
   __syncthreads();
-  const int s = threadIdx.x;
-  if (s < lines * ncomp) {
-    double * q = lds + s * stride;
-    tdm_sweeps(m, tab, n, l, q, 1);
-    if (periodic) tdm_periodic_fix(n, tab, l, u, q, 1);
+  for (int s = kSwLines * w; s < nsys; s += kSwLines * nw)
+    lines_sweep_rows(h, tab, m, S + (size_t)s * ld, ld, min(kSwLines, nsys - s), lane);
+  __syncthreads();
+  if (periodic) {
+    for (int s = (int)threadIdx.x; s < nsys; s += kWThreads) {
+      const double * q = S + (size_t)s * ld;
+      qlast[s] = tdm_periodic_last(n, tab, l, u, qlast[s], q[0], q[n - 2]);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < run; e += blockDim.x) {
-    const int jl = e / (n * ncomp);
-    const int rem = e - jl * n * ncomp;
-    const int i = rem / ncomp;
-    const int r = rem - i * ncomp;
-    g[e] = lds[(jl * ncomp + r) * stride + i];
+  const double * q1 = tdm_q1(tab, m);
+#pragma unroll 4
+  for (int p = w; p < np; p += nw) {
+    int ll, i;
+    place(p, ll, i);
+    if (i < n) {
+      T v;
+#pragma unroll
+      for (int e = 0; e < NC; e++) {
+        const int s = ll * NC + e;
+        double x = i < m ? S[(size_t)s * ld + i] : qlast[s];
+        if (periodic && i < m) x = x + qlast[s] * q1[i];
+        v.c[e] = x;
+      }
+      g[(size_t)ll * n + i] = v;
+    }
+  }
+}
+
+// launched from host-only code below: instantiated here for the device pass
+template __global__ void k_tdm_lines<1>(int, int, int, int, const double * __restrict__, const double * __restrict__,
+                                        const double * __restrict__, double * __restrict__);
+template __global__ void k_tdm_lines<2>(int, int, int, int, const double * __restrict__, const double * __restrict__,
+                                        const double * __restrict__, double * __restrict__);
+
+// lines too long for LDS: one lane per system in global memory
+__global__ __launch_bounds__(256) void k_tdm_long(int n, int nrhs, int periodic, int ncomp,
+                                                  const double * __restrict__ l, const double * __restrict__ u,
+                                                  const double * __restrict__ tab, double * __restrict__ data) {
+  const int m = periodic ? n - 1 : n;
+  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= (long)nrhs * ncomp) return;
+  const size_t st = (size_t)ncomp;
+  double * q = data + (s / ncomp) * (size_t)n * ncomp + (s % ncomp);
+  tdm_sweeps(m, tab, q, st);
+  if (periodic) {
+    const double * q1 = tdm_q1(tab, m);
+    const double last = tdm_periodic_last(n, tab, l, u, q[(n - 1) * st], q[0], q[(n - 2) * st]);
+    q[(n - 1) * st] = last;
+    for (int i = 0; i < n - 1; i++) q[i * st] = q[i * st] + last * q1[i];
   }
 }
 }  // namespace vofk
 
 // host-only: the vtable object must not be emitted by the device pass
 #if !defined(__HIP_DEVICE_COMPILE__)
-// lines per work-group of k_tdm_lines within 64 KiB of LDS and 256 systems
-// (0: the line does not fit, one lane per system in global memory)
-static int tdm_lines_per_group(int n, int ncomp) {
-  const size_t row = sizeof(double) * (size_t)(n | 1);
-  const size_t by_lds = (size_t)65536 / (row * ncomp);
-  const size_t by_lanes = 256 / ncomp;
-  return (int)(by_lds < by_lanes ? by_lds : by_lanes);
+// lines per work-group of k_tdm_lines: as the predictor's (48 (line, chunk)
+// pairs of a system, fewer where that leaves compute units idle), within 64
+// KiB of LDS; 0 where one line does not fit
+static int tdm_lines_per_group(int n, int ncomp, int nrhs) {
+  const int nch = (n + 63) / 64;
+  const long want = (long)nrhs * ncomp / 256;
+  long lpb = 48 / (nch * ncomp);
+  lpb = lpb < 1 ? 1 : lpb;
+  if (lpb > want) lpb = want > 4 / ncomp ? want : 4 / ncomp;
+  if (lpb > 48 / (nch * ncomp)) lpb = 48 / (nch * ncomp);
+  if (lpb < 1) lpb = 1;
+  while (lpb > 1 && sizeof(double) * (size_t)(vofk::tdm_stride(n, (int)lpb * ncomp) + 1) * ncomp * lpb > 65536) lpb--;
+  return sizeof(double) * (size_t)(vofk::tdm_stride(n, ncomp) + 1) * ncomp <= 65536 ? (int)lpb : 0;
 }
 
 // the table and line kernels of one solve on `st`
 static int tdm_enqueue(int n, int nrhs, bool periodic, bool cplx, const double * l, const double * c,
                        const double * u, double * tab, void * data, hipStream_t st) {
   const int ncomp = cplx ? 2 : 1;
-  hipLaunchKernelGGL(vofk::k_tdm_table, dim3(1), dim3(64), 0, st, n, (int)periodic, l, c, u, tab);
+  hipLaunchKernelGGL(vofk::k_tdm_table, dim3(1), dim3(vofk::kTdmT), 0, st, n, (int)periodic, l, c, u, tab);
   LAUNCHCHK();
-  const int lpb = tdm_lines_per_group(n, ncomp);
+  const int lpb = tdm_lines_per_group(n, ncomp, nrhs);
   if (lpb > 0) {
-    const long nb = ((long)nrhs + lpb - 1) / lpb;
-    const size_t shm = sizeof(double) * (size_t)(n | 1) * ncomp * lpb;
-    hipLaunchKernelGGL(vofk::k_tdm_lines, dim3((unsigned)nb), dim3(256), shm, st, n, nrhs, (int)periodic, ncomp,
-                       lpb, l, u, (const double *)tab, (double *)data);
+    const dim3 nb((unsigned)(((long)nrhs + lpb - 1) / lpb)), b(vofk::kWThreads);
+    const size_t shm = sizeof(double) * (size_t)(vofk::tdm_stride(n, lpb * ncomp) + 1) * ncomp * lpb;
+    if (cplx)
+      hipLaunchKernelGGL(vofk::k_tdm_lines<2>, nb, b, shm, st, n, nrhs, (int)periodic, lpb, l, u, (const double *)tab,
+                         (double *)data);
+    else
+      hipLaunchKernelGGL(vofk::k_tdm_lines<1>, nb, b, shm, st, n, nrhs, (int)periodic, lpb, l, u, (const double *)tab,
+                         (double *)data);
   } else {
     const long nb = ((long)nrhs * ncomp + 255) / 256;
-    hipLaunchKernelGGL(vofk::k_tdm_lines, dim3((unsigned)nb), dim3(256), 0, st, n, nrhs, (int)periodic, ncomp, 0,
-                       l, u, (const double *)tab, (double *)data);
+    hipLaunchKernelGGL(vofk::k_tdm_long, dim3((unsigned)nb), dim3(256), 0, st, n, nrhs, (int)periodic, ncomp, l, u,
+                       (const double *)tab, (double *)data);
   }
   LAUNCHCHK();
   return 0;
@@ -4248,17 +4399,17 @@ static int tdm_construct(const int size, const int nrhs, const bool is_periodic,
   t->nrhs = nrhs;
   t->is_periodic = is_periodic;
   t->is_complex = is_complex;
-  t->l = (double *)calloc(size, sizeof(double));
-  t->c = (double *)calloc(size, sizeof(double));
-  t->u = (double *)calloc(size, sizeof(double));
+  t->l = (double *)calloc(3 * (size_t)size, sizeof(double));   // l, c, u: one copy to the device
+  t->c = t->l ? t->l + size : nullptr;
+  t->u = t->l ? t->l + 2 * (size_t)size : nullptr;
   t->d_luc = nullptr;
   t->d_tab = nullptr;
   t->stream = nullptr;
   hipError_t e = hipMalloc(&t->d_luc, sizeof(double) * 3 * size);
   if (e == hipSuccess) e = hipMalloc(&t->d_tab, sizeof(double) * vofk::tdm_table_len(size));
   if (e == hipSuccess) e = hipStreamCreate(&t->stream);
-  if (e != hipSuccess || !t->l || !t->c || !t->u) {
-    free(t->l); free(t->c); free(t->u);
+  if (e != hipSuccess || !t->l) {
+    free(t->l);
     dev_free(t->d_luc); dev_free(t->d_tab);
     if (t->stream) (void)hipStreamDestroy(t->stream);
     delete t;
@@ -4298,9 +4449,7 @@ static int tdm_solve(const tdm_info_t * info, void * data) {
   if (!data) return fail("ERROR(solve): data is NULL");
   const int n = info->size;
   hipStream_t st = info->stream;
-  HIPCHK(hipMemcpyAsync(info->d_luc, info->l, sizeof(double) * n, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(info->d_luc + n, info->c, sizeof(double) * n, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(info->d_luc + 2 * n, info->u, sizeof(double) * n, hipMemcpyHostToDevice, st));
+  HIPCHK(hipMemcpyAsync(info->d_luc, info->l, sizeof(double) * 3 * n, hipMemcpyHostToDevice, st));
   if (tdm_enqueue(n, info->nrhs, info->is_periodic, info->is_complex, info->d_luc, info->d_luc + n,
                   info->d_luc + 2 * n, info->d_tab, data, st))
     return 1;
@@ -4309,7 +4458,7 @@ static int tdm_solve(const tdm_info_t * info, void * data) {
 }
 static int tdm_destruct(tdm_info_t * info) {
   if (!info) return fail("ERROR(destruct): info is NULL");
-  free(info->l); free(info->c); free(info->u);
+  free(info->l);
   dev_free(info->d_luc); dev_free(info->d_tab);
   if (info->stream) (void)hipStreamDestroy(info->stream);
   delete info;
@@ -4331,7 +4480,7 @@ extern "C" const tdm_t tdm = {
 #endif  // !__HIP_DEVICE_COMPILE__
 
 constexpr int kTdmNoallocMax = 16384;   // largest system size of tdm_solve_noalloc
-__device__ __align__(256) double scratch[3 * kTdmNoallocMax + 3];
+__device__ __align__(256) double scratch[4 * kTdmNoallocMax + 4];
 
 #if !defined(__HIP_DEVICE_COMPILE__)
 static std::mutex g_scratch_mu;
