@@ -263,13 +263,13 @@ struct vof_ctx {
   double * d_tab;
   double * h_tab;                        // pinned
   hipEvent_t tab_done[4 * 3];
-  // all tables of one step, in one copy: kTabRing pinned slots and one device
-  // block, laid out [stage][ux, uy = uz, t]
-  double * h_step;
+  // all tables of one step, in one copy into one device block, laid out
+  // [stage][ux, uy = uz, t]: from behind h_scalar where the stream is idle,
+  // else from the next of kTabRing pinned slots (allocated on first use)
   double * d_step;
-  hipEvent_t step_done[4];
-  bool step_copied[4];                   // a copy left the slot that step_done does not cover
-  int step_slot;
+  double * h_ring;
+  hipEvent_t ring_done[kTabRing];
+  int ring_slot;
   const double * step_tab[3][4];         // device tables of the running step; null outside of one
   // Poisson
   int nh;
@@ -1215,15 +1215,14 @@ static int ctx_create(domain_t * domain) {
   // Thomas tables: header 4 + l, val, v
   ctx->tab_stride = 4 + 3 * (size_t)nx;
   // one block each: reduction partials, a step's tables and k_dt_partial's
-  // count on the device; a scalar and the tables' slots in pinned memory
+  // count on the device; a scalar and a step's tables in pinned memory
   {
     const size_t part = (size_t)ctx->npart * vofk::kDiagN, step = ctx->tab_stride * 9;
     HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * (part + step + 1)));
     ctx->d_step = ctx->d_part + part;
     ctx->d_ticket = (unsigned *)(ctx->d_step + step);
     HIPCHK(hipMemsetAsync(ctx->d_ticket, 0, sizeof(unsigned), ctx->stream));
-    HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * (64 + step * kTabRing)));
-    ctx->h_step = ctx->h_scalar + 64;
+    HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * (64 + step)));
   }
   ctx->tab_rk = 4 * ctx->tab_stride;
   HIPCHK(hipMalloc(&ctx->d_tab, sizeof(double) * ctx->tab_stride * 12));
@@ -1300,7 +1299,8 @@ extern "C" int domain_finalise(domain_t * domain) {
     for (int m = 0; m < 12; m++)
       if (ctx->tab_done[m]) (void)hipEventDestroy(ctx->tab_done[m]);
     for (int m = 0; m < kTabRing; m++)
-      if (ctx->step_done[m]) (void)hipEventDestroy(ctx->step_done[m]);
+      if (ctx->ring_done[m]) (void)hipEventDestroy(ctx->ring_done[m]);
+    host_free(ctx->h_ring);
     dev_free(ctx->d_twy); if (ctx->d_twz) dev_free(ctx->d_twz);
     dev_free(ctx->d_pl); dev_free(ctx->d_pu); dev_free(ctx->d_ey); dev_free(ctx->d_ez); dev_free(ctx->d_stab);
     dev_free(ctx->d_spec32); dev_free(ctx->d_twy32); dev_free(ctx->d_twz32);
@@ -1607,23 +1607,22 @@ static int upload_tab(vof_ctx * ctx, int field, int rkstep, double prefactor, co
 // the context's stream; upload_tab then hands them out until step_tabs_end.
 // A table is built once where fields share it (uy and uz always; t too where
 // its diffusivity is the momentum's).  `idle`: everything issued before on the
-// stream is done (integrate has just waited for dt), so no slot is in use and
-// the copy needs no event
+// stream is done (integrate has just waited for dt), so no earlier copy is
+// under way and this one needs no event
 static int step_tabs_begin(vof_ctx * ctx, const fluid_t * fluid, double dt, bool idle) {
   if (!ctx->h_tab || !ctx->d_tab)
     return fail("this case has no Thomas tables (their allocation failed when its batch was destroyed)");
   const size_t n = ctx->tab_stride;
-  if (idle)
-    for (int m = 0; m < kTabRing; m++) ctx->step_copied[m] = false;
-  const int slot = ctx->step_slot = (ctx->step_slot + 1) % kTabRing;
+  double * h = ctx->h_scalar + 64;
   if (!idle) {
-    if (!ctx->step_done[slot]) HIPCHK(hipEventCreateWithFlags(&ctx->step_done[slot], hipEventDisableTiming));
-    if (ctx->step_copied[slot])
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-    else
-      HIPCHK(hipEventSynchronize(ctx->step_done[slot]));
+    if (!ctx->h_ring) {
+      HIPCHK(hipHostMalloc(&ctx->h_ring, sizeof(double) * n * 9 * kTabRing));
+      for (int m = 0; m < kTabRing; m++) HIPCHK(hipEventCreateWithFlags(&ctx->ring_done[m], hipEventDisableTiming));
+    }
+    ctx->ring_slot = (ctx->ring_slot + 1) % kTabRing;
+    HIPCHK(hipEventSynchronize(ctx->ring_done[ctx->ring_slot]));
+    h = ctx->h_ring + n * 9 * ctx->ring_slot;
   }
-  double * h = ctx->h_step + n * 9 * slot;
   const bool t_own = fluid->t_dif != fluid->m_dif;
   for (int rk = 0; rk < 3; rk++) {
     const double pm = 0.5 * kRk[rk][2] * dt * fluid->m_dif;
@@ -1636,8 +1635,7 @@ static int step_tabs_begin(vof_ctx * ctx, const fluid_t * fluid, double dt, bool
     ctx->step_tab[rk][3] = ctx->d_step + n * (3 * rk + (t_own ? 2 : 1));
   }
   HIPCHK(hipMemcpyAsync(ctx->d_step, h, sizeof(double) * n * 9, hipMemcpyHostToDevice, ctx->stream));
-  ctx->step_copied[slot] = idle;
-  if (!idle) HIPCHK(hipEventRecord(ctx->step_done[slot], ctx->stream));
+  if (!idle) HIPCHK(hipEventRecord(ctx->ring_done[ctx->ring_slot], ctx->stream));
   return 0;
 }
 static void step_tabs_end(vof_ctx * ctx) { memset(ctx->step_tab, 0, sizeof(ctx->step_tab)); }
