@@ -397,11 +397,13 @@ int vof_batch_autotune(vof_batch_t * batch, int steps, char * report, size_t len
  * 2048 complex values per LDS buffer of the FFT kernels, "lines_lpb" = lines
  * per work-group of the predictor's x solver (0 = automatic); "xcd_bands" =
  * 1 walks the 3D stencil tiles band by band per XCD; "rhs_rows" = 1, 2, 4,
- * 8 (default) or 16 rows of one column per thread of the source kernel;
+ * 8 or 16 rows of one column per thread of the source kernel (default: by
+ * the grid's size, 1 on the smallest, 8 on large ones; in a batch by the
+ * cases' together);
  * "pred_rows" = 1, 2, 4 or 8 (default) rows per thread of the one-kernel
  * predictor (fewer where its x lines would not fit 64 KiB of LDS);
- * "iface_planes" = 0 (blocks), 4, 8 (default) or 16 z planes marched per
- * work-group by the 3D interface kernel;
+ * "iface_planes" = 0 (blocks), 4, 8 or 16 z planes marched per work-group by
+ * the 3D interface kernel (default: by the grid's size, 0, 4 or 8);
  * "iface_overlap" = 1 runs the interface kernel of RK stages 2 and 3 on a
  * second stream from the end of the previous stage's source kernel (beside
  * its x solve, Poisson solve and correction), 2 from the start of its

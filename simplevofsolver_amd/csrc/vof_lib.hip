@@ -233,6 +233,7 @@ struct vof_ctx {
   int lines_lpb;                         // lines per work-group of the x solver (0 = auto)
   int rhs_rows;                          // rows marched per thread by the source kernel (1 = one DOF per thread)
   int iface_planes;                      // z planes marched per work-group by the 3D interface kernel (0 = blocks)
+  bool rhs_auto, iface_auto;             // the two above are tile_rules' choice, not the caller's
   int fft_radix;                         // 16: 256-point transforms on the register radix-16 path; 4: mixed radix
   int thomas_rows;                       // rows per prefetched chunk of the spectral Thomas kernel (8, 16, 32)
   int thomas_part;                       // 1: partitioned spectral x solve (k_thomas_part) where 4 <= nx <= 256
@@ -994,6 +995,38 @@ static std::vector<double2> make_twiddles(int n) {
 // k_thomas_spec; 33024 lines 255 against 194)
 static bool thomas_seq_lines(size_t nlines) { return nlines <= 16384; }
 
+// rows per thread of the source kernel and planes per work-group of the 3D
+// interface kernel, for cases whose launches run together (one case, or a
+// batch's): 8 where that leaves 16 work-groups of 256 threads per CU, 4 where
+// it leaves 8, else 2 rows from one work-group per CU on, else 1 (no march):
+// each row or plane marched saves re-reading its neighbours, but a grid of
+// few work-groups is bound by the march itself.  Measured, us per launch at
+// 1 / 2 / 4 / 8 rows: 128 x 256 7.4 / 8.0 / 11.1 / 17.2, 256 x 512 9.6 / 8.6 /
+// 11.8 / 18.0, 512 x 1024 20.9 / 18.1 / 18.4 / 20.5, 64 x 32 x 32 9.6 / 10.0 /
+// 14.1 / 23.1, 150 x 135 x 100 128 / 104 / 106 / 111, 128^3 111 / 92 / 88 / 91,
+// 192^3 381 / 300 / 297 / 304, 256^3 904 / 711 / 680 / 674; at 0 / 4 / 8
+// planes: 64 x 32 x 32 14 / 28 / 45, 96^3 35 / 45 / 57, 128^3 64 / 64 / 69,
+// 150 x 135 x 100 59 / 52 / 60, 192^3 162 / 125 / 127, 256^3 343 / 260 / 263.
+static void tile_rules(const std::vector<vof_ctx *> & cs) {
+  const size_t full = 2048, twice = 4096;
+  auto groups = [&](size_t tx, size_t ty, size_t tz) {
+    size_t n = 0;
+    for (const vof_ctx * c : cs) n += ((c->nx + tx - 1) / tx) * ((c->ny + ty - 1) / ty) * ((c->nz + tz - 1) / tz);
+    return n;
+  };
+  const size_t bx = kBlk.x, by = kBlk.y;
+  const int rows = groups(bx, 8 * by, 1) >= twice ? 8 : groups(bx, 4 * by, 1) >= full ? 4
+                   : groups(bx, 2 * by, 1) >= 256 ? 2 : 1;
+  int planes = 0;
+#if NDIMS == 3
+  planes = groups(vofk::kMX, vofk::kMY, 8) >= twice ? 8 : groups(vofk::kMX, vofk::kMY, 4) >= full ? 4 : 0;
+#endif
+  for (vof_ctx * c : cs) {
+    if (c->rhs_auto) c->rhs_rows = rows;
+    if (c->iface_auto) c->iface_planes = planes;
+  }
+}
+
 static int ctx_create(domain_t * domain) {
   vof_ctx * ctx = new vof_ctx();
   domain->info = ctx;
@@ -1023,8 +1056,8 @@ static int ctx_create(domain_t * domain) {
   ctx->poisson_refine = -1;
   ctx->adj_floor = 1e-2;
   ctx->lines_lpb = 0;
-  ctx->rhs_rows = 8;
-  ctx->iface_planes = 8;
+  ctx->rhs_auto = ctx->iface_auto = true;
+  tile_rules({ctx});
   ctx->d_vof_spare = nullptr;
   ctx->vof_bytes = 0;
   for (int m = 0; m < 4; m++) ctx->d_fspare[m] = nullptr;
@@ -2687,11 +2720,13 @@ extern "C" int vof_set_tuning(domain_t * domain, const char name[], int value) {
   if (!strcmp(name, "iface_planes")) {
     if (value != 0 && value != 4 && value != 8 && value != 16) return fail("iface_planes must be 0, 4, 8 or 16");
     ctx->iface_planes = value;
+    ctx->iface_auto = false;
     return 0;
   }
   if (!strcmp(name, "rhs_rows")) {
     if (value != 1 && value != 2 && value != 4 && value != 8 && value != 16) return fail("rhs_rows must be 1, 2, 4, 8 or 16");
     ctx->rhs_rows = value;
+    ctx->rhs_auto = false;
     return 0;
   }
   if (!strcmp(name, "pred_rows")) {
@@ -2925,6 +2960,7 @@ static int batch_create_one(int ncases, const domain_t * const domains[], fluid_
     nt = nt > ncases - 1 ? ncases - 1 : nt;
     if (nt > 0) B->pool.start(nt);
   }
+  tile_rules(B->ctx);
   *out = B;
   return 0;
 }
@@ -3098,6 +3134,7 @@ extern "C" int vof_batch_destroy(vof_batch_t * B) {
   // (upload_tab then refuses to step it) and the call reports the failure.
   int rc = 0;
   for (auto * ctx : B->ctx) {
+    tile_rules({ctx});
     if (!ctx->tab_shared) continue;
     double * h = nullptr;
     double * d = nullptr;
@@ -3283,6 +3320,7 @@ static int tune_run(const std::vector<vof_ctx *> & cs, std::vector<std::unique_p
     return 0;
   };
   std::vector<TuneKnob> knobs = tune_knobs(cs);
+  for (vof_ctx * c : cs) c->rhs_auto = c->iface_auto = false;  // from here on the tuner's choice
   double best = 0.;
   rc = trial(&best);
   if (!rc) {
