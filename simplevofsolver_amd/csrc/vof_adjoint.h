@@ -1,9 +1,14 @@
 // vof_adjoint.h -- reverse-mode (adjoint) kernels of the 2D fused time step.
 //
-// Each kernel is the transpose of the linearisation of one forward stage,
-// written in scatter form: a thread recomputes the forward quantities of the
-// outputs it owns and adds (output adjoint) x (partial derivative) into the
-// adjoints of the inputs it read, with FP64 atomic adds.  Adjoint arrays use
+// Each kernel is the transpose of the linearisation of forward stages.  The
+// linear ones with few neighbours gather (ka_psi_rfft_y, ka_mid), the others
+// scatter: a thread recomputes the forward quantities of the outputs it owns
+// and adds (output adjoint) x (partial derivative) into the adjoints of the
+// inputs it read, with FP64 atomic adds.  A stage is bound by its launches
+// (each kernel takes 3 .. 12 us at 256 x 256), so the parts that do not wait
+// for each other share one: 10 launches in place of 16 kernels and 6 fills,
+// with which a gradient over 20 steps at 256 x 256 took 18.8 ms, now 14.9.  Adjoint
+// arrays use
 // the forward arrays' padded layouts but hold values only on canonical
 // entries: a contribution to a periodic halo image is added to the interior
 // entry it images, one to a Dirichlet wall value (a constant) is dropped,
@@ -59,73 +64,122 @@ __device__ inline void add_m(double * a, int nx, int ny, int i, int j, double vx
   aadd(p + 1, vy);
 }
 
-// ---------------------------------------------------------------------------
-// R1: correction and pressure update (correct_velocity/*.c, update_pressure.c)
+// copies of a stage's vof, ux and uy in one launch
+__global__ void ka_tape(const double * __restrict__ a0, double * __restrict__ b0, size_t n0,
+                        const double * __restrict__ a1, double * __restrict__ b1, size_t n1,
+                        const double * __restrict__ a2, double * __restrict__ b2, size_t n2) {
+  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n0) b0[q] = a0[q];
+  if (q < n1) b1[q] = a1[q];
+  if (q < n2) b2[q] = a2[q];
+}
+
+// R1 and the input of R2.  Correction and pressure update
+// (correct_velocity/*.c, update_pressure.c)
 //   u = u* - pc / dx (psi_c - psi_m),  p += psi - pp / dxf (Lx psi)
-// lambda_u* = lambda_u (in place), lambda_p unchanged; lambda_psi accumulated.
-__global__ void ka_corr(Grid g, double pc, double pp, const double * __restrict__ lux,
-                        const double * __restrict__ luy, const double * __restrict__ lp,
-                        double * __restrict__ lpsi) {
+// lambda_u* = lambda_u (in place), lambda_p unchanged; lambda_psi gathered,
+// and D^-1 lambda_psi (scaled by `scale`) transformed in y as k_div_rfft_y
+// does for the divergence
+template <int ELEMS>
+__global__ __launch_bounds__(vofk::kFftThreads) void ka_psi_rfft_y(
+    Grid g, vofk::FftPlan P, const double2 * __restrict__ tw, double pc, double pp, const double * __restrict__ lux,
+    const double * __restrict__ luy, const double * __restrict__ lp, double scale, double2 * __restrict__ spec) {
+  __shared__ double2 sa[ELEMS], sb[ELEMS];
   const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  if (i >= 2) {
-    const double a = pc / g.dxc[i - 1] * lux[I_UX(i, j, 1)];
-    add_cn(lpsi, nx, ny, i, j, -a);
-    add_cn(lpsi, nx, ny, i - 1, j, +a);
-  }
-  {
-    const double a = pc / g.dy * luy[I_C1(i, j, 1)];
-    add_cn(lpsi, nx, ny, i, j, -a);
-    add_cn(lpsi, nx, ny, i, j - 1, +a);
-  }
-  {
-    const double l = lp[I_C1(i, j, 1)];
-    const double a = pp / g.dxf[i - 1] * l;
+  const int N = g.ny;
+  const int NC = P.cols;
+  const int x0 = blockIdx.x * 2 * NC;
+  for (int e = threadIdx.x; e < 2 * NC * N; e += blockDim.x) {
+    const int xl = e % (2 * NC), j = e / (2 * NC) + 1;
+    // a column past the grid is a copy of the last one (not stored)
+    const int i = min(x0 + xl + 1, nx), im = max(i - 1, 1), ip = min(i + 1, nx);
     const double rm = 1. / g.dxc[i - 1], rp = 1. / g.dxc[i];
-    add_cn(lpsi, nx, ny, i, j, l + a * (rm + rp));
-    add_cn(lpsi, nx, ny, i - 1, j, -a * rm);
-    add_cn(lpsi, nx, ny, i + 1, j, -a * rp);
+    const double uxm = lux[I_UX(max(i, 2), j, 1)], uxp = lux[I_UX(ip, j, 1)];
+    const double uym = luy[I_C1(i, j, 1)], uyp = luy[I_C1(i, wrapj(j + 1, ny), 1)];
+    const double pm = lp[I_C1(im, j, 1)], p0 = lp[I_C1(i, j, 1)], pq = lp[I_C1(ip, j, 1)];
+    const double dxm = g.dxf[im - 1], dx0 = g.dxf[i - 1], dxp = g.dxf[ip - 1];
+    double l = p0 + pp / dx0 * p0 * (rm + rp);
+    l -= i > 1 ? pc / g.dxc[i - 1] * uxm : 0.;
+    l += i < nx ? pc / g.dxc[i] * uxp : 0.;
+    l += pc / g.dy * uyp - pc / g.dy * uym;
+    // the Neumann images of the walls fold back into the cell itself
+    l -= pp / dxm * pm * rm;
+    l -= pp / dxp * pq * rp;
+    const double r = x0 + xl < nx ? scale * (l / dx0) : 0.;
+    double * slot = reinterpret_cast<double *>(&sa[(xl >> 1) * N + j - 1]);
+    slot[xl & 1] = r;
+  }
+  __syncthreads();
+  double2 * res = vofk::lds_fft<double2>(sa, sb, NC, P, tw, -1.);
+  const int nh = N / 2 + 1;
+  for (int e = threadIdx.x; e < NC * nh; e += blockDim.x) {
+    const int c = e / nh, ky = e % nh;
+    const double2 z = res[c * N + ky];
+    const double2 zc = res[c * N + (N - ky) % N];
+    const double2 A = make_double2(0.5 * (z.x + zc.x), 0.5 * (z.y - zc.y));
+    const double2 B = make_double2(0.5 * (z.y + zc.y), -0.5 * (z.x - zc.x));
+    const int xa = x0 + 2 * c, xb = xa + 1;
+    if (xa < nx) spec[(size_t)xa * nh + ky] = A;
+    if (xb < nx) spec[(size_t)xb * nh + ky] = B;
   }
 }
 
-// D^-1 lambda_psi into the interior right-hand side b[(i-1) + nx (j-1)]
-__global__ void ka_psi_rhs(Grid g, const double * __restrict__ lpsi, double * __restrict__ b) {
-  const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  b[(size_t)(i - 1) + (size_t)nx * (size_t)(j - 1)] = lpsi[I_C1(i, j, 1)] / g.dxf[i - 1];
-}
+struct AdjMid {
+  const double * x;       // G D^-1 lambda_psi, with its images
+  double * lux;           // lambda_u*, accumulated
+  double * luy;
+  double * vx;            // D^-1 lambda_u* per DOF: line-major slabs for the x solver
+  double * vy;            // (ux: n = nx - 1 per line, D = DXC; uy: n = nx, D = DXF)
+  double * qx;            // cleared here: the x solver and ka_stage add to them
+  double * qy;
+  double * lnrm;
+  double * lcurv;
+  double * lm;
+  const double * lvof;
+  double * ls;
+  double * cs;
+  double pref, dta, dtb;
+};
 
-// R2: lambda_r = D x (x = G D^-1 lambda_psi); r = pref div u*:
-// lambda_u* += pref div^T lambda_r
-__global__ void ka_div_t(Grid g, double pref, const double * __restrict__ x, double * __restrict__ lux,
-                         double * __restrict__ luy) {
+// what lies between the Poisson and the x-line solves, one thread per cell:
+// R2, lambda_r = D x; r = pref div u*: lambda_u* += pref div^T lambda_r;
+// R3's input; R7, vof_new = vof + dta s + dtb s_prev: lambda_s = dta
+// lambda_vof + carry, new carry dtb lambda_vof (lambda_vof itself passes
+// through unchanged, and nothing else of the stage has added to it yet)
+__global__ void ka_mid(Grid g, AdjMid a) {
   const int nx = g.nx, ny = g.ny;
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
   const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  const double lr = g.dxf[i - 1] * x[I_C1(i, j, 1)];
-  const double ax = pref * lr / g.dxf[i - 1];
-  add_ux(lux, nx, ny, i + 1, j, +ax);
-  add_ux(lux, nx, ny, i, j, -ax);
-  const double ay = pref * lr / g.dy;
-  add_cd(luy, nx, ny, i, j + 1, +ay);
-  add_cd(luy, nx, ny, i, j, -ay);
-}
-
-// R3 input: v = D^-1 lambda_u* per DOF, line-major slabs for the x solver
-// (ux: n = nx - 1 per line, D = DXC; uy: n = nx, D = DXF)
-__global__ void ka_lines_in(Grid g, const double * __restrict__ lux, const double * __restrict__ luy,
-                            double * __restrict__ vx, double * __restrict__ vy) {
-  const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  if (i >= 2) vx[(size_t)(j - 1) * (nx - 1) + (i - 2)] = lux[I_UX(i, j, 1)] / g.dxc[i - 1];
-  vy[(size_t)(j - 1) * nx + (i - 1)] = luy[I_C1(i, j, 1)] / g.dxf[i - 1];
+  if (i > nx + 1 || j > ny) return;
+  {
+    double * m = a.lm + 2 * I_DVOF(i, j, 1);
+    m[0] = 0.;
+    m[1] = 0.;
+  }
+  if (i > nx) return;
+  const double x = a.x[I_C1(i, j, 1)], dx = g.dxf[i - 1];
+  if (i >= 2) {
+    const double dxm = g.dxf[i - 2];
+    const double l = a.lux[I_UX(i, j, 1)] + a.pref * (dxm * a.x[I_C1(i - 1, j, 1)]) / dxm - a.pref * (dx * x) / dx;
+    a.lux[I_UX(i, j, 1)] = l;
+    a.vx[(size_t)(j - 1) * (nx - 1) + (i - 2)] = l / g.dxc[i - 1];
+    a.qx[I_UX(i, j, 1)] = 0.;
+  }
+  {
+    const double l = a.luy[I_C1(i, j, 1)] + a.pref * (dx * a.x[I_C1(i, j - 1, 1)]) / g.dy - a.pref * (dx * x) / g.dy;
+    a.luy[I_C1(i, j, 1)] = l;
+    a.vy[(size_t)(j - 1) * nx + (i - 1)] = l / dx;
+    a.qy[I_C1(i, j, 1)] = 0.;
+  }
+  double * n = a.lnrm + 3 * I_NRM(i, j, 1);
+  n[0] = 0.;
+  n[1] = 0.;
+  n[2] = 0.;
+  a.lcurv[I_C1(i, j, 1)] = 0.;
+  const size_t is = I_SC(i, j, 1);
+  const double l = a.lvof[I_VOF(i, j, 1)];
+  a.ls[is] = a.dta * l + a.cs[is];
+  a.cs[is] = a.dtb * l;
 }
 
 struct AdjRhs {
@@ -140,169 +194,150 @@ struct AdjRhs {
   double * lp;            // lambda_p (accumulates)
   double * csx;           // beta carry of lambda_sa (in: from the next stage, out: to the previous)
   double * csy;
-  double * lfx;           // lambda of the interface force
-  double * lfy;
-  double ca, cb, cg, dif;
+  const double * vof;     // forward quantities of the interface at the stage
+  const double * curv;
+  const double * normal;
+  const double * ls;      // lambda of the vof source
+  double * lvof;
+  double * lcurv;
+  double * lnrm;
+  double ca, cb, cg, dif, tension;
 };
 
 // R4 + R5: lambda_delta = D q; lambda_sa = ca lambda_delta + carry, new carry
 // cb lambda_delta; lambda_sg = cg lambda_delta; then the transposed source
-// stencils of compute_rhs_ux / compute_rhs_uy (predict/ux.c, predict/uy.c)
-__global__ void ka_rhs(Grid g, AdjRhs a) {
+// stencils of compute_rhs_ux / compute_rhs_uy (predict/ux.c, predict/uy.c).
+// Returns lambda_sa, which is also the interface force's.
+__device__ __forceinline__ double rhs_ux_t(const Grid & g, const AdjRhs & a, int i, int j) {
   const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
   const double * ux = a.ux;
   const double * uy = a.uy;
-  if (i >= 2) {
-    const double dxci = g.dxc[i - 1];
-    const size_t is = I_SX(i, j, 1);
-    const double ld = dxci * a.qx[I_UX(i, j, 1)];
-    const double lsa = a.ca * ld + a.csx[is];
-    a.csx[is] = a.cb * ld;
-    const double lsg = a.cg * ld;
-    a.lfx[is] = lsa;
-    const double u_c = ux[I_UX(i, j, 1)];
-    const double u_xm = ux[I_UX(i - 1, j, 1)], u_xp = ux[I_UX(i + 1, j, 1)];
-    const double u_ym = ux[I_UX(i, j - 1, 1)], u_yp = ux[I_UX(i, j + 1, 1)];
-    double d_xm = 0., d_c = 0., d_xp = 0., d_ym = 0., d_yp = 0.;
-    {  // advection_x
-      const double l = +0.5 / dxci * (+0.5 * u_xm + 0.5 * u_c);
-      const double u = -0.5 / dxci * (+0.5 * u_c + 0.5 * u_xp);
-      d_xm += l + (u_xm - u_c) * (0.25 / dxci);
-      d_c += -l - u + (u_xm - u_c) * (0.25 / dxci) - (u_xp - u_c) * (0.25 / dxci);
-      d_xp += u - (u_xp - u_c) * (0.25 / dxci);
-    }
-    const double w_xm = 0.5 * g.dxf[i - 2] / dxci;
-    const double w_xp = 0.5 * g.dxf[i - 1] / dxci;
-    {  // advection_y
-      const double uy_l = w_xm * uy[I_C1(i - 1, j, 1)] + w_xp * uy[I_C1(i, j, 1)];
-      const double uy_u = w_xm * uy[I_C1(i - 1, j + 1, 1)] + w_xp * uy[I_C1(i, j + 1, 1)];
-      const double l = +0.5 / g.dy * uy_l;
-      const double u = -0.5 / g.dy * uy_u;
-      d_ym += l;
-      d_c += -l - u;
-      d_yp += u;
-      const double bl = lsa * (u_ym - u_c) * (0.5 / g.dy);
-      const double bu = lsa * (u_yp - u_c) * (-0.5 / g.dy);
-      add_cd(a.luy, nx, ny, i - 1, j, bl * w_xm);
-      add_cd(a.luy, nx, ny, i, j, bl * w_xp);
-      add_cd(a.luy, nx, ny, i - 1, j + 1, bu * w_xm);
-      add_cd(a.luy, nx, ny, i, j + 1, bu * w_xp);
-    }
-    {  // diffusion_y
-      const double ly = +1. / g.dy / g.dy, cy = -2. / g.dy / g.dy;
-      d_ym += a.dif * ly;
-      d_c += a.dif * cy;
-      d_yp += a.dif * ly;
-    }
-    const double * L = a.lapx_ux + 3 * (i - 2);
-    add_ux(a.lux, nx, ny, i - 1, j, lsa * d_xm + lsg * a.dif * L[0]);
-    add_ux(a.lux, nx, ny, i, j, lsa * d_c + lsg * a.dif * L[1]);
-    add_ux(a.lux, nx, ny, i + 1, j, lsa * d_xp + lsg * a.dif * L[2]);
-    add_ux(a.lux, nx, ny, i, j - 1, lsa * d_ym);
-    add_ux(a.lux, nx, ny, i, j + 1, lsa * d_yp);
-    // sg -= (p_i - p_{i-1}) / dxc
-    add_cn(a.lp, nx, ny, i, j, -lsg / dxci);
-    add_cn(a.lp, nx, ny, i - 1, j, +lsg / dxci);
+  const double dxci = g.dxc[i - 1];
+  const size_t is = I_SX(i, j, 1);
+  const double ld = dxci * a.qx[I_UX(i, j, 1)];
+  const double lsa = a.ca * ld + a.csx[is];
+  a.csx[is] = a.cb * ld;
+  const double lsg = a.cg * ld;
+  const double u_c = ux[I_UX(i, j, 1)];
+  const double u_xm = ux[I_UX(i - 1, j, 1)], u_xp = ux[I_UX(i + 1, j, 1)];
+  const double u_ym = ux[I_UX(i, j - 1, 1)], u_yp = ux[I_UX(i, j + 1, 1)];
+  double d_xm = 0., d_c = 0., d_xp = 0., d_ym = 0., d_yp = 0.;
+  {  // advection_x
+    const double l = +0.5 / dxci * (+0.5 * u_xm + 0.5 * u_c);
+    const double u = -0.5 / dxci * (+0.5 * u_c + 0.5 * u_xp);
+    d_xm += l + (u_xm - u_c) * (0.25 / dxci);
+    d_c += -l - u + (u_xm - u_c) * (0.25 / dxci) - (u_xp - u_c) * (0.25 / dxci);
+    d_xp += u - (u_xp - u_c) * (0.25 / dxci);
+  }
+  const double w_xm = 0.5 * g.dxf[i - 2] / dxci;
+  const double w_xp = 0.5 * g.dxf[i - 1] / dxci;
+  {  // advection_y
+    const double uy_l = w_xm * uy[I_C1(i - 1, j, 1)] + w_xp * uy[I_C1(i, j, 1)];
+    const double uy_u = w_xm * uy[I_C1(i - 1, j + 1, 1)] + w_xp * uy[I_C1(i, j + 1, 1)];
+    const double l = +0.5 / g.dy * uy_l;
+    const double u = -0.5 / g.dy * uy_u;
+    d_ym += l;
+    d_c += -l - u;
+    d_yp += u;
+    const double bl = lsa * (u_ym - u_c) * (0.5 / g.dy);
+    const double bu = lsa * (u_yp - u_c) * (-0.5 / g.dy);
+    add_cd(a.luy, nx, ny, i - 1, j, bl * w_xm);
+    add_cd(a.luy, nx, ny, i, j, bl * w_xp);
+    add_cd(a.luy, nx, ny, i - 1, j + 1, bu * w_xm);
+    add_cd(a.luy, nx, ny, i, j + 1, bu * w_xp);
+  }
+  {  // diffusion_y
+    const double ly = +1. / g.dy / g.dy, cy = -2. / g.dy / g.dy;
+    d_ym += a.dif * ly;
+    d_c += a.dif * cy;
+    d_yp += a.dif * ly;
+  }
+  const double * L = a.lapx_ux + 3 * (i - 2);
+  add_ux(a.lux, nx, ny, i - 1, j, lsa * d_xm + lsg * a.dif * L[0]);
+  add_ux(a.lux, nx, ny, i, j, lsa * d_c + lsg * a.dif * L[1]);
+  add_ux(a.lux, nx, ny, i + 1, j, lsa * d_xp + lsg * a.dif * L[2]);
+  add_ux(a.lux, nx, ny, i, j - 1, lsa * d_ym);
+  add_ux(a.lux, nx, ny, i, j + 1, lsa * d_yp);
+  // sg -= (p_i - p_{i-1}) / dxc
+  add_cn(a.lp, nx, ny, i, j, -lsg / dxci);
+  add_cn(a.lp, nx, ny, i - 1, j, +lsg / dxci);
+  return lsa;
+}
+__device__ __forceinline__ double rhs_uy_t(const Grid & g, const AdjRhs & a, int i, int j) {
+  const int nx = g.nx, ny = g.ny;
+  const double * ux = a.ux;
+  const double * uy = a.uy;
+  const double dxfi = g.dxf[i - 1];
+  const size_t is = I_SC(i, j, 1);
+  const double ld = dxfi * a.qy[I_C1(i, j, 1)];
+  const double lsa = a.ca * ld + a.csy[is];
+  a.csy[is] = a.cb * ld;
+  const double lsg = a.cg * ld;
+  const double v_c = uy[I_C1(i, j, 1)];
+  const double v_xm = uy[I_C1(i - 1, j, 1)], v_xp = uy[I_C1(i + 1, j, 1)];
+  const double v_ym = uy[I_C1(i, j - 1, 1)], v_yp = uy[I_C1(i, j + 1, 1)];
+  double d_xm = 0., d_c = 0., d_xp = 0., d_ym = 0., d_yp = 0.;
+  {  // advection_x
+    const double ux_l = +0.5 * ux[I_UX(i, j - 1, 1)] + 0.5 * ux[I_UX(i, j, 1)];
+    const double ux_u = +0.5 * ux[I_UX(i + 1, j - 1, 1)] + 0.5 * ux[I_UX(i + 1, j, 1)];
+    const double l = +0.5 / dxfi * ux_l;
+    const double u = -0.5 / dxfi * ux_u;
+    d_xm += l;
+    d_c += -l - u;
+    d_xp += u;
+    const double bl = lsa * (v_xm - v_c) * (0.25 / dxfi);
+    const double bu = lsa * (v_xp - v_c) * (-0.25 / dxfi);
+    add_ux(a.lux, nx, ny, i, j - 1, bl);
+    add_ux(a.lux, nx, ny, i, j, bl);
+    add_ux(a.lux, nx, ny, i + 1, j - 1, bu);
+    add_ux(a.lux, nx, ny, i + 1, j, bu);
+  }
+  {  // advection_y
+    const double l = +0.5 / g.dy * (+0.5 * v_ym + 0.5 * v_c);
+    const double u = -0.5 / g.dy * (+0.5 * v_c + 0.5 * v_yp);
+    d_ym += l + (v_ym - v_c) * (0.25 / g.dy);
+    d_c += -l - u + (v_ym - v_c) * (0.25 / g.dy) - (v_yp - v_c) * (0.25 / g.dy);
+    d_yp += u - (v_yp - v_c) * (0.25 / g.dy);
   }
   {
-    const double dxfi = g.dxf[i - 1];
-    const size_t is = I_SC(i, j, 1);
-    const double ld = dxfi * a.qy[I_C1(i, j, 1)];
-    const double lsa = a.ca * ld + a.csy[is];
-    a.csy[is] = a.cb * ld;
-    const double lsg = a.cg * ld;
-    a.lfy[is] = lsa;
-    const double v_c = uy[I_C1(i, j, 1)];
-    const double v_xm = uy[I_C1(i - 1, j, 1)], v_xp = uy[I_C1(i + 1, j, 1)];
-    const double v_ym = uy[I_C1(i, j - 1, 1)], v_yp = uy[I_C1(i, j + 1, 1)];
-    double d_xm = 0., d_c = 0., d_xp = 0., d_ym = 0., d_yp = 0.;
-    {  // advection_x
-      const double ux_l = +0.5 * ux[I_UX(i, j - 1, 1)] + 0.5 * ux[I_UX(i, j, 1)];
-      const double ux_u = +0.5 * ux[I_UX(i + 1, j - 1, 1)] + 0.5 * ux[I_UX(i + 1, j, 1)];
-      const double l = +0.5 / dxfi * ux_l;
-      const double u = -0.5 / dxfi * ux_u;
-      d_xm += l;
-      d_c += -l - u;
-      d_xp += u;
-      const double bl = lsa * (v_xm - v_c) * (0.25 / dxfi);
-      const double bu = lsa * (v_xp - v_c) * (-0.25 / dxfi);
-      add_ux(a.lux, nx, ny, i, j - 1, bl);
-      add_ux(a.lux, nx, ny, i, j, bl);
-      add_ux(a.lux, nx, ny, i + 1, j - 1, bu);
-      add_ux(a.lux, nx, ny, i + 1, j, bu);
-    }
-    {  // advection_y
-      const double l = +0.5 / g.dy * (+0.5 * v_ym + 0.5 * v_c);
-      const double u = -0.5 / g.dy * (+0.5 * v_c + 0.5 * v_yp);
-      d_ym += l + (v_ym - v_c) * (0.25 / g.dy);
-      d_c += -l - u + (v_ym - v_c) * (0.25 / g.dy) - (v_yp - v_c) * (0.25 / g.dy);
-      d_yp += u - (v_yp - v_c) * (0.25 / g.dy);
-    }
-    {
-      const double ly = +1. / g.dy / g.dy, cy = -2. / g.dy / g.dy;
-      d_ym += a.dif * ly;
-      d_c += a.dif * cy;
-      d_yp += a.dif * ly;
-    }
-    const double * L = a.lapx_c + 3 * (i - 1);
-    add_cd(a.luy, nx, ny, i - 1, j, lsa * d_xm + lsg * a.dif * L[0]);
-    add_cd(a.luy, nx, ny, i, j, lsa * d_c + lsg * a.dif * L[1]);
-    add_cd(a.luy, nx, ny, i + 1, j, lsa * d_xp + lsg * a.dif * L[2]);
-    add_cd(a.luy, nx, ny, i, j - 1, lsa * d_ym);
-    add_cd(a.luy, nx, ny, i, j + 1, lsa * d_yp);
-    add_cn(a.lp, nx, ny, i, j, -lsg / g.dy);
-    add_cn(a.lp, nx, ny, i, j - 1, +lsg / g.dy);
+    const double ly = +1. / g.dy / g.dy, cy = -2. / g.dy / g.dy;
+    d_ym += a.dif * ly;
+    d_c += a.dif * cy;
+    d_yp += a.dif * ly;
   }
+  const double * L = a.lapx_c + 3 * (i - 1);
+  add_cd(a.luy, nx, ny, i - 1, j, lsa * d_xm + lsg * a.dif * L[0]);
+  add_cd(a.luy, nx, ny, i, j, lsa * d_c + lsg * a.dif * L[1]);
+  add_cd(a.luy, nx, ny, i + 1, j, lsa * d_xp + lsg * a.dif * L[2]);
+  add_cd(a.luy, nx, ny, i, j - 1, lsa * d_ym);
+  add_cd(a.luy, nx, ny, i, j + 1, lsa * d_yp);
+  add_cn(a.lp, nx, ny, i, j, -lsg / g.dy);
+  add_cn(a.lp, nx, ny, i, j - 1, +lsg / g.dy);
+  return lsa;
 }
 
 // R6: CSF force (force.c:11-66) from the stage's vof and curvature
-__global__ void ka_force(Grid g, double tension, const double * __restrict__ vof,
-                         const double * __restrict__ curv, const double * __restrict__ lfx,
-                         const double * __restrict__ lfy, double * __restrict__ lvof,
-                         double * __restrict__ lcurv) {
+__device__ __forceinline__ void force_x_t(const Grid & g, const AdjRhs & a, int i, int j, double lf) {
   const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  const double v = vof[I_VOF(i, j, 1)];
-  const double cv = curv[I_C1(i, j, 1)];
-  if (i >= 2) {
-    const double l = lfx[I_SX(i, j, 1)] * tension;
-    const double rdx = 1. / g.dxc[i - 1];
-    const double grad = rdx * (-vof[I_VOF(i - 1, j, 1)] + v);
-    const double kappa = 0.5 * (curv[I_C1(i - 1, j, 1)] + cv);
-    add_vof(lvof, nx, ny, i, j, l * rdx * kappa);
-    add_vof(lvof, nx, ny, i - 1, j, -l * rdx * kappa);
-    add_cd(lcurv, nx, ny, i, j, l * grad * 0.5);
-    add_cd(lcurv, nx, ny, i - 1, j, l * grad * 0.5);
-  }
-  {
-    const double l = lfy[I_SC(i, j, 1)] * tension;
-    const double rdy = 1. / g.dy;
-    const double grad = rdy * (-vof[I_VOF(i, j - 1, 1)] + v);
-    const double kappa = 0.5 * (curv[I_C1(i, j - 1, 1)] + cv);
-    add_vof(lvof, nx, ny, i, j, l * rdy * kappa);
-    add_vof(lvof, nx, ny, i, j - 1, -l * rdy * kappa);
-    add_cd(lcurv, nx, ny, i, j, l * grad * 0.5);
-    add_cd(lcurv, nx, ny, i, j - 1, l * grad * 0.5);
-  }
+  const double l = lf * a.tension;
+  const double rdx = 1. / g.dxc[i - 1];
+  const double grad = rdx * (-a.vof[I_VOF(i - 1, j, 1)] + a.vof[I_VOF(i, j, 1)]);
+  const double kappa = 0.5 * (a.curv[I_C1(i - 1, j, 1)] + a.curv[I_C1(i, j, 1)]);
+  add_vof(a.lvof, nx, ny, i, j, l * rdx * kappa);
+  add_vof(a.lvof, nx, ny, i - 1, j, -l * rdx * kappa);
+  add_cd(a.lcurv, nx, ny, i, j, l * grad * 0.5);
+  add_cd(a.lcurv, nx, ny, i - 1, j, l * grad * 0.5);
 }
-
-// R7: vof_new = vof + dta s + dtb s_prev: lambda_s = dta lambda_vof + carry,
-// new carry dtb lambda_vof (lambda_vof itself passes through unchanged)
-__global__ void ka_vof_src(Grid g, double dta, double dtb, const double * __restrict__ lvof,
-                           double * __restrict__ ls, double * __restrict__ cs) {
+__device__ __forceinline__ void force_y_t(const Grid & g, const AdjRhs & a, int i, int j, double lf) {
   const int nx = g.nx, ny = g.ny;
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
-  const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  const size_t is = I_SC(i, j, 1);
-  const double l = lvof[I_VOF(i, j, 1)];
-  ls[is] = dta * l + cs[is];
-  cs[is] = dtb * l;
+  const double l = lf * a.tension;
+  const double rdy = 1. / g.dy;
+  const double grad = rdy * (-a.vof[I_VOF(i, j - 1, 1)] + a.vof[I_VOF(i, j, 1)]);
+  const double kappa = 0.5 * (a.curv[I_C1(i, j - 1, 1)] + a.curv[I_C1(i, j, 1)]);
+  add_vof(a.lvof, nx, ny, i, j, l * rdy * kappa);
+  add_vof(a.lvof, nx, ny, i, j - 1, -l * rdy * kappa);
+  add_cd(a.lcurv, nx, ny, i, j, l * grad * 0.5);
+  add_cd(a.lcurv, nx, ny, i, j - 1, l * grad * 0.5);
 }
 
 // indicator and its derivative in z = n.x + d
@@ -310,74 +345,96 @@ __device__ inline double thinc_h(const double * n, double x, double y) {
   return 1. / (1. + exp(-2. * vofk::kVofBeta * (n[0] * x + n[1] * y + n[2])));
 }
 
-// R8: THINC fluxes (update/flxx.c, flxy.c): a thread owns the x face i and
-// the y face j of cell (i, j); lambda_F from lambda_s, then the upwind
-// cell's vof or (normal, intercept) and the face velocity
-__global__ void ka_flux(Grid g, const double * __restrict__ ux, const double * __restrict__ uy,
-                        const double * __restrict__ vof, const double * __restrict__ normal,
-                        const double * __restrict__ ls, double * __restrict__ lux,
-                        double * __restrict__ luy, double * __restrict__ lvof, double * __restrict__ lnrm) {
+// R8: THINC fluxes (update/flxx.c, flxy.c) of the x face i and of the y face
+// j of cell (i, j); lambda_F from lambda_s, then the upwind cell's vof or
+// (normal, intercept) and the face velocity
+__device__ __forceinline__ void flux_x_t(const Grid & g, const AdjRhs & a, int i, int j) {
   const int nx = g.nx, ny = g.ny;
+  const double beta2 = 2. * vofk::kVofBeta;
+  const double * vof = a.vof;
+  const double * normal = a.normal;
+  const double * ls = a.ls;
+  double * lnrm = a.lnrm;
+  // s(i) += F(i) / dxf(i); s(i-1) -= F(i) / dxf(i-1)
+  const double lF = ls[I_SC(i, j, 1)] / g.dxf[i - 1] - ls[I_SC(i - 1, j, 1)] / g.dxf[i - 2];
+  const double vel = a.ux[I_UX(i, j, 1)];
+  const int ii = vel < 0. ? i : i - 1;
+  const double x = vel < 0. ? -0.5 : +0.5;
+  const double lv = vof[I_VOF(ii, j, 1)];
+  if (lv < vofk::kVofMin || 1. - vofk::kVofMin < lv) {
+    add_ux(a.lux, nx, ny, i, j, lF * lv);
+    add_vof(a.lvof, nx, ny, ii, j, lF * vel);
+  } else {
+    const double * n = normal + 3 * I_NRM(ii, j, 1);
+    double hs = 0., gx = 0., gy = 0., gd = 0.;
+    for (int q = 0; q < NGAUSS; q++) {
+      const double y = vofk::kGaussP[q];
+      const double h = thinc_h(n, x, y);
+      hs += vofk::kGaussW[q] * h;
+      const double c = lF * vel * vofk::kGaussW[q] * beta2 * h * (1. - h);
+      gx += c * x;
+      gy += c * y;
+      gd += c;
+    }
+    add_ux(a.lux, nx, ny, i, j, lF * hs);
+    double * o = lnrm + 3 * I_NRM(ii, wrapj(j, ny), 1);
+    aadd(o, gx);
+    aadd(o + 1, gy);
+    aadd(o + 2, gd);
+  }
+}
+__device__ __forceinline__ void flux_y_t(const Grid & g, const AdjRhs & a, int i, int j) {
+  const int nx = g.nx, ny = g.ny;
+  const double beta2 = 2. * vofk::kVofBeta;
+  const double * vof = a.vof;
+  const double * normal = a.normal;
+  const double * ls = a.ls;
+  double * lnrm = a.lnrm;
+  const double lF = (ls[I_SC(i, j, 1)] - ls[I_SC(i, wrapj(j - 1, ny), 1)]) / g.dy;
+  const double vel = a.uy[I_C1(i, j, 1)];
+  const int jj = vel < 0. ? j : j - 1;
+  const double y = vel < 0. ? -0.5 : +0.5;
+  const double lv = vof[I_VOF(i, jj, 1)];
+  if (lv < vofk::kVofMin || 1. - vofk::kVofMin < lv) {
+    add_cd(a.luy, nx, ny, i, j, lF * lv);
+    add_vof(a.lvof, nx, ny, i, jj, lF * vel);
+  } else {
+    const double * n = normal + 3 * I_NRM(i, jj, 1);
+    double hs = 0., gx = 0., gy = 0., gd = 0.;
+    for (int q = 0; q < NGAUSS; q++) {
+      const double x = vofk::kGaussP[q];
+      const double h = thinc_h(n, x, y);
+      hs += vofk::kGaussW[q] * h;
+      const double c = lF * vel * vofk::kGaussW[q] * beta2 * h * (1. - h);
+      gx += c * x;
+      gy += c * y;
+      gd += c;
+    }
+    add_cd(a.luy, nx, ny, i, j, lF * hs);
+    double * o = lnrm + 3 * I_NRM(i, wrapj(jj, ny), 1);
+    aadd(o, gx);
+    aadd(o + 1, gy);
+    aadd(o + 2, gd);
+  }
+}
+
+// R4 - R6 and R8: blockIdx.z takes ux's sources with the force in x, uy's
+// with the force in y, the x fluxes and the y fluxes.  All add to the same
+// arrays and none reads what another adds to; side by side they fill the
+// chip, which one part's work-groups at 256 x 256 (one per CU) do not
+__global__ void ka_stage(Grid g, AdjRhs a) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
   const int j = (int)(blockIdx.y * blockDim.y + threadIdx.y) + 1;
-  if (i > nx || j > ny) return;
-  const double beta2 = 2. * vofk::kVofBeta;
-  if (i >= 2) {
-    // s(i) += F(i) / dxf(i); s(i-1) -= F(i) / dxf(i-1)
-    const double lF = ls[I_SC(i, j, 1)] / g.dxf[i - 1] - ls[I_SC(i - 1, j, 1)] / g.dxf[i - 2];
-    const double vel = ux[I_UX(i, j, 1)];
-    const int ii = vel < 0. ? i : i - 1;
-    const double x = vel < 0. ? -0.5 : +0.5;
-    const double lv = vof[I_VOF(ii, j, 1)];
-    if (lv < vofk::kVofMin || 1. - vofk::kVofMin < lv) {
-      add_ux(lux, nx, ny, i, j, lF * lv);
-      add_vof(lvof, nx, ny, ii, j, lF * vel);
-    } else {
-      const double * n = normal + 3 * I_NRM(ii, j, 1);
-      double hs = 0., gx = 0., gy = 0., gd = 0.;
-      for (int q = 0; q < NGAUSS; q++) {
-        const double y = vofk::kGaussP[q];
-        const double h = thinc_h(n, x, y);
-        hs += vofk::kGaussW[q] * h;
-        const double c = lF * vel * vofk::kGaussW[q] * beta2 * h * (1. - h);
-        gx += c * x;
-        gy += c * y;
-        gd += c;
-      }
-      add_ux(lux, nx, ny, i, j, lF * hs);
-      double * o = lnrm + 3 * I_NRM(ii, wrapj(j, ny), 1);
-      aadd(o, gx);
-      aadd(o + 1, gy);
-      aadd(o + 2, gd);
-    }
-  }
-  {
-    const double lF = (ls[I_SC(i, j, 1)] - ls[I_SC(i, wrapj(j - 1, ny), 1)]) / g.dy;
-    const double vel = uy[I_C1(i, j, 1)];
-    const int jj = vel < 0. ? j : j - 1;
-    const double y = vel < 0. ? -0.5 : +0.5;
-    const double lv = vof[I_VOF(i, jj, 1)];
-    if (lv < vofk::kVofMin || 1. - vofk::kVofMin < lv) {
-      add_cd(luy, nx, ny, i, j, lF * lv);
-      add_vof(lvof, nx, ny, i, jj, lF * vel);
-    } else {
-      const double * n = normal + 3 * I_NRM(i, jj, 1);
-      double hs = 0., gx = 0., gy = 0., gd = 0.;
-      for (int q = 0; q < NGAUSS; q++) {
-        const double x = vofk::kGaussP[q];
-        const double h = thinc_h(n, x, y);
-        hs += vofk::kGaussW[q] * h;
-        const double c = lF * vel * vofk::kGaussW[q] * beta2 * h * (1. - h);
-        gx += c * x;
-        gy += c * y;
-        gd += c;
-      }
-      add_cd(luy, nx, ny, i, j, lF * hs);
-      double * o = lnrm + 3 * I_NRM(i, wrapj(jj, ny), 1);
-      aadd(o, gx);
-      aadd(o + 1, gy);
-      aadd(o + 2, gd);
-    }
+  if (i > g.nx || j > g.ny) return;
+  switch (blockIdx.z) {
+    case 0:
+      if (i >= 2) force_x_t(g, a, i, j, rhs_ux_t(g, a, i, j));
+      break;
+    case 1: force_y_t(g, a, i, j, rhs_uy_t(g, a, i, j)); break;
+    case 2:
+      if (i >= 2) flux_x_t(g, a, i, j);
+      break;
+    default: flux_y_t(g, a, i, j);
   }
 }
 
@@ -477,39 +534,6 @@ __global__ void ka_gradient(Grid g, double floor, const double * __restrict__ vo
   add_vof(lvof, nx, ny, i, j - 1, +lgx * rdx - lgy * rdy);
   add_vof(lvof, nx, ny, i - 1, j, -lgx * rdx + lgy * rdy);
   add_vof(lvof, nx, ny, i, j, +lgx * rdx + lgy * rdy);
-}
-
-// FFT in y of an interior right-hand side b (scaled by `scale`), as
-// k_div_rfft_y does for the divergence
-template <int ELEMS>
-__global__ __launch_bounds__(vofk::kFftThreads) void ka_vec_rfft_y(
-    Grid g, vofk::FftPlan P, const double2 * __restrict__ tw, const double * __restrict__ b, double scale,
-    double2 * __restrict__ spec) {
-  __shared__ double2 sa[ELEMS], sb[ELEMS];
-  const int nx = g.nx;
-  const int N = g.ny;
-  const int NC = ELEMS / N;
-  const int x0 = blockIdx.x * 2 * NC;
-  for (int e = threadIdx.x; e < 2 * NC * N; e += blockDim.x) {
-    const int xl = e % (2 * NC), j = e / (2 * NC);
-    const int i = x0 + xl;
-    const double r = i < nx ? scale * b[(size_t)i + (size_t)nx * (size_t)j] : 0.;
-    double * slot = reinterpret_cast<double *>(&sa[(xl >> 1) * N + j]);
-    slot[xl & 1] = r;
-  }
-  __syncthreads();
-  double2 * res = vofk::lds_fft<double2>(sa, sb, NC, P, tw, -1.);
-  const int nh = N / 2 + 1;
-  for (int e = threadIdx.x; e < NC * nh; e += blockDim.x) {
-    const int c = e / nh, ky = e % nh;
-    const double2 z = res[c * N + ky];
-    const double2 zc = res[c * N + (N - ky) % N];
-    const double2 A = make_double2(0.5 * (z.x + zc.x), 0.5 * (z.y - zc.y));
-    const double2 B = make_double2(0.5 * (z.y + zc.y), -0.5 * (z.x - zc.x));
-    const int xa = x0 + 2 * c, xb = xa + 1;
-    if (xa < nx) spec[(size_t)xa * nh + ky] = A;
-    if (xb < nx) spec[(size_t)xb * nh + ky] = B;
-  }
 }
 
 }  // namespace vofa

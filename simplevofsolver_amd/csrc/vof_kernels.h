@@ -1637,6 +1637,7 @@ struct FftPlan {
   int n;
   int nst;
   int rad[16];
+  int cols;     // columns per work-group of the launch
 };
 
 // complex element types of the transforms: FP64 (double2) for the plain

@@ -2556,10 +2556,14 @@ static int integrate_fused_stages(const domain_t * domain, fluid_t * fluid, inte
     if (ctx->tape) {
       // the adjoint's recomputation records each stage's input state
       double ** t = ctx->tape + 3 * rk;
-      HIPCHK(hipMemcpyAsync(t[0], interface->vof.data, interface->vof.datasize, hipMemcpyDeviceToDevice,
-                            ctx->stream));
-      HIPCHK(hipMemcpyAsync(t[1], fluid->ux.data, fluid->ux.datasize, hipMemcpyDeviceToDevice, ctx->stream));
-      HIPCHK(hipMemcpyAsync(t[2], fluid->uy.data, fluid->uy.datasize, hipMemcpyDeviceToDevice, ctx->stream));
+#if NDIMS == 2
+      const size_t n0 = interface->vof.datasize / sizeof(double), n1 = fluid->ux.datasize / sizeof(double),
+                   n2 = fluid->uy.datasize / sizeof(double);
+      hipLaunchKernelGGL(vofa::ka_tape, dim3((unsigned)((std::max(n0, std::max(n1, n2)) + 255) / 256)), dim3(256), 0,
+                         ctx->stream, (const double *)interface->vof.data, t[0], n0, (const double *)fluid->ux.data,
+                         t[1], n1, (const double *)fluid->uy.data, t[2], n2);
+      LAUNCHCHK();
+#endif
     }
     // curvature tensor (curvature_tensor.c:178-186)
     if (fz & F_IFACE) {
@@ -3565,16 +3569,27 @@ extern "C" int vof_adjoint_loss(const domain_t * domain, const interface_t * int
   return 0;
 }
 
+// the work arrays of one gradient, in one allocation (one by one the 110 of
+// them at 20 steps were a tenth of the call)
 struct AdjBuf {
-  std::vector<void *> all;
-  int get(double ** p, size_t bytes) {
-    if (hipMalloc(p, bytes) != hipSuccess) return fail("adjoint: allocation of %zu bytes failed", bytes);
-    all.push_back(*p);
+  std::vector<std::pair<double **, size_t>> want;
+  void * mem = nullptr;
+  void get(double ** p, size_t bytes) { want.push_back({p, (bytes + 255) & ~(size_t)255}); }
+  int alloc() {
+    size_t n = 0;
+    for (auto & w : want) n += w.second;
+    if (hipMalloc(&mem, n) != hipSuccess) {
+      mem = nullptr;
+      return fail("adjoint: allocation of %zu bytes failed", n);
+    }
+    char * q = (char *)mem;
+    for (auto & w : want) {
+      *w.first = (double *)q;
+      q += w.second;
+    }
     return 0;
   }
-  ~AdjBuf() {
-    for (void * p : all) dev_free(p);
-  }
+  ~AdjBuf() { dev_free(mem); }
 };
 
 extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, interface_t * interface, int nsteps,
@@ -3602,10 +3617,27 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
   const int nck = (nsteps + every - 1) / every;
   std::vector<double *> ck(4 * (size_t)nck);
   for (int c = 0; c < nck; c++) {
-    if (B.get(&ck[4 * c + 0], bvof) || B.get(&ck[4 * c + 1], bux) || B.get(&ck[4 * c + 2], buy) ||
-        B.get(&ck[4 * c + 3], bp))
-      return 1;
+    B.get(&ck[4 * c + 0], bvof);
+    B.get(&ck[4 * c + 1], bux);
+    B.get(&ck[4 * c + 2], buy);
+    B.get(&ck[4 * c + 3], bp);
   }
+  // tapes of one segment: (vof, ux, uy) per stage
+  std::vector<double *> tape(9 * (size_t)(every < nsteps ? every : nsteps));
+  for (size_t t = 0; t < tape.size(); t += 3) {
+    B.get(&tape[t + 0], bvof);
+    B.get(&tape[t + 1], bux);
+    B.get(&tape[t + 2], buy);
+  }
+  // adjoint state and scratch
+  double *lux, *luy, *lp, *lvof, *lcurv, *lm, *lnrm, *ls, *csx, *csy, *cs, *qx, *qy, *vx, *vy, *x;
+  const size_t bsx = sizeof(double) * (size_t)(nx - 1) * ny, bsc = sizeof(double) * ncell;
+  const std::pair<double **, size_t> scratch[] = {
+      {&lux, bux}, {&luy, buy}, {&lp, bp}, {&lvof, bvof}, {&lcurv, interface->curv.datasize},
+      {&lm, interface->dvof.datasize}, {&lnrm, interface->normal.datasize}, {&ls, bsc}, {&csx, bsx}, {&csy, bsc},
+      {&cs, bsc}, {&qx, bux}, {&qy, buy}, {&vx, bsx}, {&vy, bsc}, {&x, bp}};
+  for (auto & w : scratch) B.get(w.first, w.second);
+  if (B.alloc()) return 1;
   auto save = [&](int c) -> int {
     HIPCHK(hipMemcpyAsync(ck[4 * c + 0], interface->vof.data, bvof, hipMemcpyDeviceToDevice, st));
     HIPCHK(hipMemcpyAsync(ck[4 * c + 1], fluid->ux.data, bux, hipMemcpyDeviceToDevice, st));
@@ -3629,40 +3661,8 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
   std::vector<double> hv(bvof / sizeof(double)), hg;
   HIPCHK(hipMemcpyAsync(hv.data(), interface->vof.data, bvof, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  const double L = loss_of(ctx, domain, hv, &hg);
-  // adjoint state and scratch
-  double *lux, *luy, *lp, *lvof, *lpsi, *lcurv, *lm, *lnrm, *lfx, *lfy, *ls, *csx, *csy, *cs, *qx, *qy, *vx, *vy,
-      *b, *x;
-  const size_t bcurv = interface->curv.datasize, bdvof = interface->dvof.datasize;
-  const size_t bnrm = interface->normal.datasize;
-  if (B.get(&lux, bux) || B.get(&luy, buy) || B.get(&lp, bp) || B.get(&lvof, bvof) || B.get(&lpsi, bp) ||
-      B.get(&lcurv, bcurv) || B.get(&lm, bdvof) || B.get(&lnrm, bnrm) ||
-      B.get(&lfx, sizeof(double) * (size_t)(nx - 1) * ny) || B.get(&lfy, sizeof(double) * ncell) ||
-      B.get(&ls, sizeof(double) * ncell) || B.get(&csx, sizeof(double) * (size_t)(nx - 1) * ny) ||
-      B.get(&csy, sizeof(double) * ncell) || B.get(&cs, sizeof(double) * ncell) || B.get(&qx, bux) ||
-      B.get(&qy, buy) || B.get(&vx, sizeof(double) * (size_t)(nx - 1) * ny) || B.get(&vy, sizeof(double) * ncell) ||
-      B.get(&b, sizeof(double) * ncell) || B.get(&x, bp))
-    return 1;
-  HIPCHK(hipMemsetAsync(lux, 0, bux, st));
-  HIPCHK(hipMemsetAsync(luy, 0, buy, st));
-  HIPCHK(hipMemsetAsync(lp, 0, bp, st));
-  HIPCHK(hipMemsetAsync(csx, 0, sizeof(double) * (size_t)(nx - 1) * ny, st));
-  HIPCHK(hipMemsetAsync(csy, 0, sizeof(double) * ncell, st));
-  HIPCHK(hipMemsetAsync(cs, 0, sizeof(double) * ncell, st));
-  HIPCHK(hipMemcpyAsync(lvof, hg.data(), bvof, hipMemcpyHostToDevice, st));
-  // tapes of one segment: (vof, ux, uy) per stage
-  std::vector<double *> tape(9 * (size_t)every);
-  for (size_t t = 0; t < tape.size(); t += 3) {
-    if (B.get(&tape[t + 0], bvof) || B.get(&tape[t + 1], bux) || B.get(&tape[t + 2], buy)) return 1;
-  }
-  const dim3 blk(64, 4);
-  const dim3 gc((unsigned)((nx + 2 + 63) / 64), (unsigned)((ny + 3) / 4));
-  const Grid g = ctx->grid;
-  const double m_dif = fluid->m_dif;
-  const int NC = 1024 / ny > 0 ? 1024 / ny : 1;
-  const int nbx = (nx + 2 * NC - 1) / (2 * NC);
-  const int use1024 = ny <= 1024;
-  for (int c = nck - 1; c >= 0; c--) {
+  // a segment's stage states, recomputed from its checkpoint
+  auto record = [&](int c) -> int {
     const int s0 = c * every, s1 = s0 + every < nsteps ? s0 + every : nsteps;
     if (restore(c)) return 1;
     for (int n = s0; n < s1; n++) {
@@ -3671,6 +3671,30 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
       ctx->tape = nullptr;
       if (rc) return 1;
     }
+    return 0;
+  };
+  // the last segment needs no gradient yet: it runs while the host forms the loss
+  if (record(nck - 1)) return 1;
+  const double L = loss_of(ctx, domain, hv, &hg);
+  HIPCHK(hipMemsetAsync(lux, 0, bux, st));
+  HIPCHK(hipMemsetAsync(luy, 0, buy, st));
+  HIPCHK(hipMemsetAsync(lp, 0, bp, st));
+  HIPCHK(hipMemsetAsync(csx, 0, bsx, st));
+  HIPCHK(hipMemsetAsync(csy, 0, bsc, st));
+  HIPCHK(hipMemsetAsync(cs, 0, bsc, st));
+  HIPCHK(hipMemcpyAsync(lvof, hg.data(), bvof, hipMemcpyHostToDevice, st));
+  const dim3 blk(64, 4);
+  const dim3 gc((unsigned)((nx + 2 + 63) / 64), (unsigned)((ny + 3) / 4));
+  const Grid g = ctx->grid;
+  const double m_dif = fluid->m_dif;
+  const int use1024 = ny <= 1024;
+  const int NC = (use1024 ? 1024 : 2048) / ny;
+  FftPlan py = ctx->plan_y;
+  py.cols = NC;
+  const int nbx = (nx + 2 * NC - 1) / (2 * NC);
+  for (int c = nck - 1; c >= 0; c--) {
+    const int s0 = c * every, s1 = s0 + every < nsteps ? s0 + every : nsteps;
+    if (c != nck - 1 && record(c)) return 1;
     for (int n = s1 - 1; n >= s0; n--) {
       const double dt = dts[n];
       struct TabsEnd {
@@ -3694,20 +3718,15 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
                            (const double *)interface->dvof.data, (double *)interface->normal.data,
                            (double *)interface->curv.data);
         LAUNCHCHK();
-        // R1 correction / pressure
-        HIPCHK(hipMemsetAsync(lpsi, 0, bp, st));
-        hipLaunchKernelGGL(vofa::ka_corr, gc, blk, 0, st, g, pc, pp, (const double *)lux, (const double *)luy,
-                           (const double *)lp, lpsi);
-        // R2 Poisson: x = G D^-1 lambda_psi, lambda_u* += pref div^T D x
-        hipLaunchKernelGGL(vofa::ka_psi_rhs, gc, blk, 0, st, g, (const double *)lpsi, b);
+        // R1 correction / pressure, R2 Poisson: x = G D^-1 lambda_psi
+#define PSI_ARGS g, py, (const double2 *)ctx->d_twy, pc, pp, (const double *)lux, (const double *)luy, \
+                 (const double *)lp, 1. / (double)ny, ctx->d_spec
         if (use1024) {
-          hipLaunchKernelGGL(vofa::ka_vec_rfft_y<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y,
-                             (const double2 *)ctx->d_twy, (const double *)b, 1. / (double)ny, ctx->d_spec);
+          hipLaunchKernelGGL(vofa::ka_psi_rfft_y<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, PSI_ARGS);
         } else {
-          hipLaunchKernelGGL(vofa::ka_vec_rfft_y<2048>, dim3((nx + 2 * (2048 / ny) - 1) / (2 * (2048 / ny))),
-                             dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y, (const double2 *)ctx->d_twy,
-                             (const double *)b, 1. / (double)ny, ctx->d_spec);
+          hipLaunchKernelGGL(vofa::ka_psi_rfft_y<2048>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, PSI_ARGS);
         }
+#undef PSI_ARGS
         if (launch_thomas<double2>(ctx, "k_thomas_spec", ctx->d_spec, ctx->nh)) return 1;
         if (use1024) {
           hipLaunchKernelGGL(vofk::k_irfft_y_psi<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y,
@@ -3717,12 +3736,29 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
                              dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y, (const double2 *)ctx->d_twy,
                              (const double2 *)ctx->d_spec, x, 1);
         }
-        hipLaunchKernelGGL(vofa::ka_div_t, gc, blk, 0, st, g, pref, (const double *)x, lux, luy);
-        LAUNCHCHK();
+        // R2 lambda_u* += pref div^T D x, R3 input, R7 vof source
+        {
+          vofa::AdjMid a{};
+          a.x = x;
+          a.lux = lux;
+          a.luy = luy;
+          a.vx = vx;
+          a.vy = vy;
+          a.qx = qx;
+          a.qy = qy;
+          a.lnrm = lnrm;
+          a.lcurv = lcurv;
+          a.lm = lm;
+          a.lvof = lvof;
+          a.ls = ls;
+          a.cs = cs;
+          a.pref = pref;
+          a.dta = ca;
+          a.dtb = cb;
+          hipLaunchKernelGGL(vofa::ka_mid, gc, blk, 0, st, g, a);
+          LAUNCHCHK();
+        }
         // R3 x-line solves: q = M^-1 D^-1 lambda_u*
-        hipLaunchKernelGGL(vofa::ka_lines_in, gc, blk, 0, st, g, (const double *)lux, (const double *)luy, vx, vy);
-        HIPCHK(hipMemsetAsync(qx, 0, bux, st));
-        HIPCHK(hipMemsetAsync(qy, 0, buy, st));
         {
           vofk::LineJob lj{};
           lj.nlines = ny;
@@ -3738,10 +3774,7 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
           lj.f[1] = vofk::LineField{ty, nullptr, nullptr, nullptr, vy, qy, nx, nx + 2, 1};
           if (launch_lines(ctx, lj, 2)) return 1;
         }
-        // R7 vof source (before anything else adds to lambda_vof)
-        hipLaunchKernelGGL(vofa::ka_vof_src, gc, blk, 0, st, g, kRk[rk][0] * dt, kRk[rk][1] * dt,
-                           (const double *)lvof, ls, cs);
-        // R4 + R5 predictor sources
+        // R4 + R5 predictor sources, R6 force, R8 fluxes
         {
           vofa::AdjRhs a{};
           a.ux = ux;
@@ -3755,23 +3788,21 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
           a.lp = lp;
           a.csx = csx;
           a.csy = csy;
-          a.lfx = lfx;
-          a.lfy = lfy;
+          a.vof = vof;
+          a.curv = (const double *)interface->curv.data;
+          a.normal = (const double *)interface->normal.data;
+          a.ls = ls;
+          a.lvof = lvof;
+          a.lcurv = lcurv;
+          a.lnrm = lnrm;
           a.ca = ca;
           a.cb = cb;
           a.cg = cg;
           a.dif = m_dif;
-          hipLaunchKernelGGL(vofa::ka_rhs, gc, blk, 0, st, g, a);
+          a.tension = interface->tension;
+          hipLaunchKernelGGL(vofa::ka_stage, dim3(gc.x, gc.y, 4), blk, 0, st, g, a);
         }
-        // R8 fluxes, R6 force, R9-R11 interface geometry
-        HIPCHK(hipMemsetAsync(lnrm, 0, bnrm, st));
-        HIPCHK(hipMemsetAsync(lcurv, 0, bcurv, st));
-        HIPCHK(hipMemsetAsync(lm, 0, bdvof, st));
-        hipLaunchKernelGGL(vofa::ka_flux, gc, blk, 0, st, g, ux, uy, vof, (const double *)interface->normal.data,
-                           (const double *)ls, lux, luy, lvof, lnrm);
-        hipLaunchKernelGGL(vofa::ka_force, gc, blk, 0, st, g, interface->tension, vof,
-                           (const double *)interface->curv.data, (const double *)lfx, (const double *)lfy, lvof,
-                           lcurv);
+        // R9-R11 interface geometry
         hipLaunchKernelGGL(vofa::ka_normal_curv, gc, blk, 0, st, g, vof, (const double *)interface->dvof.data,
                            (const double *)interface->normal.data, (const double *)lnrm, (const double *)lcurv,
                            lvof, lm);
