@@ -1637,7 +1637,7 @@ struct FftPlan {
   int n;
   int nst;
   int rad[16];
-  int cols;     // columns per work-group of the launch
+  int cols;     // columns per work-group of the launch (mixed-radix path)
 };
 
 // complex element types of the transforms: FP64 (double2) for the plain
@@ -1715,16 +1715,19 @@ __device__ inline void fft_stage(const T2 * a, T2 * b, int ncols, int N, int Ns,
     const T2 * in = a + (size_t)col * N;
     T2 * out = b + (size_t)col * N;
     const int kk = jj % Ns;
-    T2 v[R];
+    // the twiddles of a butterfly are loaded together, also where kk = 0 does
+    // not use them: under a branch each load waits for the one before
+    T2 v[R], w[R];
+#pragma unroll
+    for (int r = 1; r < R; r++) w[r] = tw[kk * r * tstride];
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const T2 x = in[jj + r * nb];
-      if (r == 0 || kk == 0) {
-        v[r] = x;
-      } else {
-        const T2 w = tw[kk * r * tstride];
-        const S ws = sign * w.y;
-        v[r] = C::mk(x.x * w.x - x.y * ws, x.x * ws + x.y * w.x);
+      v[r] = x;
+      if (r != 0) {
+        const S ws = sign * w[r].y;
+        const T2 y = C::mk(x.x * w[r].x - x.y * ws, x.x * ws + x.y * w[r].x);
+        v[r] = C::mk(kk == 0 ? x.x : y.x, kk == 0 ? x.y : y.y);
       }
     }
     butterfly<R, T2>(v, sign);
@@ -1806,12 +1809,17 @@ __device__ __forceinline__ void dft16(T2 * v, typename Cx<T2>::S sign) {
 // 16-point DFTs in registers (n = n2 + 16 n1, k = k1 + 16 k2):
 //   pass 1, thread (c, n2): Y[n2][k1] = W^(n2 k1) DFT16_n1(x[n2 + 16 n1])[k1]
 //   pass 2, thread (c, k1): X[k1 + 16 k2] = DFT16_n2(Y[n2][k1])[k2]
-// with W = exp(sign 2 pi i / 256), tw[m] = (cos, sin)(2 pi m / 256).  A
+// with W = exp(sign 2 pi i / 256).  Pass 1 reads the twiddles from an LDS
+// table wl[k1][n2] = W^(n2 k1) (thread t of the work-group brings its entry
+// t), since half of the loads from memory waited for each other: y
+// transforms of 256^3 144 -> 137 and 97 -> 89 us, of 128 x 256 12.4 -> 11.8
+// and 13.0 -> 12.2; FP32, 512 x 256 x 256: inverse y 153 -> 141, z 68 -> 64.  A
 // column is a 16 x 17 matrix (row stride 17: both passes are bank-conflict
 // free); x[n] sits at row n / 16, column n % 16 (f256_in), Y[n2][k1] at
 // (k1, n2) and X[k] at (k % 16, k / 16) (f256_out).  Each thread owns one
 // matrix column in pass 1 and one row in pass 2, so both run in place.
 constexpr int kF256Cols = 8;      // transforms per work-group of the y kernels (16 x columns = 128-byte rows)
+constexpr int kF256ColsS = 2;     // the same on grids of few columns
 constexpr int kF256ColsZ = 16;    // transforms per work-group of the z kernel (every thread of the FFT passes busy)
 constexpr int kF256Stride = 273;  // complex values per column: 16 x 17 plus one, so that the
                                   // columns of a work-group start in different LDS banks
@@ -1819,7 +1827,7 @@ __device__ inline int f256_in(int n) { return (n >> 4) * 17 + (n & 15); }
 __device__ inline int f256_out(int k) { return (k & 15) * 17 + (k >> 4); }
 
 template <class T2>
-__device__ __forceinline__ void fft256(T2 * buf, int ncols, const T2 * __restrict__ tw, typename Cx<T2>::S sign) {
+__device__ __forceinline__ void fft256(T2 * buf, int ncols, const T2 * wl, typename Cx<T2>::S sign) {
   using S = typename Cx<T2>::S;
   for (int t = threadIdx.x; t < ncols * 16; t += blockDim.x) {
     T2 * col = buf + (t >> 4) * kF256Stride;
@@ -1831,10 +1839,11 @@ __device__ __forceinline__ void fft256(T2 * buf, int ncols, const T2 * __restric
 #pragma unroll
     for (int k1 = 0; k1 < 16; k1++) {
       T2 x = v[dft16_slot(k1)];
-      if (k1 != 0 && n2 != 0) {
-        const T2 w = tw[n2 * k1];
+      if (k1 != 0) {
+        const T2 w = wl[k1 * 16 + n2];
         const S ws = sign * w.y;
-        x = Cx<T2>::mk(x.x * w.x - x.y * ws, x.x * ws + x.y * w.x);
+        const T2 y = Cx<T2>::mk(x.x * w.x - x.y * ws, x.x * ws + x.y * w.x);
+        x = Cx<T2>::mk(n2 == 0 ? x.x : y.x, n2 == 0 ? x.y : y.y);
       }
       col[k1 * 17 + n2] = x;
     }
@@ -1854,16 +1863,29 @@ __device__ __forceinline__ void fft256(T2 * buf, int ncols, const T2 * __restric
 
 // column layout of the two transform engines: F256 = the 256-point register
 // path (one padded buffer), else the mixed-radix Stockham path (two buffers)
-template <bool F256> __device__ inline int fft_in(int n) { return F256 ? f256_in(n) : n; }
-template <bool F256> __device__ inline int fft_out(int k) { return F256 ? f256_out(k) : k; }
-template <bool F256, class T2>
+// (F256 is the number of columns per work-group, 0 the mixed-radix path)
+template <int F256> __device__ inline int fft_in(int n) { return F256 ? f256_in(n) : n; }
+template <int F256> __device__ inline int fft_out(int k) { return F256 ? f256_out(k) : k; }
+// this thread's entry of fft256's twiddle table, loaded before the data
+template <int F256, class T2> __device__ __forceinline__ T2 fft_tw(const T2 * __restrict__ tw) {
+  static_assert(kFftThreads == 256, "one twiddle per thread");
+  if constexpr (F256) return tw[(threadIdx.x >> 4) * (threadIdx.x & 15)];
+  return Cx<T2>::mk(0, 0);
+}
+// transforms the columns the work-group has put into a; wt = fft_tw's value,
+// wl = the 256 entries of LDS it goes to
+template <int F256, class T2>
 __device__ __forceinline__ T2 * fft_cols(T2 * a, T2 * b, int ncols, const FftPlan & P,
-                                     const T2 * __restrict__ tw, typename Cx<T2>::S sign) {
+                                     const T2 * __restrict__ tw, T2 * wl, T2 wt, typename Cx<T2>::S sign) {
   if constexpr (F256) {
-    (void)b; (void)P;
-    fft256<T2>(a, ncols, tw, sign);
+    (void)b; (void)P; (void)tw;
+    wl[threadIdx.x] = wt;
+    __syncthreads();
+    fft256<T2>(a, ncols, wl, sign);
     return a;
   } else {
+    (void)wl; (void)wt;
+    __syncthreads();
     return lds_fft<T2>(a, b, ncols, P, tw, sign);
   }
 }
@@ -1873,16 +1895,17 @@ constexpr int kFftElems = 2048;   // complex elements per LDS buffer
 // assign_input (dft.c:315-345) fused with the real transform in y.  Two x
 // columns are packed into one complex column; the r2c halves are separated
 // after the transform.  Output spec[x][k][ky].
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __device__ __forceinline__ void k_div_rfft_y_body(const VBlock & vb, 
     Grid g, const FftPlan & P, const double2 * __restrict__ tw, const double * __restrict__ ux,
     const double * __restrict__ uy, const double * __restrict__ uz, double prefactor,
     double2 * __restrict__ spec) {
-  __shared__ double2 sa[F256 ? kF256Cols * kF256Stride : ELEMS];
-  __shared__ double2 sb[F256 ? 1 : ELEMS];
+  __shared__ double2 sa[F256 ? F256 * kF256Stride : ELEMS];
+  __shared__ double2 sb[F256 ? 256 : ELEMS];
+  const double2 wt = fft_tw<F256>(tw);
   const int nx = g.nx, ny = g.ny;
   const int N = ny;
-  const int NC = F256 ? kF256Cols : ELEMS / N;   // complex columns per block
+  const int NC = F256 ? F256 : P.cols;           // complex columns per block
   const int CS = F256 ? kF256Stride : N;         // LDS column stride
   const Tile3 tile = xcd_tile(vb);
   const int x0 = tile.x * 2 * NC;          // first interior x (0-based)
@@ -1940,8 +1963,7 @@ __device__ __forceinline__ void k_div_rfft_y_body(const VBlock & vb,
       slot[xl & 1] = r;
     }
   }
-  __syncthreads();
-  double2 * res = fft_cols<F256, double2>(sa, sb, NC, P, tw, -1.);
+  double2 * res = fft_cols<F256, double2>(sa, sb, NC, P, tw, sb, wt, -1.);
   const int nh = N / 2 + 1;
   for (int e = threadIdx.x; e < NC * nh; e += blockDim.x) {
     const int c = e / nh, ky = e % nh;
@@ -1956,7 +1978,7 @@ __device__ __forceinline__ void k_div_rfft_y_body(const VBlock & vb,
   }
 }
 
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __global__ __launch_bounds__(kFftThreads) void k_div_rfft_y(
     Grid g, FftPlan P, const double2 * __restrict__ tw, const double * __restrict__ ux,
     const double * __restrict__ uy, const double * __restrict__ uz, double prefactor,
@@ -1966,13 +1988,14 @@ __global__ __launch_bounds__(kFftThreads) void k_div_rfft_y(
 
 #if NDIMS == 3
 // complex transform in z of spec[x][kz][ky] for a run of ky at one x
-template <int ELEMS, class T2, bool F256 = false>
+template <int ELEMS, class T2, int F256 = 0>
 __device__ __forceinline__ void k_fft_z_body(const VBlock & vb, Grid g, const FftPlan & P, const T2 * __restrict__ tw,
                                                       T2 * __restrict__ spec, int nh, typename Cx<T2>::S sign) {
-  __shared__ T2 sa[F256 ? kF256ColsZ * kF256Stride : ELEMS];
-  __shared__ T2 sb[F256 ? 1 : ELEMS];
+  __shared__ T2 sa[F256 ? F256 * kF256Stride : ELEMS];
+  __shared__ T2 sb[F256 ? 256 : ELEMS];
+  const T2 wt = fft_tw<F256>(tw);
   const int N = g.nz;
-  const int NC = F256 ? kF256ColsZ : ELEMS / N;
+  const int NC = F256 ? F256 : P.cols;
   const int CS = F256 ? kF256Stride : N;
   const Tile3 tile = xcd_tile(vb);
   const int ky0 = tile.x * NC;
@@ -1984,6 +2007,7 @@ __device__ __forceinline__ void k_fft_z_body(const VBlock & vb, Grid g, const Ff
 #pragma unroll
     for (int u = 0; u < kFftLoadU; u++) {
       const int e = e0 + u * (int)blockDim.x;
+      // (predicated: with clamped unconditional loads 64 -> 82 us at 256^3)
       const int c = e % NC, kz = e / NC;
       const int ky = ky0 + c;
       v[u] = e < total && ky < nh ? base[(size_t)kz * nh + ky] : Cx<T2>::mk(0, 0);
@@ -1994,17 +2018,16 @@ __device__ __forceinline__ void k_fft_z_body(const VBlock & vb, Grid g, const Ff
       if (e < total) sa[(e % NC) * CS + fft_in<F256>(e / NC)] = v[u];
     }
   }
-  __syncthreads();
   T2 * res;
   if constexpr (F256) {
     using S = typename Cx<T2>::S;
     // the direction as a constant, so the twiddle signs fold
     if (sign < 0)
-      res = fft_cols<true, T2>(sa, sb, NC, P, tw, (S)-1);
+      res = fft_cols<F256, T2>(sa, sb, NC, P, tw, sb, wt, (S)-1);
     else
-      res = fft_cols<true, T2>(sa, sb, NC, P, tw, (S)+1);
+      res = fft_cols<F256, T2>(sa, sb, NC, P, tw, sb, wt, (S)+1);
   } else {
-    res = lds_fft<T2>(sa, sb, NC, P, tw, sign);
+    res = fft_cols<F256, T2>(sa, sb, NC, P, tw, sb, wt, sign);
   }
   for (int e = threadIdx.x; e < NC * N; e += blockDim.x) {
     const int c = e % NC, kz = e / NC;
@@ -2013,7 +2036,7 @@ __device__ __forceinline__ void k_fft_z_body(const VBlock & vb, Grid g, const Ff
   }
 }
 
-template <int ELEMS, class T2, bool F256 = false>
+template <int ELEMS, class T2, int F256 = 0>
 __global__ __launch_bounds__(kFftThreads) void k_fft_z(Grid g, FftPlan P, const T2 * __restrict__ tw,
                                                       T2 * __restrict__ spec, int nh, typename Cx<T2>::S sign) {
   k_fft_z_body<ELEMS, T2, F256>(hw_block(), g, P, tw, spec, nh, sign);
@@ -2687,15 +2710,16 @@ __global__ __launch_bounds__(64) void k_thomas_seq(int n, int nlines, const doub
 
 // inverse real transform in y (c2r: the imaginary parts of the k = 0 and
 // k = n/2 bins do not contribute) and extract_output (dft.c:347-362)
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __device__ __forceinline__ void k_irfft_y_psi_body(const VBlock & vb, 
     Grid g, const FftPlan & P, const double2 * __restrict__ tw, const double2 * __restrict__ spec,
     double * __restrict__ psi, int images) {
-  __shared__ double2 sa[F256 ? kF256Cols * kF256Stride : ELEMS];
-  __shared__ double2 sb[F256 ? 1 : ELEMS];
+  __shared__ double2 sa[F256 ? F256 * kF256Stride : ELEMS];
+  __shared__ double2 sb[F256 ? 256 : ELEMS];
+  const double2 wt = fft_tw<F256>(tw);
   const int nx = g.nx, ny = g.ny;
   const int N = ny;
-  const int NC = F256 ? kF256Cols : ELEMS / N;
+  const int NC = F256 ? F256 : P.cols;
   const int CS = F256 ? kF256Stride : N;
   const Tile3 tile = xcd_tile(vb);
   const int x0 = tile.x * 2 * NC;
@@ -2714,13 +2738,12 @@ __device__ __forceinline__ void k_irfft_y_psi_body(const VBlock & vb,
     double2 As[kFftLoadU], Bs[kFftLoadU];
 #pragma unroll
     for (int u = 0; u < kFftLoadU; u++) {
-      const int e = e0 + u * (int)blockDim.x;
+      // unconditional loads (indices clamped to the grid), all in flight together
+      const int e = min(e0 + u * (int)blockDim.x, total - 1);
       const int c = e / nh, kk = e % nh;
-      const int xa = x0 + 2 * c, xb = xa + 1;
-      As[u] = make_double2(0., 0.);
-      Bs[u] = make_double2(0., 0.);
-      if (e < total && xa < nx) As[u] = spec[((size_t)xa * nz + (k - 1)) * nh + kk];
-      if (e < total && xb < nx) Bs[u] = spec[((size_t)xb * nz + (k - 1)) * nh + kk];
+      const int xa = min(x0 + 2 * c, nx - 1), xb = min(x0 + 2 * c + 1, nx - 1);
+      As[u] = spec[((size_t)xa * nz + (k - 1)) * nh + kk];
+      Bs[u] = spec[((size_t)xb * nz + (k - 1)) * nh + kk];
     }
 #pragma unroll
     for (int u = 0; u < kFftLoadU; u++) {
@@ -2728,6 +2751,7 @@ __device__ __forceinline__ void k_irfft_y_psi_body(const VBlock & vb,
       if (e >= total) break;
       const int c = e / nh, kk = e % nh;
       double2 A = As[u], B = Bs[u];
+      if (x0 + 2 * c + 1 >= nx) B = make_double2(0., 0.);  // an odd nx: the last column has no partner
       if (kk == 0 || 2 * kk == N) { A.y = 0.; B.y = 0.; }
       // Z = A + i B at ky = kk; the conjugates (imaginary parts times -1) at N - kk
       sa[c * CS + fft_in<F256>(kk)] = make_double2(A.x - B.y, A.y + B.x);
@@ -2737,8 +2761,7 @@ __device__ __forceinline__ void k_irfft_y_psi_body(const VBlock & vb,
       }
     }
   }
-  __syncthreads();
-  double2 * res = fft_cols<F256, double2>(sa, sb, NC, P, tw, +1.);
+  double2 * res = fft_cols<F256, double2>(sa, sb, NC, P, tw, sb, wt, +1.);
   for (int e = threadIdx.x; e < 2 * NC * N; e += blockDim.x) {
     const int xl = e % (2 * NC), j = e / (2 * NC);
     const int i = x0 + xl + 1;
@@ -2757,7 +2780,7 @@ __device__ __forceinline__ void k_irfft_y_psi_body(const VBlock & vb,
   }
 }
 
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __global__ __launch_bounds__(kFftThreads) void k_irfft_y_psi(
     Grid g, FftPlan P, const double2 * __restrict__ tw, const double2 * __restrict__ spec,
     double * __restrict__ psi, int images) {
@@ -2777,17 +2800,18 @@ __global__ __launch_bounds__(kFftThreads) void k_irfft_y_psi(
 // mode 0: r = prefactor * div u, stored in rhs when store_rhs (a refinement
 // pass follows); mode 1: r = rhs - A psi.  Then (float)(r * scale) is
 // transformed in y as k_div_rfft_y does.
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __device__ __forceinline__ void k_res_rfft32_y_body(const VBlock & vb, 
     Grid g, const FftPlan & P, const float2 * __restrict__ tw, const double * __restrict__ ux,
     const double * __restrict__ uy, const double * __restrict__ uz, double prefactor, double scale,
     double * __restrict__ rhs, const double * __restrict__ psi, const double * __restrict__ pl,
     const double * __restrict__ pu, int mode, int store_rhs, float2 * __restrict__ spec) {
-  __shared__ float2 sa[F256 ? kF256Cols * kF256Stride : ELEMS];
-  __shared__ float2 sb[F256 ? 1 : ELEMS];
+  __shared__ float2 sa[F256 ? F256 * kF256Stride : ELEMS];
+  __shared__ float2 sb[F256 ? 256 : ELEMS];
+  const float2 wt = fft_tw<F256>(tw);
   const int nx = g.nx, ny = g.ny;
   const int N = ny;
-  const int NC = F256 ? kF256Cols : ELEMS / N;
+  const int NC = F256 ? F256 : P.cols;
   const int CS = F256 ? kF256Stride : N;
   const Tile3 tile = xcd_tile(vb);
   const int x0 = tile.x * 2 * NC;
@@ -2878,8 +2902,7 @@ __device__ __forceinline__ void k_res_rfft32_y_body(const VBlock & vb,
       slot[xl & 1] = r32;
     }
   }
-  __syncthreads();
-  float2 * res = fft_cols<F256, float2>(sa, sb, NC, P, tw, -1.f);
+  float2 * res = fft_cols<F256, float2>(sa, sb, NC, P, tw, sb, wt, -1.f);
   const int nh = N / 2 + 1;
   for (int e = threadIdx.x; e < NC * nh; e += blockDim.x) {
     const int c = e / nh, ky = e % nh;
@@ -2893,7 +2916,7 @@ __device__ __forceinline__ void k_res_rfft32_y_body(const VBlock & vb,
   }
 }
 
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __global__ __launch_bounds__(kFftThreads) void k_res_rfft32_y(
     Grid g, FftPlan P, const float2 * __restrict__ tw, const double * __restrict__ ux,
     const double * __restrict__ uy, const double * __restrict__ uz, double prefactor, double scale,
@@ -2905,15 +2928,16 @@ __global__ __launch_bounds__(kFftThreads) void k_res_rfft32_y(
 
 // inverse real transform in y in FP32; psi = delta (accumulate 0) or
 // psi += delta (accumulate 1) in FP64, with halo images and Neumann walls
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __device__ __forceinline__ void k_irfft32_y_psi_body(const VBlock & vb, 
     Grid g, const FftPlan & P, const float2 * __restrict__ tw, const float2 * __restrict__ spec,
     double * __restrict__ psi, int accumulate) {
-  __shared__ float2 sa[F256 ? kF256Cols * kF256Stride : ELEMS];
-  __shared__ float2 sb[F256 ? 1 : ELEMS];
+  __shared__ float2 sa[F256 ? F256 * kF256Stride : ELEMS];
+  __shared__ float2 sb[F256 ? 256 : ELEMS];
+  const float2 wt = fft_tw<F256>(tw);
   const int nx = g.nx, ny = g.ny;
   const int N = ny;
-  const int NC = F256 ? kF256Cols : ELEMS / N;
+  const int NC = F256 ? F256 : P.cols;
   const int CS = F256 ? kF256Stride : N;
   const Tile3 tile = xcd_tile(vb);
   const int x0 = tile.x * 2 * NC;
@@ -2932,13 +2956,12 @@ __device__ __forceinline__ void k_irfft32_y_psi_body(const VBlock & vb,
     float2 As[kFftLoadU], Bs[kFftLoadU];
 #pragma unroll
     for (int u = 0; u < kFftLoadU; u++) {
-      const int e = e0 + u * (int)blockDim.x;
+      // unconditional loads (indices clamped to the grid), all in flight together
+      const int e = min(e0 + u * (int)blockDim.x, total - 1);
       const int c = e / nh, kk = e % nh;
-      const int xa = x0 + 2 * c, xb = xa + 1;
-      As[u] = make_float2(0.f, 0.f);
-      Bs[u] = make_float2(0.f, 0.f);
-      if (e < total && xa < nx) As[u] = spec[((size_t)xa * nz + (k - 1)) * nh + kk];
-      if (e < total && xb < nx) Bs[u] = spec[((size_t)xb * nz + (k - 1)) * nh + kk];
+      const int xa = min(x0 + 2 * c, nx - 1), xb = min(x0 + 2 * c + 1, nx - 1);
+      As[u] = spec[((size_t)xa * nz + (k - 1)) * nh + kk];
+      Bs[u] = spec[((size_t)xb * nz + (k - 1)) * nh + kk];
     }
 #pragma unroll
     for (int u = 0; u < kFftLoadU; u++) {
@@ -2946,6 +2969,7 @@ __device__ __forceinline__ void k_irfft32_y_psi_body(const VBlock & vb,
       if (e >= total) break;
       const int c = e / nh, kk = e % nh;
       float2 A = As[u], B = Bs[u];
+      if (x0 + 2 * c + 1 >= nx) B = make_float2(0.f, 0.f);  // an odd nx: the last column has no partner
       if (kk == 0 || 2 * kk == N) { A.y = 0.f; B.y = 0.f; }
       sa[c * CS + fft_in<F256>(kk)] = make_float2(A.x - B.y, A.y + B.x);
       if (kk != 0 && 2 * kk != N) {
@@ -2954,8 +2978,7 @@ __device__ __forceinline__ void k_irfft32_y_psi_body(const VBlock & vb,
       }
     }
   }
-  __syncthreads();
-  float2 * res = fft_cols<F256, float2>(sa, sb, NC, P, tw, +1.f);
+  float2 * res = fft_cols<F256, float2>(sa, sb, NC, P, tw, sb, wt, +1.f);
   for (int e = threadIdx.x; e < 2 * NC * N; e += blockDim.x) {
     const int xl = e % (2 * NC), j = e / (2 * NC);
     const int i = x0 + xl + 1;
@@ -2970,7 +2993,7 @@ __device__ __forceinline__ void k_irfft32_y_psi_body(const VBlock & vb,
   }
 }
 
-template <int ELEMS, bool F256 = false>
+template <int ELEMS, int F256 = 0>
 __global__ __launch_bounds__(kFftThreads) void k_irfft32_y_psi(
     Grid g, FftPlan P, const float2 * __restrict__ tw, const float2 * __restrict__ spec,
     double * __restrict__ psi, int accumulate) {

@@ -234,6 +234,7 @@ struct vof_ctx {
   int rhs_rows;                          // rows marched per thread by the source kernel (1 = one DOF per thread)
   int iface_planes;                      // z planes marched per work-group by the 3D interface kernel (0 = blocks)
   bool rhs_auto, iface_auto;             // the two above are tile_rules' choice, not the caller's
+  size_t cols_y, cols_z;                 // transforms that the y and z kernels' launches hold (a batch's together)
   int fft_radix;                         // 16: 256-point transforms on the register radix-16 path; 4: mixed radix
   int thomas_rows;                       // rows per prefetched chunk of the spectral Thomas kernel (8, 16, 32)
   int thomas_part;                       // 1: partitioned spectral x solve (k_thomas_part) where 4 <= nx <= 256
@@ -1021,10 +1022,35 @@ static void tile_rules(const std::vector<vof_ctx *> & cs) {
 #if NDIMS == 3
   planes = groups(vofk::kMX, vofk::kMY, 8) >= twice ? 8 : groups(vofk::kMX, vofk::kMY, 4) >= full ? 4 : 0;
 #endif
+  size_t cy = 0, cz = 0;
+  for (const vof_ctx * c : cs) {
+    cy += ((size_t)c->nx + 1) / 2 * c->nz;
+    cz += (size_t)c->nx * (c->ny / 2 + 1);
+  }
   for (vof_ctx * c : cs) {
     if (c->rhs_auto) c->rhs_rows = rows;
     if (c->iface_auto) c->iface_planes = planes;
+    c->cols_y = cy;
+    c->cols_z = cz;
   }
+}
+
+// transforms per work-group of an FFT kernel whose launch holds `cols` of
+// length n: as many as its LDS takes (`most`), but on grids of few columns so
+// few that 2 work-groups per CU come out, down to 256 elements (one per
+// thread).  A work-group's time is its chain of passes, which more columns
+// lengthen: us per launch, most columns /
+// this rule: 128 x 256 y transforms 11.8 / 8.3 and 12.2 / 8.6, 64 x 32 x 32
+// 11.2 / 7.9, 16.8 / 8.6 and z 9.2 / 7.0, 32 x 48 9.2 / 7.7 and 9.3 / 7.3; 256
+// and 1024 in place of 512 came out the same
+constexpr size_t kFftGroups = 512;
+static int fft_share(int most, size_t cols, int n) {
+  const int least = std::max(1, vofk::kFftThreads / n), share = (int)((cols + kFftGroups - 1) / kFftGroups);
+  return std::min(most, std::max(least, share));
+}
+// the same for the 256-point path, which has two sizes of work-group
+static int f256_share(size_t cols) {
+  return cols < kFftGroups * vofk::kF256Cols ? vofk::kF256ColsS : vofk::kF256Cols;
 }
 
 static int ctx_create(domain_t * domain) {
@@ -2019,13 +2045,18 @@ static int potential_mixed(vof_ctx * ctx, size_t rkstep, double dt, fluid_t * fl
   const int elems = 2048;
   // 256-point transforms take the register radix-16 path, as in potential()
   const bool f256y = ny == 256 && ctx->fft_radix == 16;
-  const int NC = f256y ? vofk::kF256Cols : elems / ny;
+  const int NC = f256y ? f256_share(ctx->cols_y) : fft_share(elems / ny, ctx->cols_y, ny);
+  const bool f256ys = f256y && NC == vofk::kF256ColsS;
+  FftPlan py = ctx->plan_y;
+  py.cols = NC;
   const int nbx = (nx + 2 * NC - 1) / (2 * NC);
   const dim3 gy(nbx, NDIMS == 3 ? nz : 1), bf(vofk::kFftThreads);
 #if NDIMS == 3
   const double * uz = (const double *)fluid->uz.data;
   const bool f256z = nz == 256 && ctx->fft_radix == 16;
-  const int NCz = f256z ? vofk::kF256ColsZ : elems / nz;
+  const int NCz = f256z ? vofk::kF256ColsZ : fft_share(elems / nz, ctx->cols_z, nz);
+  FftPlan pz = ctx->plan_z;
+  pz.cols = NCz;
   const dim3 gz((ctx->nh + NCz - 1) / NCz, nx);
 #else
   const double * uz = nullptr;
@@ -2035,12 +2066,15 @@ static int potential_mixed(vof_ctx * ctx, size_t rkstep, double dt, fluid_t * fl
   for (int pass = 0; pass <= ctx->poisson_refine; pass++) {
     // the FP64 right-hand side is kept only when a refinement pass reads it
     const int store_rhs = ctx->poisson_refine > 0;
-#define RES_ARGS ctx->grid, ctx->plan_y, ctx->d_twy32, (const double *)fluid->ux.data, (const double *)fluid->uy.data, uz, \
+#define RES_ARGS ctx->grid, py, ctx->d_twy32, (const double *)fluid->ux.data, (const double *)fluid->uy.data, uz, \
                  prefactor, scale, ctx->d_delta, (const double *)psi, ctx->d_pl, ctx->d_pu, pass == 0 ? 0 : 1, store_rhs, \
                  ctx->d_spec32
-    if (f256y) {
-      KLB(ctx, "k_res_rfft32_y", vofk::kFftThreads, (vofk::k_res_rfft32_y_body<2048, true>),
-          (vofk::k_res_rfft32_y<2048, true>), gy, bf, 0, RES_ARGS);
+    if (f256ys) {
+      KLB(ctx, "k_res_rfft32_y", vofk::kFftThreads, (vofk::k_res_rfft32_y_body<2048, vofk::kF256ColsS>),
+          (vofk::k_res_rfft32_y<2048, vofk::kF256ColsS>), gy, bf, 0, RES_ARGS);
+    } else if (f256y) {
+      KLB(ctx, "k_res_rfft32_y", vofk::kFftThreads, (vofk::k_res_rfft32_y_body<2048, vofk::kF256Cols>),
+          (vofk::k_res_rfft32_y<2048, vofk::kF256Cols>), gy, bf, 0, RES_ARGS);
     } else {
       KLB(ctx, "k_res_rfft32_y", vofk::kFftThreads, vofk::k_res_rfft32_y_body<2048>, vofk::k_res_rfft32_y<2048>, gy, bf,
           0, RES_ARGS);
@@ -2051,21 +2085,24 @@ static int potential_mixed(vof_ctx * ctx, size_t rkstep, double dt, fluid_t * fl
       if (zp == 1 && launch_thomas<float2>(ctx, "k_thomas_spec32", ctx->d_spec32, nlines)) return 1;
       const float sign = zp == 0 ? -1.f : +1.f;
       if (f256z) {
-        KLB(ctx, "k_fft32_z", vofk::kFftThreads, (vofk::k_fft_z_body<1024, float2, true>),
-            (vofk::k_fft_z<1024, float2, true>), gz, bf, 0, ctx->grid, ctx->plan_z, ctx->d_twz32, ctx->d_spec32,
+        KLB(ctx, "k_fft32_z", vofk::kFftThreads, (vofk::k_fft_z_body<1024, float2, vofk::kF256ColsZ>),
+            (vofk::k_fft_z<1024, float2, vofk::kF256ColsZ>), gz, bf, 0, ctx->grid, pz, ctx->d_twz32, ctx->d_spec32,
             ctx->nh, sign);
       } else {
         KLB(ctx, "k_fft32_z", vofk::kFftThreads, (vofk::k_fft_z_body<2048, float2>), (vofk::k_fft_z<2048, float2>), gz,
-            bf, 0, ctx->grid, ctx->plan_z, ctx->d_twz32, ctx->d_spec32, ctx->nh, sign);
+            bf, 0, ctx->grid, pz, ctx->d_twz32, ctx->d_spec32, ctx->nh, sign);
       }
     }
 #else
     if (launch_thomas<float2>(ctx, "k_thomas_spec32", ctx->d_spec32, nlines)) return 1;
 #endif
-#define IRF32_ARGS ctx->grid, ctx->plan_y, ctx->d_twy32, (const float2 *)ctx->d_spec32, psi, pass == 0 ? 0 : 1
-    if (f256y) {
-      KLB(ctx, "k_irfft32_y_psi", vofk::kFftThreads, (vofk::k_irfft32_y_psi_body<2048, true>),
-          (vofk::k_irfft32_y_psi<2048, true>), gy, bf, 0, IRF32_ARGS);
+#define IRF32_ARGS ctx->grid, py, ctx->d_twy32, (const float2 *)ctx->d_spec32, psi, pass == 0 ? 0 : 1
+    if (f256ys) {
+      KLB(ctx, "k_irfft32_y_psi", vofk::kFftThreads, (vofk::k_irfft32_y_psi_body<2048, vofk::kF256ColsS>),
+          (vofk::k_irfft32_y_psi<2048, vofk::kF256ColsS>), gy, bf, 0, IRF32_ARGS);
+    } else if (f256y) {
+      KLB(ctx, "k_irfft32_y_psi", vofk::kFftThreads, (vofk::k_irfft32_y_psi_body<2048, vofk::kF256Cols>),
+          (vofk::k_irfft32_y_psi<2048, vofk::kF256Cols>), gy, bf, 0, IRF32_ARGS);
     } else {
       KLB(ctx, "k_irfft32_y_psi", vofk::kFftThreads, vofk::k_irfft32_y_psi_body<2048>, vofk::k_irfft32_y_psi<2048>, gy,
           bf, 0, IRF32_ARGS);
@@ -2086,7 +2123,10 @@ static int potential(const domain_t * domain, size_t rkstep, double dt, fluid_t 
   // 256-point transforms take the register radix-16 path (8 columns per
   // work-group in y, 16 in z), other lengths the mixed-radix Stockham path
   const bool f256y = ny == 256 && ctx->fft_radix == 16;
-  const int NC = f256y ? vofk::kF256Cols : elems / ny;
+  const int NC = f256y ? f256_share(ctx->cols_y) : fft_share(elems / ny, ctx->cols_y, ny);
+  const bool f256ys = f256y && NC == vofk::kF256ColsS;
+  FftPlan py = ctx->plan_y;
+  py.cols = NC;
   const int nbx = (nx + 2 * NC - 1) / (2 * NC);
   const dim3 gy(nbx, NDIMS == 3 ? nz : 1), bf(vofk::kFftThreads);
 #if NDIMS == 3
@@ -2094,11 +2134,14 @@ static int potential(const domain_t * domain, size_t rkstep, double dt, fluid_t 
 #else
   const double * uz = nullptr;
 #endif
-#define DIV_ARGS ctx->grid, ctx->plan_y, ctx->d_twy, (const double *)fluid->ux.data, (const double *)fluid->uy.data, uz, \
+#define DIV_ARGS ctx->grid, py, ctx->d_twy, (const double *)fluid->ux.data, (const double *)fluid->uy.data, uz, \
                  prefactor, ctx->d_spec
-  if (f256y) {
-    KLB(ctx, "k_div_rfft_y", vofk::kFftThreads, (vofk::k_div_rfft_y_body<1024, true>), (vofk::k_div_rfft_y<1024, true>), gy,
-        bf, 0, DIV_ARGS);
+  if (f256ys) {
+    KLB(ctx, "k_div_rfft_y", vofk::kFftThreads, (vofk::k_div_rfft_y_body<1024, vofk::kF256ColsS>),
+        (vofk::k_div_rfft_y<1024, vofk::kF256ColsS>), gy, bf, 0, DIV_ARGS);
+  } else if (f256y) {
+    KLB(ctx, "k_div_rfft_y", vofk::kFftThreads, (vofk::k_div_rfft_y_body<1024, vofk::kF256Cols>),
+        (vofk::k_div_rfft_y<1024, vofk::kF256Cols>), gy, bf, 0, DIV_ARGS);
   } else if (elems == 1024) {
     KLB(ctx, "k_div_rfft_y", vofk::kFftThreads, vofk::k_div_rfft_y_body<1024>, vofk::k_div_rfft_y<1024>, gy, bf, 0, DIV_ARGS);
   } else {
@@ -2107,7 +2150,9 @@ static int potential(const domain_t * domain, size_t rkstep, double dt, fluid_t 
 #undef DIV_ARGS
 #if NDIMS == 3
   const bool f256z = nz == 256 && ctx->fft_radix == 16;
-  const int NCz = f256z ? vofk::kF256ColsZ : elems / nz;
+  const int NCz = f256z ? vofk::kF256ColsZ : fft_share(elems / nz, ctx->cols_z, nz);
+  FftPlan pz = ctx->plan_z;
+  pz.cols = NCz;
   const dim3 gz((ctx->nh + NCz - 1) / NCz, nx);
   for (int pass = 0; pass < 2; pass++) {
     if (pass == 1) {
@@ -2116,14 +2161,14 @@ static int potential(const domain_t * domain, size_t rkstep, double dt, fluid_t 
     }
     const double sign = pass == 0 ? -1. : +1.;
     if (f256z) {
-      KLB(ctx, "k_fft_z", vofk::kFftThreads, (vofk::k_fft_z_body<1024, double2, true>), (vofk::k_fft_z<1024, double2, true>),
-          gz, bf, 0, ctx->grid, ctx->plan_z, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
+      KLB(ctx, "k_fft_z", vofk::kFftThreads, (vofk::k_fft_z_body<1024, double2, vofk::kF256ColsZ>), (vofk::k_fft_z<1024, double2, vofk::kF256ColsZ>),
+          gz, bf, 0, ctx->grid, pz, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
     } else if (elems == 1024) {
       KLB(ctx, "k_fft_z", vofk::kFftThreads, (vofk::k_fft_z_body<1024, double2>), (vofk::k_fft_z<1024, double2>), gz, bf, 0,
-          ctx->grid, ctx->plan_z, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
+          ctx->grid, pz, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
     } else {
       KLB(ctx, "k_fft_z", vofk::kFftThreads, (vofk::k_fft_z_body<2048, double2>), (vofk::k_fft_z<2048, double2>), gz, bf, 0,
-          ctx->grid, ctx->plan_z, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
+          ctx->grid, pz, ctx->d_twz, ctx->d_spec, ctx->nh, sign);
     }
   }
 #else
@@ -2132,10 +2177,13 @@ static int potential(const domain_t * domain, size_t rkstep, double dt, fluid_t 
     if (launch_thomas<double2>(ctx, "k_thomas_spec", ctx->d_spec, ctx->nh * nz)) return 1;
   }
 #endif
-#define IRF_ARGS ctx->grid, ctx->plan_y, ctx->d_twy, ctx->d_spec, (double *)fluid->psi.data, images
-  if (f256y) {
-    KLB(ctx, "k_irfft_y_psi", vofk::kFftThreads, (vofk::k_irfft_y_psi_body<1024, true>), (vofk::k_irfft_y_psi<1024, true>),
-        gy, bf, 0, IRF_ARGS);
+#define IRF_ARGS ctx->grid, py, ctx->d_twy, ctx->d_spec, (double *)fluid->psi.data, images
+  if (f256ys) {
+    KLB(ctx, "k_irfft_y_psi", vofk::kFftThreads, (vofk::k_irfft_y_psi_body<1024, vofk::kF256ColsS>),
+        (vofk::k_irfft_y_psi<1024, vofk::kF256ColsS>), gy, bf, 0, IRF_ARGS);
+  } else if (f256y) {
+    KLB(ctx, "k_irfft_y_psi", vofk::kFftThreads, (vofk::k_irfft_y_psi_body<1024, vofk::kF256Cols>),
+        (vofk::k_irfft_y_psi<1024, vofk::kF256Cols>), gy, bf, 0, IRF_ARGS);
   } else if (elems == 1024) {
     KLB(ctx, "k_irfft_y_psi", vofk::kFftThreads, vofk::k_irfft_y_psi_body<1024>, vofk::k_irfft_y_psi<1024>, gy, bf, 0,
         IRF_ARGS);
@@ -3688,7 +3736,7 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
   const Grid g = ctx->grid;
   const double m_dif = fluid->m_dif;
   const int use1024 = ny <= 1024;
-  const int NC = (use1024 ? 1024 : 2048) / ny;
+  const int NC = fft_share((use1024 ? 1024 : 2048) / ny, ctx->cols_y, ny);
   FftPlan py = ctx->plan_y;
   py.cols = NC;
   const int nbx = (nx + 2 * NC - 1) / (2 * NC);
@@ -3729,11 +3777,11 @@ extern "C" int vof_adjoint_gradient(const domain_t * domain, fluid_t * fluid, in
 #undef PSI_ARGS
         if (launch_thomas<double2>(ctx, "k_thomas_spec", ctx->d_spec, ctx->nh)) return 1;
         if (use1024) {
-          hipLaunchKernelGGL(vofk::k_irfft_y_psi<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y,
+          hipLaunchKernelGGL(vofk::k_irfft_y_psi<1024>, dim3(nbx), dim3(vofk::kFftThreads), 0, st, g, py,
                              (const double2 *)ctx->d_twy, (const double2 *)ctx->d_spec, x, 1);
         } else {
-          hipLaunchKernelGGL(vofk::k_irfft_y_psi<2048>, dim3((nx + 2 * (2048 / ny) - 1) / (2 * (2048 / ny))),
-                             dim3(vofk::kFftThreads), 0, st, g, ctx->plan_y, (const double2 *)ctx->d_twy,
+          hipLaunchKernelGGL(vofk::k_irfft_y_psi<2048>, dim3(nbx),
+                             dim3(vofk::kFftThreads), 0, st, g, py, (const double2 *)ctx->d_twy,
                              (const double2 *)ctx->d_spec, x, 1);
         }
         // R2 lambda_u* += pref div^T D x, R3 input, R7 vof source
