@@ -991,10 +991,14 @@ static std::vector<double2> make_twiddles(int n) {
 // ---------------------------------------------------------------------------
 // domain
 
-// lines few enough for k_thomas_seq (8 lines per wavefront): up to two
-// wavefronts per SIMD (513 lines of 512 rows: 28 us against 141 for
-// k_thomas_spec; 33024 lines 255 against 194)
-static bool thomas_seq_lines(size_t nlines) { return nlines <= 16384; }
+// lines few enough for k_thomas_seq: it shortens the chain of a line, but with
+// a wavefront per 8 lines it also issues more, which counts once the lines
+// fill the chip.  One solve alone, kept factors / k_thomas_spec: 513 lines of
+// 512 rows 28 / 141 us, 6800 of 300 rows 35 / 86, 33024 of 512 255 / 194.  Three
+// solves on three streams: 6120 lines of 300 rows 122 / 123 us per solve, but
+// 6125 of 512 (FP32) 179 / 172, 8208 of 270 149 / 143, 14040 of 291 (FP32, one
+// refinement) 503 / 475, 15150 of 400 456 / 418
+static bool thomas_seq_lines(size_t nlines) { return nlines <= 3072; }
 
 // rows per thread of the source kernel and planes per work-group of the 3D
 // interface kernel, for cases whose launches run together (one case, or a
