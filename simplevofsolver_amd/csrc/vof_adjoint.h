@@ -7,8 +7,8 @@
 // inputs it read, with FP64 atomic adds.  A stage is bound by its launches
 // (each kernel takes 3 .. 12 us at 256 x 256), so the parts that do not wait
 // for each other share one: 10 launches in place of 16 kernels and 6 fills,
-// with which a gradient over 20 steps at 256 x 256 took 18.8 ms, now 14.9.  Adjoint
-// arrays use
+// with which a gradient over 20 steps at 256 x 256 took 18.8 ms, then 14.9
+// (13.7 with the transforms' narrower work-groups).  Adjoint arrays use
 // the forward arrays' padded layouts but hold values only on canonical
 // entries: a contribution to a periodic halo image is added to the interior
 // entry it images, one to a Dirichlet wall value (a constant) is dropped,
