@@ -145,3 +145,20 @@ def test_batch_autotune_restores_state_and_keeps_results(tmp_path):
         batch.close()
         for s in singles + members:
             s.close()
+
+
+@pytest.mark.parametrize("glsizes", [(32, 48), (16, 12, 20)])
+def test_autotune_baseline_is_a_step(glsizes, tmp_path):
+    """The figure that the candidates of a new solver are held against is that
+    of a step: not half again what the fastest candidate takes (the tile
+    parameters change a step of these grids by a few per cent; with the step
+    graph's build in it the first trial showed several times a step)."""
+    for k in range(2):
+        g = sva.solver_from_ic(random_fields(glsizes, seed=91 + k, uniformx=False), str(tmp_path / str(k)))
+        try:
+            rep = g.autotune(steps=1)
+        finally:
+            g.close()
+        assert rep[0][0] == "start"
+        fastest = min(ms for name, _, ms in rep[1:] if not name.startswith("best:"))
+        assert rep[0][2] < 1.5 * fastest, rep[:4]
