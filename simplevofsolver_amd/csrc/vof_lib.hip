@@ -4479,7 +4479,10 @@ __global__ __launch_bounds__(256) void k_tdm_long(int n, int nrhs, int periodic,
 #if !defined(__HIP_DEVICE_COMPILE__)
 // lines per work-group of k_tdm_lines: as the predictor's (48 (line, chunk)
 // pairs of a system, fewer where that leaves compute units idle), within 64
-// KiB of LDS; 0 where one line does not fit
+// KiB of LDS; 0 where the rows of one line do not fit.  One line alone may
+// take its padding to whole segments past that (the launch takes up to the
+// chip's 160 KiB): 64 lines of 8191 real rows 2.9 ms with one lane per line
+// in LDS, 3.8 by k_tdm_long, 0.87 so; 4095 complex rows 1.47, 1.81, 0.60
 static int tdm_lines_per_group(int n, int ncomp, int nrhs) {
   const int nch = (n + 63) / 64;
   const long want = (long)nrhs * ncomp / 256;
@@ -4489,7 +4492,7 @@ static int tdm_lines_per_group(int n, int ncomp, int nrhs) {
   if (lpb > 48 / (nch * ncomp)) lpb = 48 / (nch * ncomp);
   if (lpb < 1) lpb = 1;
   while (lpb > 1 && sizeof(double) * (size_t)(vofk::tdm_stride(n, (int)lpb * ncomp) + 1) * ncomp * lpb > 65536) lpb--;
-  return sizeof(double) * (size_t)(vofk::tdm_stride(n, ncomp) + 1) * ncomp <= 65536 ? (int)lpb : 0;
+  return sizeof(double) * (size_t)(n | 1) * ncomp <= 65536 ? (int)lpb : 0;
 }
 
 // the table and line kernels of one solve on `st`

@@ -79,6 +79,42 @@ def test_tdm_matches_oracle(n, nrhs, periodic, cplx):
     assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("n", [4080, 4081, 4095, 4096, 4097, 4098, 8176, 8177, 8191, 8192])
+@pytest.mark.parametrize("periodic", [False, True], ids=["thomas", "periodic"])
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+def test_tdm_at_the_edges_of_the_lds_line(n, periodic, cplx):
+    """Whole and partial 16-row segments up to the longest line of 64 KiB
+    (8191 real rows, 4095 complex ones) and past it, and both sides of the
+    longest correction vector swept in LDS (4096 rows, 4097 with the last)."""
+    test_tdm_matches_oracle(n, 5, periodic, cplx)
+
+
+@pytest.mark.parametrize("n,fits,cplx", [(8177, 8176, False), (8191, 8176, False), (4081, 4080, True),
+                                         (4095, 4080, True)])
+def test_tdm_longest_lds_lines_cost_as_their_neighbours(n, fits, cplx):
+    """Lines of up to 64 KiB are swept in LDS: the last partial segment costs
+    no more than half again the whole ones before it (one lane per line in
+    global memory takes 3 times as long)."""
+    import time
+
+    def best(m):
+        t = sva.Tdm(m, 64, False, cplx)
+        t.l[:], t.c[:], t.u[:] = 1.0, -2.5, 1.0
+        buf = DeviceBuffer.from_array(np.ones((64, m), dtype=np.complex128 if cplx else np.float64))
+        try:
+            took = []
+            for _ in range(8):
+                t0 = time.perf_counter()
+                t.solve(buf.ptr)             # waits for its stream
+                took.append(time.perf_counter() - t0)
+            return min(took)
+        finally:
+            t.destruct()
+            buf.free()
+
+    assert best(n) < 1.5 * best(fits)
+
+
 @pytest.mark.parametrize("n", [8, 256, 512])
 @pytest.mark.parametrize("periodic", [False, True], ids=["neumann", "periodic"])
 @pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
