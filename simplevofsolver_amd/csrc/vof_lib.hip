@@ -4456,6 +4456,58 @@ template __global__ void k_tdm_lines<1>(int, int, int, int, const double * __res
 template __global__ void k_tdm_lines<2>(int, int, int, int, const double * __restrict__, const double * __restrict__,
                                         const double * __restrict__, double * __restrict__);
 
+// Many lines of few rows: 256 systems per work-group, their run brought into
+// LDS element by element (rows n | 1 apart: distinct banks) and swept there, a
+// lane per system.  k_tdm_lines gives each line a wavefront's chunk of 64
+// rows, most of whose lanes have no row then.  Bound by the launches and the
+// table; us per solve by k_tdm_lines / here: 100000 lines of 2 rows 37.8 /
+// 21.9, complex periodic ones of 5 rows 48.2 / 26.7, 65536 lines of 16 rows
+// 34.1 / 25.8
+constexpr int kTdmShort = 16;   // rows of the longest such line: what the 16-bit reciprocal below is exact for
+template <int NC>
+__global__ __launch_bounds__(256) void k_tdm_short(int n, int nrhs, int periodic, const double * __restrict__ l,
+                                                   const double * __restrict__ u, const double * __restrict__ tab,
+                                                   double * __restrict__ data) {
+  constexpr int kLines = 256 / NC, kLoads = 4;
+  __shared__ double S[256 * (kTdmShort + 1)];
+  const int m = periodic ? n - 1 : n, ld = n | 1;
+  const long j0 = (long)blockIdx.x * kLines;
+  const int lines = (int)min((long)kLines, (long)nrhs - j0), run = lines * n * NC;
+  double * g = data + j0 * (size_t)n * NC;
+  // element e is component e % NC of row (e / NC) % n; the quotient by n from
+  // a 16-bit reciprocal (e / NC < 256 x 16, times its error of at most 15: below 65536)
+  const int inv = (65536 + n - 1) / n;
+  auto at = [&](int e) {
+    const int q = e / NC, line = (q * inv) >> 16;
+    return (line * NC + e % NC) * ld + (q - line * n);
+  };
+  for (int e0 = (int)threadIdx.x; e0 < run; e0 += 256 * kLoads) {
+    double v[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; k++) v[k] = g[min(e0 + 256 * k, run - 1)];
+#pragma unroll
+    for (int k = 0; k < kLoads; k++) S[at(min(e0 + 256 * k, run - 1))] = v[k];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < lines * NC) {
+    double * q = S + (int)threadIdx.x * ld;
+    tdm_sweeps(m, tab, q, 1);
+    if (periodic) {
+      const double * q1 = tdm_q1(tab, m);
+      const double last = tdm_periodic_last(n, tab, l, u, q[n - 1], q[0], q[n - 2]);
+      q[n - 1] = last;
+      for (int i = 0; i < n - 1; i++) q[i] = q[i] + last * q1[i];
+    }
+  }
+  __syncthreads();
+  for (int e = (int)threadIdx.x; e < run; e += 256) g[e] = S[at(e)];
+}
+
+template __global__ void k_tdm_short<1>(int, int, int, const double * __restrict__, const double * __restrict__,
+                                        const double * __restrict__, double * __restrict__);
+template __global__ void k_tdm_short<2>(int, int, int, const double * __restrict__, const double * __restrict__,
+                                        const double * __restrict__, double * __restrict__);
+
 // lines too long for LDS: one lane per system in global memory
 __global__ __launch_bounds__(256) void k_tdm_long(int n, int nrhs, int periodic, int ncomp,
                                                   const double * __restrict__ l, const double * __restrict__ u,
@@ -4482,7 +4534,7 @@ __global__ __launch_bounds__(256) void k_tdm_long(int n, int nrhs, int periodic,
 // KiB of LDS; 0 where the rows of one line do not fit.  One line alone may
 // take its padding to whole segments past that (the launch takes up to the
 // chip's 160 KiB): 64 lines of 8191 real rows 2.9 ms with one lane per line
-// in LDS, 3.8 by k_tdm_long, 0.87 so; 4095 complex rows 1.47, 1.81, 0.60
+// in LDS, 3.8 by k_tdm_long, 0.88 so; 4095 complex rows 1.46, 1.81, 0.44
 static int tdm_lines_per_group(int n, int ncomp, int nrhs) {
   const int nch = (n + 63) / 64;
   const long want = (long)nrhs * ncomp / 256;
@@ -4495,12 +4547,29 @@ static int tdm_lines_per_group(int n, int ncomp, int nrhs) {
   return sizeof(double) * (size_t)(n | 1) * ncomp <= 65536 ? (int)lpb : 0;
 }
 
+// lines from which k_tdm_short runs: 4096 lines of 16 rows take it 25.1 us, 23.6
+// in k_tdm_lines, whose serial rows are shorter; 5000 of them 25.1 and 24.7,
+// 16384 25.2 and 27.0; lines of 2 to 12 rows are the same or faster from 4096 on
+constexpr int kTdmShortLines = 6000;
+
 // the table and line kernels of one solve on `st`
 static int tdm_enqueue(int n, int nrhs, bool periodic, bool cplx, const double * l, const double * c,
                        const double * u, double * tab, void * data, hipStream_t st) {
   const int ncomp = cplx ? 2 : 1;
   hipLaunchKernelGGL(vofk::k_tdm_table, dim3(1), dim3(vofk::kTdmT), 0, st, n, (int)periodic, l, c, u, tab);
   LAUNCHCHK();
+  if (n <= vofk::kTdmShort && nrhs >= kTdmShortLines) {
+    const int per = 256 / ncomp;
+    const dim3 nb((unsigned)(((long)nrhs + per - 1) / per)), b(256);
+    if (cplx)
+      hipLaunchKernelGGL(vofk::k_tdm_short<2>, nb, b, 0, st, n, nrhs, (int)periodic, l, u, (const double *)tab,
+                         (double *)data);
+    else
+      hipLaunchKernelGGL(vofk::k_tdm_short<1>, nb, b, 0, st, n, nrhs, (int)periodic, l, u, (const double *)tab,
+                         (double *)data);
+    LAUNCHCHK();
+    return 0;
+  }
   const int lpb = tdm_lines_per_group(n, ncomp, nrhs);
   if (lpb > 0) {
     const dim3 nb((unsigned)(((long)nrhs + lpb - 1) / lpb)), b(vofk::kWThreads);

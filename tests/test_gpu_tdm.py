@@ -89,30 +89,48 @@ def test_tdm_at_the_edges_of_the_lds_line(n, periodic, cplx):
     test_tdm_matches_oracle(n, 5, periodic, cplx)
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 9, 15, 16, 17])
+@pytest.mark.parametrize("nrhs", [5999, 6000, 6143, 6145])
+@pytest.mark.parametrize("periodic", [False, True], ids=["thomas", "periodic"])
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+def test_tdm_many_short_lines(n, nrhs, periodic, cplx):
+    """Both sides of the limits of rows and lines from which a lane sweeps a
+    system, and work-groups that are not full."""
+    test_tdm_matches_oracle(n, nrhs, periodic, cplx)
+
+
+def _best_time(n, nrhs, periodic, cplx):
+    import time
+    t = sva.Tdm(n, nrhs, periodic, cplx)
+    t.l[:], t.c[:], t.u[:] = 1.0, -2.5, 1.0
+    buf = DeviceBuffer.from_array(np.ones((nrhs, n), dtype=np.complex128 if cplx else np.float64))
+    try:
+        took = []
+        for _ in range(20):
+            t0 = time.perf_counter()
+            t.solve(buf.ptr)             # waits for its stream
+            took.append(time.perf_counter() - t0)
+        return min(took)
+    finally:
+        t.destruct()
+        buf.free()
+
+
+@pytest.mark.parametrize("n,periodic", [(2, False), (5, True)])
+def test_tdm_short_lines_cost_little_more_than_one(n, periodic):
+    """100000 lines of a few rows are 3 to 16 MB: no more than half again the
+    time of one line (their traffic is a few microseconds; a wavefront for
+    each line takes nearly as long again as the call)."""
+    assert _best_time(n, 100000, periodic, True) < 1.5 * _best_time(n, 1, periodic, True)
+
+
 @pytest.mark.parametrize("n,fits,cplx", [(8177, 8176, False), (8191, 8176, False), (4081, 4080, True),
                                          (4095, 4080, True)])
 def test_tdm_longest_lds_lines_cost_as_their_neighbours(n, fits, cplx):
     """Lines of up to 64 KiB are swept in LDS: the last partial segment costs
     no more than half again the whole ones before it (one lane per line in
     global memory takes 3 times as long)."""
-    import time
-
-    def best(m):
-        t = sva.Tdm(m, 64, False, cplx)
-        t.l[:], t.c[:], t.u[:] = 1.0, -2.5, 1.0
-        buf = DeviceBuffer.from_array(np.ones((64, m), dtype=np.complex128 if cplx else np.float64))
-        try:
-            took = []
-            for _ in range(8):
-                t0 = time.perf_counter()
-                t.solve(buf.ptr)             # waits for its stream
-                took.append(time.perf_counter() - t0)
-            return min(took)
-        finally:
-            t.destruct()
-            buf.free()
-
-    assert best(n) < 1.5 * best(fits)
+    assert _best_time(n, 64, False, cplx) < 1.5 * _best_time(fits, 64, False, cplx)
 
 
 @pytest.mark.parametrize("n", [8, 256, 512])
