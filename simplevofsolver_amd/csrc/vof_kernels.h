@@ -1183,12 +1183,30 @@ struct LineGroup {             // the lines of one work-group, uniform
   size_t g0;                   // its first increment
 };
 
-// the increments of pairs p0 + nw u into registers
-__device__ __forceinline__ void lines_load(const LineField & F, const LineGroup & G, int p0, double * v) {
+// the increments of pairs p0 + nw u into registers: F.q's, or (SRC, the
+// per-function entry point) formed from the three sources
+template <bool SRC>
+__device__ __forceinline__ void lines_load(const LineField & F, const LineJob & J, const LineGroup & G, int p0,
+                                           double * v) {
+  size_t g[kWUnroll];
 #pragma unroll
   for (int u = 0; u < kWUnroll; u++) {
     const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
-    v[u] = F.q[G.g0 + (size_t)(l * G.n + min(64 * (p - l * G.nch) + G.lane, G.n - 1))];
+    g[u] = G.g0 + (size_t)(l * G.n + min(64 * (p - l * G.nch) + G.lane, G.n - 1));
+  }
+  if constexpr (SRC) {
+    double a[kWUnroll], b[kWUnroll], c[kWUnroll];
+#pragma unroll
+    for (int u = 0; u < kWUnroll; u++) {
+      a[u] = F.srca[g[u]];
+      b[u] = F.srcb[g[u]];
+      c[u] = F.srcg[g[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kWUnroll; u++) v[u] = +J.ca * a[u] + J.cb * b[u] + J.cg * c[u];
+  } else {
+#pragma unroll
+    for (int u = 0; u < kWUnroll; u++) v[u] = F.q[g[u]];
   }
 }
 // ... and into S (clamped lanes and pairs repeat a value of their wavefront)
@@ -1565,6 +1583,7 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+template <bool SRC>
 __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJob & J, int lpb) {
   extern __shared__ __align__(16) double S[];
   const LineField & F = J.f[vb.y];
@@ -1589,24 +1608,13 @@ __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJo
   // first batch's field rows are loaded with its increments and stay in
   // registers across the sweep (the LDS barriers leave them in flight)
   double v[kWUnroll], f[kWUnroll];
-  lines_load(F, G, w, v);
+  lines_load<SRC>(F, J, G, w, v);
   const SweepHead h = sweep_head(F.tab, G.n, lane);
   lines_field(F, J, G, w, f);
-  if (F.srcg) {
-    // increments formed here from the three sources (per-function entry
-    // point); the slab just read is not used
-#pragma unroll 1
-    for (int p = w; p < G.np; p += G.nw) {
-      const int l = pair_line(p, G.inv), m = min(64 * (p - l * G.nch) + lane, G.n - 1);
-      const size_t g = G.g0 + (size_t)(l * G.n + m);
-      S[l * G.ld + m] = +J.ca * F.srca[g] + J.cb * F.srcb[g] + J.cg * F.srcg[g];
-    }
-  } else {
-    lines_stage(G, S, w, v);
-    for (int p0 = w + step; p0 < G.np; p0 += step) {
-      lines_load(F, G, p0, v);
-      lines_stage(G, S, p0, v);
-    }
+  lines_stage(G, S, w, v);
+  for (int p0 = w + step; p0 < G.np; p0 += step) {
+    lines_load<SRC>(F, J, G, p0, v);
+    lines_stage(G, S, p0, v);
   }
   lds_barrier();
   for (int l = kSwLines * w; l < nl; l += kSwLines * G.nw)
@@ -1619,8 +1627,9 @@ __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJo
   }
 }
 
+template <bool SRC>
 __global__ __launch_bounds__(kWThreads) void k_lines_lds(LineJob J, int lpb) {
-  k_lines_lds_body(hw_block(), J, lpb);
+  k_lines_lds_body<SRC>(hw_block(), J, lpb);
 }
 
 // ---------------------------------------------------------------------------

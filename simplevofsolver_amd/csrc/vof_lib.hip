@@ -1783,8 +1783,11 @@ static int launch_lines(vof_ctx * ctx, vofk::LineJob & lj, int nj) {
   if ((size_t)lpb * row > 65536) lpb = max(1, (int)(65536 / row));
   const size_t shm = (size_t)lpb * row;
   const int ngroups = (lj.nlines + lpb - 1) / lpb;
-  KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body, vofk::k_lines_lds,
-      dim3((unsigned)ngroups, (unsigned)nj), dim3(vofk::kWThreads), shm, lj, lpb);
+  const dim3 g((unsigned)ngroups, (unsigned)nj), b(vofk::kWThreads);
+  if (lj.f[0].srcg)
+    KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body<true>, vofk::k_lines_lds<true>, g, b, shm, lj, lpb);
+  else
+    KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body<false>, vofk::k_lines_lds<false>, g, b, shm, lj, lpb);
   return 0;
 }
 
