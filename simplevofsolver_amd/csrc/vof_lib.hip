@@ -1769,14 +1769,17 @@ static int pred_rows_for(const vof_ctx * ctx, int * xw) {
 static int launch_lines(vof_ctx * ctx, vofk::LineJob & lj, int nj) {
   const int nx = ctx->nx;
   lj.inv_ny = 0xffffffffu / (unsigned)lj.ny + 1u;
-  // lines per work-group: 48 (line, 64-row chunk) pairs, two full batches
-  // of each wavefront's loads and an LDS tile of about 25 KiB, so that six
+  // lines per work-group: two full batches of each wavefront's loads, 48
+  // (line, 64-row chunk) pairs, with an LDS tile of about 25 KiB, so that six
   // work-groups share a CU (256^3: 338 us at 12 lines, 342 at 11, 351 at
-  // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12, 66 at 20); fewer
-  // where that leaves compute units idle (128 x 256: 10.5 us at 4 lines,
-  // 12.4 at 16)
+  // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12 and at 8); one batch
+  // for lines of up to two chunks, whose tile is small either way (100^3:
+  // 37.0 us at 12 lines, 41.4 at 24; 16 x 200 x 200 44.8 at 24, 49.0 at 48;
+  // 128^3 54.0 at 12, 54.5 at 24); fewer where that leaves compute units idle
+  // (128 x 256: 10.5 us at 4 lines, 12.4 at 16)
   const int nch = (nx + 63) / 64;
-  int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(48 / nch, max(4, lj.nlines * nj / 256));
+  const int pairs = nch <= 2 ? 24 : 48;
+  int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(pairs / nch, max(4, lj.nlines * nj / 256));
   lpb = max(1, min(lpb, 64));
   if (sizeof(double) * (nx | 1) > 65536) return fail("x solver: nx = %d exceeds the LDS line tile", nx);
   const size_t row = sizeof(double) * (size_t)vofk::lines_stride(nx);   // at least ux's
