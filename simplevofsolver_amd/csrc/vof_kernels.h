@@ -3082,8 +3082,7 @@ constexpr int kDtU = 16;  // planes per pass of k_dt_partial (a whole 256-plane 
 __device__ __forceinline__ void k_dt_partial_body(const VBlock & vb, Grid g, const double * __restrict__ ux,
                                                             const double * __restrict__ uy,
                                                             const double * __restrict__ uz,
-                                                            double * __restrict__ part,
-                                                            unsigned * __restrict__ ticket, double * __restrict__ out) {
+                                                            double * __restrict__ part) {
   const int nx = g.nx, ny = g.ny;
 #if NDIMS == 2
   (void)uz;
@@ -3142,41 +3141,14 @@ __device__ __forceinline__ void k_dt_partial_body(const VBlock & vb, Grid g, con
 #endif
   }
   m = block_min(m);
-  const unsigned nb = vb.gx * vb.gy * vb.gz, b = vb.x + vb.gx * (vb.y + vb.gy * vb.z);
-  if (!ticket) {
-    if (threadIdx.x == 0) part[b] = m;
-    return;
-  }
-  // One launch instead of two, and no copy of the result: 128 x 256 9.4 us
-  // against 6.5 + 6.8 and a copy's 3 (each with its launch gap), 512 x 1024
-  // 11.8 against 6.8 + 6.7; with 512 work-groups the tickets alone make it 18.
-  // The work-group that takes the last ticket reduces the partial minima
-  // (agent scope: the others may run on another XCD, whose L2 is its own),
-  // writes the result and resets the count for the next launch
-  __shared__ unsigned last;
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(&part[b], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nb - 1u;
-  }
-  __syncthreads();
-  if (!last) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  m = 1.;
-  for (unsigned t = threadIdx.x; t < nb; t += kRedThreads)
-    m = fmin(m, __hip_atomic_load(&part[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  m = block_min(m);
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(out, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (threadIdx.x == 0) part[vb.x + vb.gx * (vb.y + vb.gy * vb.z)] = m;
 }
 
 __global__ __launch_bounds__(kRedThreads) void k_dt_partial(Grid g, const double * __restrict__ ux,
                                                             const double * __restrict__ uy,
                                                             const double * __restrict__ uz,
-                                                            double * __restrict__ part,
-                                                            unsigned * __restrict__ ticket, double * __restrict__ out) {
-  k_dt_partial_body(hw_block(), g, ux, uy, uz, part, ticket, out);
+                                                            double * __restrict__ part) {
+  k_dt_partial_body(hw_block(), g, ux, uy, uz, part);
 }
 
 __device__ __forceinline__ void k_min_final_body(const VBlock & vb, const double * __restrict__ part, int n,

@@ -296,7 +296,6 @@ struct vof_ctx {
   double * d_delta;                      // x1 pencil of increments
   double * d_part;
   int npart;
-  unsigned * d_ticket;                   // work-groups of k_dt_partial that have finished
   double * h_scalar;                     // pinned
   // statistics accumulators (statistics.c), allocated by statistics.init
   double * d_stat[9];
@@ -1277,14 +1276,12 @@ static int ctx_create(domain_t * domain) {
   ctx->npart = 8192;
   // Thomas tables: header 4 + l, val, v
   ctx->tab_stride = 4 + 3 * (size_t)nx;
-  // one block each: reduction partials, a step's tables and k_dt_partial's
-  // count on the device; a scalar and a step's tables in pinned memory
+  // one block each: reduction partials and a step's tables on the device; a
+  // scalar and a step's tables in pinned memory
   {
     const size_t part = (size_t)ctx->npart * vofk::kDiagN, step = ctx->tab_stride * 9;
-    HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * (part + step + 1)));
+    HIPCHK(hipMalloc(&ctx->d_part, sizeof(double) * (part + step)));
     ctx->d_step = ctx->d_part + part;
-    ctx->d_ticket = (unsigned *)(ctx->d_step + step);
-    HIPCHK(hipMemsetAsync(ctx->d_ticket, 0, sizeof(unsigned), ctx->stream));
     HIPCHK(hipHostMalloc(&ctx->h_scalar, sizeof(double) * (64 + step)));
   }
   ctx->tab_rk = 4 * ctx->tab_stride;
@@ -1532,13 +1529,15 @@ static int vbuf_store(vof_ctx * ctx) {
 // fluid_decide_dt (decide_dt.c:104-145)
 static int decide_dt_enqueue(vof_ctx * ctx, const fluid_t * fluid) {
   // 64 x 4 (i, j) tiles, z planes split over gz work-groups so that the
-  // partial minima fit d_part
+  // partial minima fit d_part.  In 2D at most 512 work-groups, whose threads
+  // take their rows 8 at a time: us per call at 128 / 256 / 512 / 1024 / any
+  // number of them 512 x 1024 18.6 / 17.3 / 17.4 / 18.8 / 21.8, 2048 x 2048
+  // 39.4 / 31.3 / 28.3 / 28.4 / 39.9, 8191 x 1024 61 / 42.9 / 38.1 / 37.7 /
+  // 44.0.  In 3D fewer only lose (128^3 34.4 / 29.8 / 27.2 / 27.1 / 27.2)
   const unsigned gx = (unsigned)((ctx->nx + 63) / 64);
   unsigned gy = (unsigned)((ctx->ny + 3) / 4);
   unsigned gz = NDIMS == 3 ? (unsigned)((ctx->nz + 15) / 16) : 1u;
-  if (NDIMS == 2) gy = min(gy, max(1u, 128u / gx));
-  if (NDIMS == 3 && ctx->rec)
-    while (gz > 1 && gx * gy * gz > 256u) gz--;
+  if (NDIMS == 2) gy = min(gy, max(1u, 512u / gx));
   while (gz > 1 && (size_t)gx * gy * gz > (size_t)ctx->npart) gz--;
   while (gy > 1 && (size_t)gx * gy * gz > (size_t)ctx->npart) gy--;
   if ((size_t)gx * gy * gz > (size_t)ctx->npart) return fail("decide_dt: %u x-tiles exceed the partial buffer", gx);
@@ -1548,19 +1547,16 @@ static int decide_dt_enqueue(vof_ctx * ctx, const fluid_t * fluid) {
 #else
   const double * uz = nullptr;
 #endif
-  // up to 256 work-groups the last to finish reduces their minima (every one
-  // takes a ticket from one counter); more of them, which only large 3D grids
-  // have, are reduced by k_min_final.  Either writes the minimum to pinned
-  // host memory: the stream's synchronisation makes it visible, and no copy
-  // is queued.  The cases of a batch record the same launches whatever their
-  // sizes
-  const bool one = nb <= 256 || ctx->rec;
+  // the second kernel writes the minimum to pinned host memory: the stream's
+  // synchronisation makes it visible, and no copy is queued.  (One kernel, whose
+  // last work-group reduces by a ticket counter, is no faster: 16.2 us per
+  // call against 16.3 at 16 x 16, 18.1 against 16.5 at 128 x 256, 25.0
+  // against 17.4 with 512 work-groups)
   KLB(ctx, "k_dt_partial", vofk::kRedThreads, vofk::k_dt_partial_body, vofk::k_dt_partial, dim3(gx, gy, gz),
       dim3(vofk::kRedThreads), 0, ctx->grid, (const double *)fluid->ux.data, (const double *)fluid->uy.data,
-      uz, ctx->d_part, one ? ctx->d_ticket : nullptr, ctx->h_scalar);
-  if (!one)
-    KLB(ctx, "k_min_final", vofk::kRedThreads, vofk::k_min_final_body, vofk::k_min_final, dim3(1),
-        dim3(vofk::kRedThreads), 0, (const double *)ctx->d_part, nb, ctx->h_scalar);
+      uz, ctx->d_part);
+  KLB(ctx, "k_min_final", vofk::kRedThreads, vofk::k_min_final_body, vofk::k_min_final, dim3(1),
+      dim3(vofk::kRedThreads), 0, (const double *)ctx->d_part, nb, ctx->h_scalar);
   return 0;
 }
 
