@@ -79,6 +79,7 @@ ABI_SYMBOLS_COMMON = [
     "statistics", "vof_statistics_output_to", "vof_set_poisson_mixed",
     "vof_batch_create", "vof_batch_integrate", "vof_batch_synchronize", "vof_batch_destroy",
     "vof_autotune", "vof_batch_autotune", "vof_batch_set_graphs", "vof_batch_graph_counts",
+    "vof_graph_counts",
     "vof_integrate_fixed_dt", "vof_device_alloc", "vof_device_free", "vof_device_copy",
     "tdm_solve_noalloc", "vof_set_freeze",
 ]
@@ -139,6 +140,7 @@ def load(ndims: int):
     lib.vof_autotune.argtypes = [vp, vp, vp, C.c_int, C.c_char_p, C.c_size_t]
     lib.vof_batch_autotune.argtypes = [vp, C.c_int, C.c_char_p, C.c_size_t]
     lib.vof_batch_set_graphs.argtypes = [vp, C.c_int]
+    lib.vof_graph_counts.argtypes = [vp] + [C.POINTER(C.c_size_t)] * 3
     lib.vof_batch_graph_counts.argtypes = [vp, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
     lib.vof_nusselt.argtypes = [vp, vp, dp]
     lib.vof_set_poisson_mixed.argtypes = [vp, C.c_int]
@@ -378,6 +380,12 @@ class Solver:
         self._chk(self.lib.vof_autotune(C.byref(self.domain), C.byref(self.fluid), C.byref(self.interface),
                                         int(steps), buf, len(buf)), "vof_autotune")
         return _tune_report(buf)
+
+    def graph_counts(self):
+        """(step graphs built, replayed, refused by the runtime) so far."""
+        n = [C.c_size_t(0) for _ in range(3)]
+        self._chk(self.lib.vof_graph_counts(C.byref(self.domain), *[C.byref(v) for v in n]), "vof_graph_counts")
+        return tuple(v.value for v in n)
 
     def profile(self, on: bool = True):
         self._chk(self.lib.vof_profile(C.byref(self.domain), int(on)), "vof_profile")

@@ -482,6 +482,7 @@ struct StepGraph {
   hipGraphExec_t exec = nullptr;
   bool warm = false;           // a step has run by plain launches
   bool off = false;            // the runtime refused a graph: plain launches from then on
+  size_t captures = 0, launches = 0, refusals = 0;   // graphs built, replayed, refused
 };
 
 static void step_graph_drop(StepGraph * S) {
@@ -2571,13 +2572,18 @@ static int graph_stages(const domain_t * domain, fluid_t * fluid, interface_t * 
       if (e == hipSuccess) S->nodes.push_back(node);
     }
     if (e == hipSuccess) e = hipGraphInstantiate(&S->exec, S->graph, nullptr, nullptr, 0);
+    if (e == hipSuccess) S->captures++;
     S->in = now;
   }
   if (e == hipSuccess) e = hipGraphLaunch(S->exec, ctx->stream);
-  if (e == hipSuccess) return 0;
+  if (e == hipSuccess) {
+    S->launches++;
+    return 0;
+  }
   // nothing of the step has been issued: its recorded launches go out plainly
   (void)hipGetLastError();
   S->off = true;
+  S->refusals++;
   for (LaunchRec & r : now) {
     const hipKernelNodeParams p = node_params(r, args);
     HIPCHK(hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes, ctx->stream));
@@ -3130,6 +3136,15 @@ extern "C" int vof_batch_integrate(vof_batch_t * B, double dts[]) {
   }
   if (dts)
     for (size_t c = 0; c < n; c++) dts[c] = dt[c];
+  return 0;
+}
+
+extern "C" int vof_graph_counts(const domain_t * domain, size_t * captures, size_t * launches, size_t * refusals) {
+  CTX_OR_FAIL(domain);
+  if (!captures || !launches || !refusals) return fail("vof_graph_counts: NULL argument");
+  *captures = ctx->sg ? ctx->sg->captures : 0;
+  *launches = ctx->sg ? ctx->sg->launches : 0;
+  *refusals = ctx->sg ? ctx->sg->refusals : 0;
   return 0;
 }
 

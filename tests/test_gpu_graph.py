@@ -47,3 +47,30 @@ def test_graph_steps_match_plain_steps(glsizes, tmp_path):
         for g, r in pairs:
             g.close()
             r.close()
+
+
+@pytest.mark.parametrize("glsizes", [(32, 48), (300, 20), (8191, 4), (16, 12, 20)])
+def test_steps_are_replayed_and_switches_build_anew(glsizes, tmp_path):
+    """The first step is issued launch by launch, the second builds the graph,
+    all others replay it; a switch that changes the launches builds one graph,
+    one that does not builds none, per-kernel timing replays none, and the
+    runtime refuses nothing (8191: x lines of more than 64 KiB of LDS)."""
+    g = sva.solver_from_ic(random_fields(glsizes, seed=5, uniformx=True), str(tmp_path / "g"))
+    try:
+        assert g.graph_counts() == (0, 0, 0)
+        g.integrate()
+        assert g.graph_counts() == (0, 0, 0)
+        built, replayed = 0, 0
+        for switch, builds, replays in [
+                (lambda: None, 1, 1), (lambda: g.set("ux", 0.5 * g.get("ux")), 0, 1), (lambda: g.set_tuning("rhs_rows", 4), 1, 1),
+                (lambda: g.set_poisson_mixed(1), 1, 1), (lambda: g.set_poisson_mixed(-1), 1, 1),
+                (lambda: g.set_tuning("xcd_bands", 1), 0, 1), (lambda: g.profile(True), 0, 0),
+                (lambda: g.profile(False), 0, 1)]:
+            switch()
+            for k in range(3):
+                g.integrate()
+                built += builds if k == 0 else 0
+                replayed += replays
+                assert g.graph_counts() == (built, replayed, 0), (k, builds)
+    finally:
+        g.close()
