@@ -406,8 +406,8 @@ int vof_batch_autotune(vof_batch_t * batch, int steps, char * report, size_t len
  * per work-group of the predictor's x solver (0 = automatic); "xcd_bands" =
  * 1 walks the 3D stencil tiles band by band per XCD; "rhs_rows" = 1, 2, 4,
  * 8 or 16 rows of one column per thread of the source kernel (default: by
- * the grid's size, 1 on the smallest, 8 on large ones; in a batch by the
- * cases' together);
+ * the grid's size, 1 on the smallest, 8 on large ones; in a batch by those of
+ * the cases of a part together);
  * "pred_rows" = 1, 2, 4 or 8 (default) rows per thread of the one-kernel
  * predictor (fewer where its x lines would not fit 64 KiB of LDS);
  * "iface_planes" = 0 (blocks), 4, 8 or 16 z planes marched per work-group by

@@ -1328,19 +1328,20 @@ __device__ __forceinline__ void lines_sweep_wave(const double * tab, int n, doub
 }
 
 // Phase 2 of k_lines_lds: one wavefront eliminates up to 16 lines (line l at
-// S + l ld) with the rows in registers.  Lane 16 h + l holds rows 128 p + 32 h
-// .. + 31 of line l (pass p), so a line runs through the four 16-lane DPP rows
+// S + l ld) with the rows in registers.  Lane 16 h + l holds rows 64 p + 16 h
+// .. + 15 of line l (pass p), so a line runs through the four 16-lane DPP rows
 // in turn: row h works under its exec mask, then hands x of its last row on
-// (rot_up / rot_dn).  The factors of a lane row's 32 matrix rows sit in two
-// registers per factor, one matrix row per lane, and reach all 16 lanes by a
+// (rot_up / rot_dn).  The factors of a lane row's 16 matrix rows sit in one
+// register per factor, one matrix row per lane, and reach all 16 lanes by a
 // 64-bit row_newbcast move; a serial row is then 2 moves + 3 FP64 operations
 // forward and 1 + 2 backward, with no LDS access and no scalar load (whose
 // out-of-order return makes each use wait for everything outstanding) on the
 // recurrence.  LDS is read and written 16 bytes at a time, twice per pass.
-// At 256 rows the sweep takes 7.6 us with the tables loaded on use, against
-// 11.2 us with rows read from LDS two groups of 8 ahead and v_readlane
-// factors, 14.7 us with one group ahead, 15.1 us with scalar-load factors
-// (16 lines, three work-groups per CU).
+// At 256 rows the sweep of 16 lines takes 9.2 us, three wavefronts per CU
+// (100 rows 4.3), against 11.2 us with rows read from LDS two groups of 8
+// ahead and v_readlane factors, 14.7 us with one group ahead, 15.1 us with
+// scalar-load factors; 32 rows per lane take 7.5 us, but 127 registers, with
+// which k_lines_lds as a whole is slower.
 // Per line the operations are gtsv's: q[0] / c0 (then row 0 is a row with L =
 // 0, VAL = 1), q[i] = VAL[i] (q[i] - L[i] q[i-1]) with VAL = rlast in the last
 // row (0 there when the last pivot is singular), back substitution q[i] -=
@@ -2526,8 +2527,9 @@ __global__ __launch_bounds__(kTpLines * kTpSeg) void k_thomas_part(int nx, int n
 // The sequential elimination of k_thomas_spec where the lines are too few to
 // fill the chip (2D: ny / 2 + 1 of them), with its factors built once per grid
 // by the same operations (k_thomas_fac; they depend on the grid alone).  One
-// wavefront runs 8 lines, the components being 16 systems, as lines_sweep_rows
-// does: lane 16 h + s holds rows 128 p + 32 h .. + 31 of system s in pass p.
+// wavefront runs 8 lines, the components being 16 systems, in turn through the
+// 16-lane rows as in lines_sweep_rows, with 32 rows per lane: lane 16 h + s
+// holds rows 128 p + 32 h .. + 31 of system s in pass p.
 // The spectrum's 8 lines are one 128-byte row per x, so a pass loads straight
 // into that layout, one pass ahead.  Per component the operations and their
 // order are those of k_thomas_spec.  Latency-bound by the serial rows: 513

@@ -1001,8 +1001,8 @@ static std::vector<double2> make_twiddles(int n) {
 static bool thomas_seq_lines(size_t nlines) { return nlines <= 3072; }
 
 // rows per thread of the source kernel and planes per work-group of the 3D
-// interface kernel, for cases whose launches run together (one case, or a
-// batch's): 8 where that leaves 16 work-groups of 256 threads per CU, 4 where
+// interface kernel, for cases whose launches run together (one case, or those
+// of a batch or of one part of it): 8 where that leaves 16 work-groups of 256 threads per CU, 4 where
 // it leaves 8, else 2 rows from one work-group per CU on, else 1 (no march):
 // each row or plane marched saves re-reading its neighbours, but a grid of
 // few work-groups is bound by the march itself.  Measured, us per launch at
@@ -2462,7 +2462,6 @@ static int freeze_slot(vof_ctx * ctx, vofk::Freeze * fz) {
 }
 #endif
 
-// RK stages rk0 .. rk1-1 (all three by default) of one step with dt known
 // fused curvature tensor (curvature_tensor.c:178-186) of the current vof
 // on ctx->stream
 static int launch_iface(vof_ctx * ctx, interface_t * interface) {
@@ -2592,6 +2591,7 @@ static int graph_stages(const domain_t * domain, fluid_t * fluid, interface_t * 
   return 0;
 }
 
+// RK stages rk0 .. rk1-1 (all three by default) of one step with dt known
 static int integrate_fused_stages(const domain_t * domain, fluid_t * fluid, interface_t * interface,
                                   const double dtv, size_t rk0, size_t rk1) {
   vof_ctx * ctx = ctx_of(domain);
@@ -3547,8 +3547,6 @@ extern "C" int vof_set_freeze(domain_t * domain, int mode) {
 #endif
 }
 
-// one step with a given dt (the frozen dt sequence of the adjoint and its
-// finite-difference checks); fused schedule
 // the stages of one step with a given dt, nothing waited for before
 static int stages_fixed_dt(const domain_t * domain, fluid_t * fluid, interface_t * interface, double dt) {
   vof_ctx * ctx = ctx_of(domain);
@@ -3557,6 +3555,8 @@ static int stages_fixed_dt(const domain_t * domain, fluid_t * fluid, interface_t
   return rc;
 }
 
+// one step with a given dt (the frozen dt sequence of the adjoint and its
+// finite-difference checks); fused schedule
 extern "C" int vof_integrate_fixed_dt(const domain_t * domain, fluid_t * fluid, interface_t * interface,
                                       double dt) {
   CTX_OR_FAIL(domain);
