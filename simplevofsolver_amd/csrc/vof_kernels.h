@@ -1169,30 +1169,43 @@ struct LineJob {
 constexpr int kWThreads = 256;
 constexpr int kWUnroll = 6;
 
-// Phases 1 and 3 walk the (line, 64-row chunk) pairs of a group: wavefront w
-// of nw owns pairs w, w + nw, ..., kWUnroll at a time with all their loads
-// issued (indices clamped, so that no branch separates them) before the
-// first value is used.  Line, row, plane and chunk are wave-uniform.  Pair p
-// is chunk p % nch of line p / nch; the quotient comes from a 16-bit
-// reciprocal (a group has at most 192 pairs and nch <= 128).
+// Phases 1 and 3 walk the (line, chunk of W rows) units of a group, 64 / W of
+// them per access of a wavefront: wavefront w of nw owns accesses w, w + nw,
+// ..., kWUnroll at a time with all their loads issued (indices clamped, so
+// that no branch separates them) before the first value is used.  With W = 64
+// line, row, plane and chunk are wave-uniform; W = 16 is for lines that leave
+// most lanes of 64-row chunks without a row.  Unit q is chunk q % nch of line
+// q / nch; the quotient comes from a 16-bit reciprocal (q times its error,
+// below nch, stays under 65536: at most 192 units of 64 rows and nch <= 128,
+// 512 of 16 rows and nch <= 8).
 __device__ __forceinline__ int pair_line(int p, int inv) { return (p * inv) >> 16; }
 
 struct LineGroup {             // the lines of one work-group, uniform
-  int n, ld, np, nch, inv;     // rows, LDS stride, pairs, chunks of a line and their reciprocal
+  int n, ld, np, nu;           // rows, LDS stride, accesses, units
+  int nch, inv;                // chunks of a line and their reciprocal
   int j0, k0, nw, lane;        // row and plane of the first line; wavefronts
   size_t g0;                   // its first increment
 };
+// line l and row m (past the line's last one in a partial chunk) of this
+// lane in access p; units past the last one are clamped to it
+template <int W>
+__device__ __forceinline__ void lines_at(const LineGroup & G, int p, int & l, int & m) {
+  const int q = W == 64 ? p : min(p * (64 / W) + G.lane / W, G.nu - 1);
+  l = pair_line(q, G.inv);
+  m = W * (q - l * G.nch) + G.lane % W;
+}
 
-// the increments of pairs p0 + nw u into registers: F.q's, or (SRC, the
+// the increments of accesses p0 + nw u into registers: F.q's, or (SRC, the
 // per-function entry point) formed from the three sources
-template <bool SRC>
+template <bool SRC, int W>
 __device__ __forceinline__ void lines_load(const LineField & F, const LineJob & J, const LineGroup & G, int p0,
                                            double * v) {
   size_t g[kWUnroll];
 #pragma unroll
   for (int u = 0; u < kWUnroll; u++) {
-    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
-    g[u] = G.g0 + (size_t)(l * G.n + min(64 * (p - l * G.nch) + G.lane, G.n - 1));
+    int l, m;
+    lines_at<W>(G, min(p0 + G.nw * u, G.np - 1), l, m);
+    g[u] = G.g0 + (size_t)(l * G.n + min(m, G.n - 1));
   }
   if constexpr (SRC) {
     double a[kWUnroll], b[kWUnroll], c[kWUnroll];
@@ -1209,12 +1222,14 @@ __device__ __forceinline__ void lines_load(const LineField & F, const LineJob & 
     for (int u = 0; u < kWUnroll; u++) v[u] = F.q[g[u]];
   }
 }
-// ... and into S (clamped lanes and pairs repeat a value of their wavefront)
+// ... and into S (clamped lanes and accesses repeat a value of their group)
+template <int W>
 __device__ __forceinline__ void lines_stage(const LineGroup & G, double * S, int p0, const double * v) {
 #pragma unroll
   for (int u = 0; u < kWUnroll; u++) {
-    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
-    S[l * G.ld + min(64 * (p - l * G.nch) + G.lane, G.n - 1)] = v[u];
+    int l, m;
+    lines_at<W>(G, min(p0 + G.nw * u, G.np - 1), l, m);
+    S[l * G.ld + min(m, G.n - 1)] = v[u];
   }
 }
 
@@ -1227,15 +1242,16 @@ __device__ __forceinline__ size_t lines_row(const LineField & F, const LineJob &
   return (size_t)F.i0 + (size_t)F.n0 * ((size_t)(j + 1) + (size_t)J.n1 * (size_t)(k + 1));
 }
 
-// the field values of the same pairs
+// the field values of the same accesses
+template <int W>
 __device__ __forceinline__ void lines_field(const LineField & F, const LineJob & J, const LineGroup & G, int p0,
                                             double * v) {
 #pragma unroll
   for (int u = 0; u < kWUnroll; u++) {
-    const int p = min(p0 + G.nw * u, G.np - 1), l = pair_line(p, G.inv);
-    int j, k;
+    int l, m, j, k;
+    lines_at<W>(G, min(p0 + G.nw * u, G.np - 1), l, m);
     const size_t r = lines_row(F, J, G, l, j, k);
-    v[u] = F.field[r + (size_t)min(64 * (p - l * G.nch) + G.lane, G.n - 1)];
+    v[u] = F.field[r + (size_t)min(m, G.n - 1)];
   }
 }
 
@@ -1538,6 +1554,7 @@ __device__ __forceinline__ bool lines_edge(const LineJob & J, int j, int k) {
 // The Dirichlet wall entries of those rows (constants the loop never changes)
 // take their images as the reference's halo copy would (overwriting values
 // left from the initial load).
+template <int W>
 __device__ __forceinline__ void lines_update(const LineField & F, const LineJob & J, const LineGroup & G, double * S,
                                              int p0, const double * v) {
   bool any = false;
@@ -1545,8 +1562,8 @@ __device__ __forceinline__ void lines_update(const LineField & F, const LineJob 
   for (int u = 0; u < kWUnroll; u++) {
     const int p = p0 + G.nw * u;
     if (p < G.np) {
-      const int l = pair_line(p, G.inv), m = 64 * (p - l * G.nch) + G.lane;
-      int j, k;
+      int l, m, j, k;
+      lines_at<W>(G, p, l, m);
       const size_t r = lines_row(F, J, G, l, j, k);
       const double x = v[u] + S[l * G.ld + min(m, G.n - 1)];
       if (m < G.n) st_stream(&F.field[r + (size_t)m], x);
@@ -1561,8 +1578,8 @@ __device__ __forceinline__ void lines_update(const LineField & F, const LineJob 
   for (int u = 0; u < kWUnroll; u++) {
     const int p = p0 + G.nw * u;
     if (p >= G.np) break;
-    const int l = pair_line(p, G.inv), m = 64 * (p - l * G.nch) + G.lane;
-    int j, k;
+    int l, m, j, k;
+    lines_at<W>(G, p, l, m);
     const size_t r = lines_row(F, J, G, l, j, k);
     if (!lines_edge(J, j, k)) continue;
     if (m < G.n) store_images(F.field, F.i0 + m, F.n0, J.n1, j + 1, k + 1, J.ny, J.nz, 1, S[l * G.ld + m]);
@@ -1584,7 +1601,7 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <bool SRC>
+template <bool SRC, int W>
 __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJob & J, int lpb) {
   extern __shared__ __align__(16) double S[];
   const LineField & F = J.f[vb.y];
@@ -1595,8 +1612,9 @@ __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJo
   LineGroup G;
   G.n = F.n;
   G.ld = lines_stride(F.n);
-  G.nch = (F.n + 63) >> 6;
-  G.np = nl * G.nch;
+  G.nch = (F.n + W - 1) / W;
+  G.nu = nl * G.nch;
+  G.np = (G.nu + 64 / W - 1) / (64 / W);
   G.inv = (65536 + G.nch - 1) / G.nch;
   G.k0 = line0 / J.ny;
   G.j0 = line0 - G.k0 * J.ny;
@@ -1609,28 +1627,28 @@ __device__ __forceinline__ void k_lines_lds_body(const VBlock & vb, const LineJo
   // first batch's field rows are loaded with its increments and stay in
   // registers across the sweep (the LDS barriers leave them in flight)
   double v[kWUnroll], f[kWUnroll];
-  lines_load<SRC>(F, J, G, w, v);
+  lines_load<SRC, W>(F, J, G, w, v);
   const SweepHead h = sweep_head(F.tab, G.n, lane);
-  lines_field(F, J, G, w, f);
-  lines_stage(G, S, w, v);
+  lines_field<W>(F, J, G, w, f);
+  lines_stage<W>(G, S, w, v);
   for (int p0 = w + step; p0 < G.np; p0 += step) {
-    lines_load<SRC>(F, J, G, p0, v);
-    lines_stage(G, S, p0, v);
+    lines_load<SRC, W>(F, J, G, p0, v);
+    lines_stage<W>(G, S, p0, v);
   }
   lds_barrier();
   for (int l = kSwLines * w; l < nl; l += kSwLines * G.nw)
     lines_sweep_rows(h, F.tab, G.n, S + (size_t)l * G.ld, G.ld, min(kSwLines, nl - l), lane);
   lds_barrier();
-  lines_update(F, J, G, S, w, f);
+  lines_update<W>(F, J, G, S, w, f);
   for (int p0 = w + step; p0 < G.np; p0 += step) {
-    lines_field(F, J, G, p0, f);
-    lines_update(F, J, G, S, p0, f);
+    lines_field<W>(F, J, G, p0, f);
+    lines_update<W>(F, J, G, S, p0, f);
   }
 }
 
-template <bool SRC>
+template <bool SRC, int W>
 __global__ __launch_bounds__(kWThreads) void k_lines_lds(LineJob J, int lpb) {
-  k_lines_lds_body<SRC>(hw_block(), J, lpb);
+  k_lines_lds_body<SRC, W>(hw_block(), J, lpb);
 }
 
 // ---------------------------------------------------------------------------

@@ -1766,17 +1766,27 @@ static int pred_rows_for(const vof_ctx * ctx, int * xw) {
 static int launch_lines(vof_ctx * ctx, vofk::LineJob & lj, int nj) {
   const int nx = ctx->nx;
   lj.inv_ny = 0xffffffffu / (unsigned)lj.ny + 1u;
-  // lines per work-group: two full batches of each wavefront's loads, 48
+  // chunks of 16 rows for lines of up to 96 rows, where 64-row chunks leave a
+  // quarter of their lanes or more without a row (not 49 to 64 rows): us at 64
+  // / 16 rows 12 x 240 x 240 59.8 / 29.4, 24 x 200 x 200 47.6 / 34.0, 48 x 200
+  // x 200 50.7 / 45.5, 65 x 128 x 128 45.4 / 38.4, 90 x 200 x 120 62.4 / 53.7;
+  // 100^3 36.7 / 35.9, but its per-function call 32.1 / 33.9, and 125 x 120 x
+  // 120 48.2 / 50.7.  Not in a batch: cases on both sides would make two merged
+  // launches of one (12 cases 24 to 100 wide 508 -> 580 us a step).
+  // Lines per work-group: two full batches of each wavefront's loads, 48
   // (line, 64-row chunk) pairs, with an LDS tile of about 25 KiB, so that six
   // work-groups share a CU (256^3: 338 us at 12 lines, 342 at 11, 351 at
   // 13, 456 at 6; 150 x 135 x 100: 59 us at 16, 64 at 12 and at 8); one batch
-  // for lines of up to two chunks, whose tile is small either way (100^3:
-  // 37.0 us at 12 lines, 41.4 at 24; 16 x 200 x 200 44.8 at 24, 49.0 at 48;
-  // 128^3 54.0 at 12, 54.5 at 24); fewer where that leaves compute units idle
-  // (128 x 256: 10.5 us at 4 lines, 12.4 at 16)
-  const int nch = (nx + 63) / 64;
-  const int pairs = nch <= 2 ? 24 : 48;
-  int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(pairs / nch, max(4, lj.nlines * nj / 256));
+  // where two of them would be little more than one round of work-groups that
+  // load, sweep and store together, for lines of up to two chunks (100^3: 37.0
+  // us at 12 lines, 41.4 at 24; but the 128^3 step 1181 us at 12 and 1168 at
+  // 24), in 16-row chunks whole sweeps of 16 lines (75 x 128 x 128: 39.4 us at
+  // 16, 41.2 at 19); fewer where that leaves compute units idle (128 x 256:
+  // 10.5 us at 4 lines, 12.4 at 16)
+  const int n64 = (nx + 63) / 64, n16 = (nx + 15) / 16, all = lj.nlines * nj;
+  const bool w16 = n16 <= 6 && n16 != 4 && !(ctx->rec && !ctx->rec->graph);
+  const int most = w16 ? 96 / n16 / 16 * 16 : n64 <= 2 && all < 2048 * (48 / n64) ? 24 / n64 : 48 / n64;
+  int lpb = ctx->lines_lpb > 0 ? ctx->lines_lpb : min(most, max(4, all / 256));
   lpb = max(1, min(lpb, 64));
   if (sizeof(double) * (nx | 1) > 65536) return fail("x solver: nx = %d exceeds the LDS line tile", nx);
   const size_t row = sizeof(double) * (size_t)vofk::lines_stride(nx);   // at least ux's
@@ -1784,10 +1794,17 @@ static int launch_lines(vof_ctx * ctx, vofk::LineJob & lj, int nj) {
   const size_t shm = (size_t)lpb * row;
   const int ngroups = (lj.nlines + lpb - 1) / lpb;
   const dim3 g((unsigned)ngroups, (unsigned)nj), b(vofk::kWThreads);
-  if (lj.f[0].srcg)
-    KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body<true>, vofk::k_lines_lds<true>, g, b, shm, lj, lpb);
-  else
-    KLB(ctx, "k_lines_lds", vofk::kWThreads, vofk::k_lines_lds_body<false>, vofk::k_lines_lds<false>, g, b, shm, lj, lpb);
+#define LINES(SRC, W)                                                                                             \
+  KLB(ctx, "k_lines_lds", vofk::kWThreads, (vofk::k_lines_lds_body<SRC, W>), (vofk::k_lines_lds<SRC, W>), g, b, shm, \
+      lj, lpb)
+  if (lj.f[0].srcg) {
+    if (w16) LINES(true, 16);
+    else LINES(true, 64);
+  } else {
+    if (w16) LINES(false, 16);
+    else LINES(false, 64);
+  }
+#undef LINES
   return 0;
 }
 

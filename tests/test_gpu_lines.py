@@ -60,3 +60,34 @@ def test_fused_lines_match_per_function_lines(glsizes, lpb, tmp_path):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("lpb", [0, 5, 64])
+@pytest.mark.parametrize("glsizes", [(4, 90), (16, 75), (32, 9), (47, 6), (48, 20), (49, 6), (80, 5), (96, 20), (97, 9),
+                                     (6, 20, 16), (48, 9, 8), (81, 5, 6), (97, 6, 5)])
+def test_lines_in_chunks_of_16_rows(glsizes, lpb, tmp_path):
+    """Both sides of the limits between chunks of 16 and of 64 rows (nx 48 / 49
+    and 96 / 97; ux has one row fewer), with the last access of a group partly
+    past its last line: the fused step against the per-function one bit for
+    bit, halo images included, and its line solves against the oracle's."""
+    import simplevofsolver_amd as sva
+    ic = random_fields(glsizes, seed=4, uniformx=False)
+    o, a = make_pair(ic, tmp_path / "a")
+    b = sva.solver_from_ic(ic, str(tmp_path / "b"), schedule=0)
+    names = ["ux", "uy", "t"] + (["uz"] if len(glsizes) == 3 else [])
+    try:
+        a.set_tuning("lines_lpb", lpb)
+        b.set_tuning("lines_lpb", lpb)
+        for _ in range(2):
+            assert a.integrate() == b.integrate()
+        for n in names:
+            assert np.array_equal(a.get(n), b.get(n)), n
+        dt = o.decide_dt()
+        copy_state(o, b)
+        o.predict(0, dt)
+        b.predict(0, dt)
+        for n in names:
+            assert np.array_equal(b.get(n), o.get(n)), n
+    finally:
+        a.close()
+        b.close()
