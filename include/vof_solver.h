@@ -330,10 +330,10 @@ int vof_set_poisson_mixed(domain_t * domain, int refinements);
 typedef struct vof_batch vof_batch_t;
 int vof_batch_create(int ncases, const domain_t * const domains[], fluid_t * const fluids[],
                      interface_t * const interfaces[], vof_batch_t ** batch);
-/* the step graph of a single case: integrate issues a case's first step (and
- * every step on two streams, with per-kernel timing, decision record or
- * partial fusion) launch by launch, and replays the others as a graph that is
- * built anew when the sequence of kernels or grids changes.  Graphs built,
+/* the step graph of a single case: integrate issues a case's first step on
+ * one stream (and every step on two streams, with per-kernel timing, decision
+ * record or partial fusion) launch by launch, and replays the others as a graph
+ * that is built anew when the sequence of kernels or grids changes.  Graphs built,
  * replayed, and refused by the runtime so far (one refusal sends the case's
  * later steps out launch by launch) */
 int vof_graph_counts(const domain_t * domain, size_t * captures, size_t * launches, size_t * refusals);

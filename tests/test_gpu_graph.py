@@ -74,3 +74,91 @@ def test_steps_are_replayed_and_switches_build_anew(glsizes, tmp_path):
                 assert g.graph_counts() == (built, replayed, 0), (k, builds)
     finally:
         g.close()
+
+
+OPTIONS = {
+    "one-kernel predictor": lambda s: s.set_fusion(127),
+    "sequential x solve": lambda s: s.set_tuning("thomas_part", 0),
+    "mixed radix": lambda s: (s.set_tuning("fft_radix", 4), s.set_tuning("fft_elems", 2048)),
+    "two refinements": lambda s: s.set_poisson_mixed(2),
+    "bands and rows": lambda s: (s.set_tuning("xcd_bands", 1), s.set_tuning("rhs_rows", 16), s.set_tuning("lines_lpb", 5)),
+    "two streams for a while": lambda s: s.set_tuning("iface_overlap", 1),
+}
+
+
+@pytest.mark.parametrize("option", list(OPTIONS))
+@pytest.mark.parametrize("glsizes", [(20, 45), (16, 256), (300, 20), (24, 20, 15)])
+def test_graph_steps_with_options(glsizes, option, tmp_path):
+    """The options that change a step's kernels or swap its buffers, set before
+    the first step and taken back (two streams, after which the next step is
+    the first on one stream) or repeated later on."""
+    nd = len(glsizes)
+    ic = random_fields(glsizes, seed=11, uniformx=False)
+    g = sva.solver_from_ic(ic, str(tmp_path / "g"))
+    r = sva.solver_from_ic(ic, str(tmp_path / "r"))
+    try:
+        r.profile(True)
+        for s in (g, r):
+            OPTIONS[option](s)
+        for step in range(9):
+            if step == 4:
+                for s in (g, r):
+                    if option == "two streams for a while":
+                        s.set_tuning("iface_overlap", 0)
+                    else:
+                        OPTIONS[option](s)
+            assert g.integrate() == r.integrate(), step
+            for n in ["ux", "uy", "p", "t", "vof"] + (["uz"] if nd == 3 else []):
+                assert np.array_equal(g.get(n), r.get(n)), (step, n)
+        built, replayed, refused = g.graph_counts()
+        assert refused == 0 and built == 1
+        assert replayed == (4 if option == "two streams for a while" else 8)
+    finally:
+        g.close()
+        r.close()
+
+
+def test_graph_steps_in_threads(tmp_path):
+    """Three solvers and a batch, each stepped by a thread of its own at the
+    same time, against the same steps one after another."""
+    import threading
+    grids = [(32, 48), (20, 45), (40, 24), (24, 30), (48, 20), (16, 36)]
+
+    def make(tag):
+        ss = [sva.solver_from_ic(random_fields(z, seed=21 + k, uniformx=k % 2 == 0), str(tmp_path / f"{tag}{k}"))
+              for k, z in enumerate(grids)]
+        return ss, sva.Batch(ss[3:])
+
+    def run(jobs, threads):
+        if not threads:
+            for j in jobs:
+                j()
+            return
+        ts = [threading.Thread(target=j) for j in jobs]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join(60)
+            assert not t.is_alive()
+
+    out = []
+    for tag, threads in (("a", False), ("b", True)):
+        ss, batch = make(tag)
+        dts = {}
+
+        def steps(k, f):
+            dts[k] = [f() for _ in range(30)]
+
+        try:
+            run([lambda k=k: steps(k, ss[k].integrate) for k in range(3)] + [lambda: steps("batch", batch.integrate)],
+                threads)
+            batch.synchronize()
+            out.append((dts, [[s.get(n) for n in ("ux", "uy", "p", "t", "vof")] for s in ss]))
+            assert all(s.graph_counts() == (1, 29, 0) for s in ss[:3])
+        finally:
+            batch.close()
+            for s in ss:
+                s.close()
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1], out[1][1]):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
